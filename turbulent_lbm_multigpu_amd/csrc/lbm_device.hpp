@@ -234,6 +234,7 @@ __host__ __device__ constexpr int cells_per_lane(int var) { return 1 << ((var >>
 // ---- per-(sub)domain launch descriptor ---------------------------------------
 struct DomDev {
     void *dd;          // blocks of kBlk cells x 19 populations
+    void *dd2;         // a second buffer of the same layout (pair_kernel), or null
     uint8_t *flags;    // one byte per cell
     void *vel;         // [3][cells] compute type, or null
     void *dens;        // [cells] compute type, or null
@@ -380,20 +381,41 @@ __device__ __forceinline__ void body_force(T *f, T rho, T gx, T gy, T gz) {
 // Alpha-kernel forcing with the reference's `#define tmp rho` alias: each term
 // is scaled by the previous term (src/cl_programs/lbm_alpha.cl:173,183-298).
 // Returns the aliased variable, which the reference stores as density.
+// ref_factor: the factor of term k, which does not depend on the cell.
+template <typename T>
+__device__ __forceinline__ T ref_factor(int k, T gx, T gy, T gz) {
+    const T w1 = LC<T>::w1, w2 = LC<T>::w2;
+    switch (k) {
+        case 0: return gx * w1;
+        case 1: return gy * (-w1);
+        case 2: return (gx - gy) * w2;
+        case 3: return (gx + gy) * w2;
+        case 4: return (gx + gz) * w2;
+        case 5: return (gx - gz) * w2;
+        case 6: return (gz - gy) * w2;
+        case 7: return (gz + gy) * (-w2);
+        default: return gz * w1;
+    }
+}
+template <typename T, class F>
+__device__ __forceinline__ T alpha_ref_chain(T *f, T rho, F &&factor) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        const T tmp = factor(k) * rho;
+        rho = tmp;
+        f[2 * k + 1] = f[2 * k + 1] - tmp;
+        f[2 * k] = f[2 * k] + tmp;
+    }
+    return rho;
+}
 template <typename T>
 __device__ __forceinline__ T alpha_ref_forcing(T *f, T rho, T gx, T gy, T gz) {
-    const T w1 = LC<T>::w1, w2 = LC<T>::w2;
-    T tmp;
-    tmp = (gx * w1) * rho;           rho = tmp; f[1] = f[1] - tmp;   f[0] = f[0] + tmp;
-    tmp = (gy * (-w1)) * rho;        rho = tmp; f[3] = f[3] - tmp;   f[2] = f[2] + tmp;
-    tmp = ((gx - gy) * w2) * rho;    rho = tmp; f[5] = f[5] - tmp;   f[4] = f[4] + tmp;
-    tmp = ((gx + gy) * w2) * rho;    rho = tmp; f[7] = f[7] - tmp;   f[6] = f[6] + tmp;
-    tmp = ((gx + gz) * w2) * rho;    rho = tmp; f[9] = f[9] - tmp;   f[8] = f[8] + tmp;
-    tmp = ((gx - gz) * w2) * rho;    rho = tmp; f[11] = f[11] - tmp; f[10] = f[10] + tmp;
-    tmp = ((gz - gy) * w2) * rho;    rho = tmp; f[13] = f[13] - tmp; f[12] = f[12] + tmp;
-    tmp = ((gz + gy) * (-w2)) * rho; rho = tmp; f[15] = f[15] - tmp; f[14] = f[14] + tmp;
-    tmp = (gz * w1) * rho;           rho = tmp; f[17] = f[17] - tmp; f[16] = f[16] + tmp;
-    return rho;
+    return alpha_ref_chain(f, rho, [&](int k) { return ref_factor<T>(k, gx, gy, gz); });
+}
+// the same from a descriptor (parameters that keep the factors have an overload of their own)
+template <typename T>
+__device__ __forceinline__ T ref_forcing(const DomDev *D, T *f, T rho) {
+    return alpha_ref_forcing(f, rho, (T)D->gx, (T)D->gy, (T)D->gz);
 }
 
 // FLUID collision shared by both kernels: optional LES rate, then BGK
@@ -457,9 +479,9 @@ __device__ __forceinline__ int wrap_idx(int a, int cells) {
 // FP32), far below the storage's rounding.  Only these storages take this
 // form: the FP32 and FP64 kernels keep the reference's expression order, which
 // their bit parity with the CPU oracle rests on.
-template <bool BETA>
-__device__ __forceinline__ bool cell_update_pairs(float *f, int flag, const DomDev *D, float &vx, float &vy,
-                                                  float &vz, float &dens_out) {
+template <bool BETA, class PP>
+__device__ __forceinline__ bool cell_update_pairs(float *f, int flag, const PP *D, float &vx, float &vy, float &vz,
+                                                  float &dens_out) {
     float s[9], d[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
@@ -516,7 +538,7 @@ __device__ __forceinline__ bool cell_update_pairs(float *f, int flag, const DomD
         }
         f[18] = om1 * f[18] + (om * LC<float>::w0) * ddp;
         if (!body) {
-            if (!BETA) dens_out = alpha_ref_forcing(f, rho_full, (float)D->gx, (float)D->gy, (float)D->gz);
+            if (!BETA) dens_out = ref_forcing(D, f, rho_full);
             else dens_out = 1.0f + ddp;  // `#define dd_param rho` (lbm_beta.cl:493)
         }
         return true;
@@ -538,7 +560,7 @@ __device__ __forceinline__ bool cell_update_pairs(float *f, int flag, const DomD
         const float dd_param = -1.5f * vel2_of(vx, vy, vz);
         feq19(dd_param, vx, vy, vz, f);
         if (BETA) dens_out = 1.0f + dd_param;
-        else if (D->forcing == 0) dens_out = alpha_ref_forcing(f, 1.0f, (float)D->gx, (float)D->gy, (float)D->gz);
+        else if (D->forcing == 0) dens_out = ref_forcing(D, f, 1.0f);
         else dens_out = 1.0f;
         return true;
     }
@@ -550,9 +572,10 @@ __device__ __forceinline__ bool cell_update_pairs(float *f, int flag, const DomD
 // entry and the values to store on exit; returns whether they are stored
 // (alpha stores FLUID and VELOCITY_INJECTION cells only, beta every cell).
 // SHIFT (the two-byte storages, f[] holding f_i - w_i) takes the pair form
-// above.
-template <typename T, bool BETA, bool SHIFT = false>
-__device__ __forceinline__ bool cell_update(T *f, int flag, const DomDev *D, T &vx, T &vy, T &vz, T &dens_out) {
+// above.  D holds the physical parameters: the domain's descriptor, or a copy
+// of them in the compute type with the same names.
+template <typename T, bool BETA, bool SHIFT = false, class PP = DomDev>
+__device__ __forceinline__ bool cell_update(T *f, int flag, const PP *D, T &vx, T &vy, T &vz, T &dens_out) {
     if constexpr (SHIFT) return cell_update_pairs<BETA>(f, flag, D, vx, vy, vz, dens_out);
     T rho;
     if (BETA) {  // summation order of lbm_beta.cl:268-483
@@ -605,7 +628,7 @@ __device__ __forceinline__ bool cell_update(T *f, int flag, const DomDev *D, T &
         if (D->forcing == 1) {
             body_force(f, rho_full, (T)D->gx, (T)D->gy, (T)D->gz);
         } else if (!BETA) {
-            dens_out = alpha_ref_forcing(f, rho_full, (T)D->gx, (T)D->gy, (T)D->gz);
+            dens_out = ref_forcing(D, f, rho_full);
         } else {
             dens_out = dd_param;  // `#define dd_param rho` (lbm_beta.cl:493)
         }
@@ -626,7 +649,7 @@ __device__ __forceinline__ bool cell_update(T *f, int flag, const DomDev *D, T &
         const T dd_param = one - T(1.5) * vel2_of(vx, vy, vz);
         feq19(dd_param, vx, vy, vz, f);
         if (BETA) dens_out = dd_param;
-        else if (D->forcing == 0) dens_out = alpha_ref_forcing(f, one, (T)D->gx, (T)D->gy, (T)D->gz);
+        else if (D->forcing == 0) dens_out = ref_forcing(D, f, one);
         else dens_out = one;
         write_dd = true;
     }

@@ -8,18 +8,23 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <limits>
 #include <mutex>
+#include <set>
+#include <shared_mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/lbm_capi.h"
+#include "device_memory.hpp"
 #include "exchange_plan.hpp"
 #include "launch_shape.hpp"
 #include "lbm_device.hpp"
+#include "lbm_pair.hpp"
 
 using namespace lbm;
 
@@ -379,7 +384,15 @@ struct lbm_solver {
     size_t staging_bytes = 0;
     double *d_partials = nullptr;
     size_t partial_count = 0;
-    unsigned version = 0;      // bumps when kernel parameters change
+    // second buffer of the fused pairs, allocated by the first run that takes
+    // them; another thread may take it away between runs (SecondBuffers)
+    std::atomic<void *> dd2{nullptr};
+    void *desc_dd2 = nullptr;    // the one d_desc names
+    bool dd2_refused = false;    // there was no memory for it
+    PairTile *d_pair = nullptr;  // tiles of the fused pairs of a run on its own
+    int npair = 0;
+    PairLaunch pair_launch{};
+    std::atomic<unsigned> version{0};  // bumps when kernel parameters change
     lbm_group *group = nullptr;
     bool external = false;     // buffers live in caller-provided device memory
     SharedBlock *block = nullptr;  // buffers live in a block shared with other solvers (lbm_solver_colocate)
@@ -428,6 +441,10 @@ struct lbm_group {
     std::string err;
     LaunchTables lt[2];        // [0]: at wg (beta, and alpha unless wg_alpha is set), [1]: alpha at wg_alpha
     long long *d_ctr = nullptr;  // device half-step counter (two slots, see step_kernel)
+    PairTile *d_pair = nullptr;  // tiles of the fused pairs (groups without exchange)
+    size_t pair_cap = 0;
+    int npair = 0;               // 0: not planned for the present members
+    PairLaunch pair_launch{};
     std::vector<unsigned> seen_versions;
     std::vector<GroupComm> comms;
     bool plan_built = false;
@@ -448,6 +465,7 @@ struct lbm_group {
     int graph_pairs = 64;  // most beta+alpha pairs one graph launch replays
     struct Graph {
         int pairs;
+        bool fused;  // pairs two by two through the second buffers
         hipGraph_t graph;
         hipGraphExec_t exec;
         unsigned long long used;
@@ -469,6 +487,26 @@ struct lbm_group {
 };
 
 namespace {
+
+// The second buffers of the solvers that took fused pairs.  They are a use of
+// memory that nothing depends on: where an allocation of this library fails,
+// they are given back and it is tried again.  Launches that use them hold the
+// mutex shared, so none is enqueued while they are taken away.
+struct SecondBuffers {
+    std::shared_mutex mutex;
+    std::set<lbm_solver *> held;
+};
+SecondBuffers &second_buffers() {
+    static SecondBuffers *b = new SecondBuffers();  // outlives every solver
+    return *b;
+}
+
+// mutex held exclusively
+void drop_second(lbm_solver *s) {
+    (void)hipFree(s->dd2.exchange(nullptr));
+    s->version++;
+    second_buffers().held.erase(s);
+}
 
 int fail(lbm_solver *s, int code, const std::string &msg) { return record(s ? &s->err : nullptr, code, msg); }
 int gfail(lbm_group *g, int code, const std::string &msg) { return record(g ? &g->err : nullptr, code, msg); }
@@ -497,6 +535,7 @@ int dispatch_storage(int storage, F &&f) {
 void fill_desc(lbm_solver *s) {
     DomDev &d = s->host_desc;
     d.dd = s->dd;
+    d.dd2 = s->dd2;
     d.flags = s->flags;
     d.vel = s->vel;
     d.dens = s->dens;
@@ -525,6 +564,7 @@ int upload_desc(lbm_solver *s) {
     fill_desc(s);
     SCHK(hipMemcpyAsync(s->d_desc, &s->host_desc, sizeof(DomDev), hipMemcpyHostToDevice, s->stream));
     SCHK(hipStreamSynchronize(s->stream));
+    s->desc_dd2 = s->host_desc.dd2;
     s->version++;
     return LBM_OK;
 }
@@ -548,6 +588,116 @@ hipError_t launch_step_kernel(int storage, bool beta, int variant, int lds, int 
     }
 }
 
+hipError_t launch_pair_kernel(int storage, const PairLaunch &L, int ntiles, const DomDev *descs, const PairTile *tiles,
+                              hipStream_t stream, long long *ctr, int flip) {
+    return storage == LBM_STORAGE_F32 ? launch_pair_storage<0>(L, ntiles, descs, tiles, stream, ctr, flip)
+                                      : launch_pair_storage<1>(L, ntiles, descs, tiles, stream, ctr, flip);
+}
+
+// Tiles and launch of the fused pairs over a set of domains of one storage.
+struct PairPlan {
+    std::vector<PairTile> tiles;
+    PairLaunch launch;
+};
+
+// Work-groups of the pair kernel that run at once: the LDS of one takes a compute unit.
+constexpr long long kPairSlots = 256;
+
+PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage) {
+    PairPlan P;
+    // The most work-items whose two LDS planes fit a compute unit (160 KB): the
+    // larger the tile, the smaller its halo's share.  FP32 256^3 in tiles of
+    // 1024 against 512: 336 and 343-375 us a step.
+    P.launch.threads = storage == LBM_STORAGE_F64 ? 512 : 1024;
+    std::vector<PairShape> shape;
+    std::vector<std::pair<long long, int>> planes;  // tiles per plane, planes
+    size_t bytes = 0;
+    for (const lbm_solver *m : doms) {
+        const int *d = m->cfg.dims;
+        shape.push_back(pair_shape(d[0], d[1], P.launch.threads));
+        planes.push_back({shape.back().tiles(), d[2]});
+        bytes += (size_t)19 * m->padded * elem_size(storage);
+    }
+    const int depth = doms.size() == 1 ? pair_depth(planes[0].second, planes[0].first, kPairSlots)
+                                       : pair_depth_of_many(planes, kPairSlots);
+    for (size_t i = 0; i < doms.size(); ++i) {
+        const int *d = doms[i]->cfg.dims;
+        const int chunks = (d[2] + depth - 1) / depth;
+        pair_tiles((int)i, d[0], d[1], d[2], shape[i], (d[2] + chunks - 1) / chunks, P.tiles);
+    }
+    // Tiles dealt to the XCDs in chunks of 8 once the state is well past the
+    // 256 MB memory-side cache, in contiguous eighths below (us a step, chunks
+    // / eighths): FP32 256^3 335 / 356, 192^3 132 / 130; FP64 256^3 563 / 608,
+    // 160^3 147 / 148.
+    P.launch.xcd_map = bytes > ((size_t)600 << 20) ? 8 : -1;
+    return P;
+}
+
+// Whether a step sequence of these domains is better off in pairs.  In place
+// against pairs, us a step of a cube: FP32 LES 64^3 8.7 / 10.3, 72^3 10.4 /
+// 10.8, 80^3 14.3 / 13.2, 96^3 23.2 / 17.0, 160^3 100.5 / 78.2, 256^3 464 /
+// 336; FP64 LES 48^3 7.7 / 10.0, 64^3 14.1 / 12.9, 96^3 40.7 / 31.6, 160^3 231
+// / 147, 256^3 922 / 563.  Small domains have too few columns to hide a walk's
+// latency.  The two-byte storages move half the bytes with as many
+// instructions, and are bound by those already.
+bool pairs_pay(const std::vector<lbm_solver *> &doms, int storage) {
+    if (elem_size(storage) == 2) return false;
+    long long cells = 0;
+    for (const lbm_solver *m : doms) {
+        if (m->external) return false;  // no memory beyond the caller's
+        cells += m->cells;
+    }
+    return cells >= (storage == LBM_STORAGE_F64 ? 250000 : 480000);
+}
+
+// Gives a solver its second buffer; false if it has to do without.  Half of
+// the device's memory is left to others.
+bool take_second(lbm_solver *s) {
+    SecondBuffers &sb = second_buffers();
+    std::unique_lock<std::shared_mutex> lock(sb.mutex);
+    if (s->dd2) return true;
+    if (s->dd2_refused) return false;
+    const size_t bytes = (size_t)19 * s->padded * elem_size(s->cfg.storage);
+    size_t free_b = 0, total_b = 0;
+    void *p = nullptr;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < bytes + total_b / 2 ||
+        hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        s->dd2_refused = true;
+        return false;
+    }
+    s->dd2 = p;
+    sb.held.insert(s);
+    s->version++;
+    return true;
+}
+
+// Second buffer and tile table of a solver stepped on its own; false: the run
+// steps in place.
+bool solver_pairs_ready(lbm_solver *s) {
+    const std::vector<lbm_solver *> one = {s};
+    if (!pairs_pay(one, s->cfg.storage)) return false;
+    if (!take_second(s)) return false;
+    if (!s->d_pair) {
+        const PairPlan P = plan_pairs(one, s->cfg.storage);
+        if (hipMalloc((void **)&s->d_pair, sizeof(PairTile) * P.tiles.size()) != hipSuccess) {
+            (void)hipGetLastError();
+            s->d_pair = nullptr;
+            return false;
+        }
+        if (hipMemcpyAsync(s->d_pair, P.tiles.data(), sizeof(PairTile) * P.tiles.size(), hipMemcpyHostToDevice,
+                           s->stream) != hipSuccess ||
+            hipStreamSynchronize(s->stream) != hipSuccess) {
+            (void)hipFree(s->d_pair);
+            s->d_pair = nullptr;
+            return false;
+        }
+        s->npair = (int)P.tiles.size();
+        s->pair_launch = P.launch;
+    }
+    return s->desc_dd2 == s->dd2 || upload_desc(s) == LBM_OK;
+}
+
 int launch_step(lbm_solver *s, bool beta) {
     SCHK(launch_step_kernel(s->cfg.storage, beta, s->cfg.kernel_variant, s->cfg.lds_per_block, s->ntiles, s->wg,
                             s->d_desc, s->d_tile, s->stream));
@@ -563,7 +713,7 @@ int ensure_staging(lbm_solver *s, size_t bytes) {
     if (s->staging) SCHK(hipFree(s->staging));
     s->staging = nullptr;
     s->staging_bytes = 0;
-    if (hipMalloc(&s->staging, bytes) != hipSuccess)
+    if (lbm_device_malloc(&s->staging, bytes) != hipSuccess)
         return fail(s, LBM_ERR_OUT_OF_MEMORY, "staging buffer allocation of " + std::to_string(bytes) + " bytes failed");
     s->staging_bytes = bytes;
     return LBM_OK;
@@ -593,6 +743,27 @@ size_t field_elem_bytes(const lbm_solver *s, int field) {
 }
 
 }  // namespace
+
+hipError_t lbm_device_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return e;
+    {
+        SecondBuffers &sb = second_buffers();
+        std::unique_lock<std::shared_mutex> lock(sb.mutex);
+        std::vector<lbm_solver *> here;
+        for (lbm_solver *s : sb.held)
+            if (s->cfg.device == device) here.push_back(s);
+        if (here.empty()) return e;
+        (void)hipDeviceSynchronize();  // launches that still use them
+        for (lbm_solver *s : here) drop_second(s);
+    }
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
+    return e;
+}
 
 // ---- library -----------------------------------------------------------------
 
@@ -752,16 +923,16 @@ static int create_solver(const lbm_solver_config *cfg, void *memory, size_t memo
         s->staging_bytes = L.staging_bytes;
     } else {
         const size_t es = elem_size(c.storage), cs = compute_size(c.storage);
-        if (hipMalloc(&s->dd, (size_t)19 * s->padded * es) != hipSuccess)
+        if (lbm_device_malloc(&s->dd, (size_t)19 * s->padded * es) != hipSuccess)
             return bail(LBM_ERR_OUT_OF_MEMORY, "distribution buffer allocation failed");
-        if (hipMalloc((void **)&s->flags, (size_t)cells) != hipSuccess)
+        if (lbm_device_malloc((void **)&s->flags, (size_t)cells) != hipSuccess)
             return bail(LBM_ERR_OUT_OF_MEMORY, "flag buffer allocation failed");
-        if (c.store_velocity && hipMalloc(&s->vel, (size_t)3 * cells * cs) != hipSuccess)
+        if (c.store_velocity && lbm_device_malloc(&s->vel, (size_t)3 * cells * cs) != hipSuccess)
             return bail(LBM_ERR_OUT_OF_MEMORY, "velocity buffer allocation failed");
-        if (c.store_density && hipMalloc(&s->dens, (size_t)cells * cs) != hipSuccess)
+        if (c.store_density && lbm_device_malloc(&s->dens, (size_t)cells * cs) != hipSuccess)
             return bail(LBM_ERR_OUT_OF_MEMORY, "density buffer allocation failed");
-        if (hipMalloc((void **)&s->d_desc, sizeof(DomDev)) != hipSuccess ||
-            hipMalloc((void **)&s->d_tile, sizeof(int) * (size_t)s->ntiles) != hipSuccess)
+        if (lbm_device_malloc((void **)&s->d_desc, sizeof(DomDev)) != hipSuccess ||
+            lbm_device_malloc((void **)&s->d_tile, sizeof(int) * (size_t)s->ntiles) != hipSuccess)
             return bail(LBM_ERR_OUT_OF_MEMORY, "descriptor allocation failed");
     }
     // all tiles of the single-domain launch belong to domain 0 (a fill
@@ -816,6 +987,11 @@ extern "C" int lbm_solver_destroy(lbm_solver *s) {
         (void)hipFree(s->staging);
     }
     if (s->d_partials) (void)hipFree(s->d_partials);
+    if (s->dd2) {
+        std::unique_lock<std::shared_mutex> lock(second_buffers().mutex);
+        drop_second(s);
+    }
+    if (s->d_pair) (void)hipFree(s->d_pair);
     if (s->own_stream) (void)hipStreamDestroy(s->own_stream);
     delete s;
     return LBM_OK;
@@ -842,7 +1018,7 @@ extern "C" int lbm_solver_colocate(lbm_solver *const *solvers, int n) {
     }
     if (hipSetDevice(device) != hipSuccess) return record(nullptr, LBM_ERR_DEVICE, "hipSetDevice failed");
     void *base = nullptr;
-    if (hipMalloc(&base, total) != hipSuccess)
+    if (lbm_device_malloc(&base, total) != hipSuccess)
         return record(nullptr, LBM_ERR_OUT_OF_MEMORY,
                       "lbm_solver_colocate: allocation of " + std::to_string(total) + " bytes failed");
     SharedBlock *blk = new SharedBlock{base, 0};
@@ -950,7 +1126,23 @@ extern "C" int lbm_solver_simulation_step(lbm_solver *s) {
 extern "C" int lbm_solver_run(lbm_solver *s, int steps) {
     if (!s) return record(nullptr, LBM_ERR_INVALID_ARGUMENT, "null solver");
     if (steps < 0) return fail(s, LBM_ERR_INVALID_ARGUMENT, "steps must be >= 0");
-    for (int i = 0; i < steps; ++i) {
+    int i = 0;
+    if (steps >= 5 && (s->step_counter & 1)) {  // pairs start on a beta step
+        int rc = lbm_solver_simulation_step(s);
+        if (rc) return rc;
+        ++i;
+    }
+    if (steps - i >= 4 && (s->step_counter & 1) == 0 && solver_pairs_ready(s)) {
+        std::shared_lock<std::shared_mutex> lock(second_buffers().mutex);
+        // two pairs at a time: into the second buffer and back
+        for (; s->dd2 && s->dd2 == s->desc_dd2 && steps - i >= 4; i += 4) {
+            for (int flip = 0; flip < 2; ++flip)
+                SCHK(launch_pair_kernel(s->cfg.storage, s->pair_launch, s->npair, s->d_desc, s->d_pair, s->stream,
+                                        nullptr, flip));
+            s->step_counter += 4;
+        }
+    }
+    for (; i < steps; ++i) {
         int rc = lbm_solver_simulation_step(s);
         if (rc) return rc;
     }
@@ -1111,7 +1303,7 @@ extern "C" int lbm_solver_mass_energy(lbm_solver *s, double *mass, double *ke) {
     if (s->partial_count < (size_t)blocks + 1) {
         if (s->d_partials) SCHK(hipFree(s->d_partials));
         s->d_partials = nullptr;
-        if (hipMalloc((void **)&s->d_partials, sizeof(double) * 2 * ((size_t)blocks + 1)) != hipSuccess)
+        if (lbm_device_malloc((void **)&s->d_partials, sizeof(double) * 2 * ((size_t)blocks + 1)) != hipSuccess)
             return fail(s, LBM_ERR_OUT_OF_MEMORY, "reduction buffer allocation failed");
         s->partial_count = (size_t)blocks + 1;
     }
@@ -1264,7 +1456,7 @@ extern "C" int lbm_copy_box(lbm_solver *src, const int src_origin[3], lbm_solver
     if (op.npop == 0) return LBM_OK;
     SCHK(hipStreamSynchronize(src->stream));
     CopyOp *d_op = nullptr;
-    SCHK(hipMalloc((void **)&d_op, sizeof(CopyOp)));
+    SCHK(lbm_device_malloc((void **)&d_op, sizeof(CopyOp)));
     SCHK(hipMemcpyAsync(d_op, &op, sizeof(CopyOp), hipMemcpyHostToDevice, s->stream));
     SCHK(exchange_launch(s->cfg.storage, d_op, 1, (op.cells / op.vec * op.npop + 255) / 256, s->stream));
     SCHK(hipStreamSynchronize(s->stream));
@@ -1470,7 +1662,7 @@ static hipError_t grow_table(T *&ptr, size_t &cap, size_t n) {
         cap = 0;
         if (e != hipSuccess) return e;
     }
-    hipError_t e = hipMalloc((void **)&ptr, sizeof(T) * c);
+    hipError_t e = lbm_device_malloc((void **)&ptr, sizeof(T) * c);
     if (e == hipSuccess) cap = c;
     return e;
 }
@@ -1704,6 +1896,7 @@ extern "C" int lbm_group_destroy(lbm_group *g) {
         (void)hipFree(T.d_chains);
     }
     (void)hipFree(g->d_ctr);
+    (void)hipFree(g->d_pair);
     if (g->stream) (void)hipStreamDestroy(g->stream);
     delete g;
     return LBM_OK;
@@ -1729,6 +1922,7 @@ extern "C" int lbm_group_add_member(lbm_group *g, lbm_solver *s, int *index) {
     s->stream = g->stream;
     g->descs_dirty = true;
     g->plan_built = false;
+    g->npair = 0;
     if (index) *index = (int)g->members.size() - 1;
     return LBM_OK;
 }
@@ -1754,6 +1948,7 @@ extern "C" int lbm_group_remove_member(lbm_group *g, int index) {
     g->comms.swap(kept);
     g->descs_dirty = true;
     g->plan_built = false;
+    g->npair = 0;
     if (upload_desc(m) != LBM_OK) return gfail(g, LBM_ERR_DEVICE, m->err);
     return LBM_OK;
 }
@@ -2005,7 +2200,8 @@ static int group_prepare(lbm_group *g) {
 // tables' addresses (a table that grew was reallocated; its contents are read
 // at replay time and may change in place).
 static std::vector<long long> group_shape(const lbm_group *g) {
-    std::vector<long long> v = {g->wg, g->wg_alpha, g->variant, g->lds, (long long)(uintptr_t)g->d_ctr};
+    std::vector<long long> v = {g->wg, g->wg_alpha, g->variant, g->lds, (long long)(uintptr_t)g->d_ctr,
+                                g->npair, (long long)(uintptr_t)g->d_pair};
     for (const LaunchTables &T : g->lt) {
         v.push_back(T.ntiles);
         v.push_back((long long)(uintptr_t)T.d_descs);
@@ -2074,15 +2270,50 @@ static void group_advance_counters(lbm_group *g, long long before, long long don
     g->step_counter = before + done;
 }
 
-// The graph replaying `pairs` beta+alpha pairs (with their exchanges):
-// captured once per launch shape and pair count, at most kMaxGraphs kept
-// (least recently used dropped first).  Capturing records launches without
-// running them.
+// Whether the next `steps` half-steps (from a beta step) may run as fused
+// pairs: no exchange between the half-steps, second buffers for every member,
+// and no member that freezes on the way (a member frozen already keeps its
+// state; one that freezes between two pairs would keep it in the wrong
+// buffer).  Brings the pair tiles and descriptors up to date.
+static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
+    *ready = false;
+    if (steps < 4 || g->timing || !g->comms.empty() || !pairs_pay(g->members, g->storage)) return LBM_OK;
+    for (const lbm_solver *m : g->members)
+        if (m->stop_at > g->step_counter && m->stop_at < g->step_counter + steps) return LBM_OK;
+    for (lbm_solver *m : g->members)
+        if (!take_second(m)) return LBM_OK;
+    if (!g->npair) {
+        const PairPlan P = plan_pairs(g->members, g->storage);
+        GCHK(grow_table(g->d_pair, g->pair_cap, P.tiles.size()));
+        GCHK(hipMemcpyAsync(g->d_pair, P.tiles.data(), sizeof(PairTile) * P.tiles.size(), hipMemcpyHostToDevice,
+                            g->stream));
+        GCHK(hipStreamSynchronize(g->stream));
+        g->npair = (int)P.tiles.size();
+        g->pair_launch = P.launch;
+    }
+    int rc = group_prepare(g);  // the descriptors carry the second buffers
+    if (rc) return rc;
+    *ready = true;
+    return LBM_OK;
+}
+
+// Two beta+alpha pairs of every member: into the second buffers and back.
+static int group_launch_two_pairs(lbm_group *g) {
+    for (int flip = 0; flip < 2; ++flip)
+        GCHK(launch_pair_kernel(g->storage, g->pair_launch, g->npair, g->lt[0].d_descs, g->d_pair, g->stream, g->d_ctr,
+                                flip));
+    return LBM_OK;
+}
+
+// The graph replaying `pairs` beta+alpha pairs (with their exchanges, or
+// fused two by two): captured once per launch shape and pair count, at most
+// kMaxGraphs kept (least recently used dropped first).  Capturing records
+// launches without running them.
 static constexpr size_t kMaxGraphs = 4;
-static int group_graph(lbm_group *g, int pairs, hipGraphExec_t *out) {
+static int group_graph(lbm_group *g, int pairs, bool fused, hipGraphExec_t *out) {
     if (!g->graphs.empty() && g->graph_shape != group_shape(g)) group_drop_graph(g);
     for (auto &e : g->graphs)
-        if (e.pairs == pairs) {
+        if (e.pairs == pairs && e.fused == fused) {
             e.used = ++g->graph_clock;
             *out = e.exec;
             return LBM_OK;
@@ -2096,9 +2327,15 @@ static int group_graph(lbm_group *g, int pairs, hipGraphExec_t *out) {
     }
     GCHK(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
     int rc = LBM_OK;
-    for (int p = 0; p < pairs && !rc; ++p) {
+    for (int p = 0; p < pairs && !rc;) {
+        if (fused && pairs - p >= 2) {
+            rc = group_launch_two_pairs(g);
+            p += 2;
+            continue;
+        }
         rc = group_launch_half(g, true, false);
         if (!rc) rc = group_launch_half(g, false, false);
+        ++p;
     }
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(g->stream, &graph);
@@ -2114,16 +2351,17 @@ static int group_graph(lbm_group *g, int pairs, hipGraphExec_t *out) {
         GCHK(ei);
     }
     if (g->graphs.empty()) g->graph_shape = group_shape(g);
-    g->graphs.push_back({pairs, graph, exec, ++g->graph_clock});
+    g->graphs.push_back({pairs, fused, graph, exec, ++g->graph_clock});
     g->graphs_captured += 1;
     *out = exec;
     return LBM_OK;
 }
 
 // Walks `steps` half-steps from the group's counter: graph replays of up to
-// graph_pairs pairs where a pair starts on a beta step, single eager launches
-// otherwise.  With run == false it only captures the graphs the walk needs.
-static int group_walk(lbm_group *g, int steps, bool run, int *done_out) {
+// graph_pairs pairs where a pair starts on a beta step, eager launches
+// otherwise; fused pairs where `fused`.  With run == false it only captures
+// the graphs the walk needs.
+static int group_walk(lbm_group *g, int steps, bool run, bool fused, int *done_out) {
     long long h = g->step_counter;
     int done = 0;
     while (done < steps) {
@@ -2132,7 +2370,7 @@ static int group_walk(lbm_group *g, int steps, bool run, int *done_out) {
         if (g->use_graph && !g->timing && beta && pairs >= 1) {
             const int P = std::min(pairs, g->graph_pairs);
             hipGraphExec_t exec = nullptr;
-            int rc = group_graph(g, P, &exec);
+            int rc = group_graph(g, P, fused && P >= 2, &exec);
             if (rc) return rc;
             if (run) {
                 GCHK(hipGraphLaunch(exec, g->stream));
@@ -2140,6 +2378,14 @@ static int group_walk(lbm_group *g, int steps, bool run, int *done_out) {
             }
             h += 2 * P;
             done += 2 * P;
+        } else if (fused && beta && pairs >= 2) {
+            if (run) {
+                int rc = group_launch_two_pairs(g);
+                if (rc) return rc;
+                g->eager_half_steps += 4;
+            }
+            h += 4;
+            done += 4;
         } else {
             if (run) {
                 int rc = group_launch_half(g, beta, g->timing);
@@ -2152,6 +2398,18 @@ static int group_walk(lbm_group *g, int steps, bool run, int *done_out) {
     }
     *done_out = done;
     return LBM_OK;
+}
+
+// group_walk with the choice between fused pairs and half-steps; launches
+// that use second buffers hold them.
+static int group_advance(lbm_group *g, int steps, bool run, int *done) {
+    bool fused = false;
+    int rc = group_pairs_ready(g, steps, &fused);
+    if (rc) return rc;
+    if (!fused) return group_walk(g, steps, run, false, done);
+    std::shared_lock<std::shared_mutex> lock(second_buffers().mutex);
+    for (const lbm_solver *m : g->members) fused = fused && m->dd2;
+    return group_walk(g, steps, run, fused, done);
 }
 
 extern "C" int lbm_group_step(lbm_group *g, int steps) {
@@ -2167,7 +2425,7 @@ extern "C" int lbm_group_step(lbm_group *g, int steps) {
         return LBM_OK;
     }
     int done = 0;
-    rc = group_walk(g, steps, true, &done);
+    rc = group_advance(g, steps, true, &done);
     if (rc) return rc;
     group_advance_counters(g, before, done);
     return LBM_OK;
@@ -2180,7 +2438,7 @@ extern "C" int lbm_group_prepare_steps(lbm_group *g, int steps) {
     int rc = group_prepare(g);
     if (rc || g->lt[0].ntiles == 0) return rc;
     int done = 0;
-    return group_walk(g, steps, false, &done);
+    return group_advance(g, steps, false, &done);
 }
 
 extern "C" int lbm_group_get_launch_counts(const lbm_group *g, long long *graph_launches, long long *eager_half_steps,

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "../../include/lbm_capi.h"
+#include "device_memory.hpp"
 #include "launch_shape.hpp"
 
 namespace {
@@ -440,7 +441,7 @@ extern "C" int lbm_server_create(const lbm_server_config *cfg, lbm_server **out)
     s->cfg.max_chunk_steps &= ~1;
     s->t0 = std::chrono::steady_clock::now();
     if (hipSetDevice(cfg->device) != hipSuccess) return LBM_ERR_DEVICE;
-    if (hipMalloc(&s->arena_base, cfg->memory_budget) != hipSuccess) {
+    if (lbm_device_malloc(&s->arena_base, cfg->memory_budget) != hipSuccess) {
         s->arena_base = nullptr;
         return LBM_ERR_OUT_OF_MEMORY;
     }

@@ -1,0 +1,184 @@
+// pair_plan.hpp -- tiles of the fused beta + alpha kernel (pair_kernel).
+// Plain C++: the plan is checked on the CPU.
+#pragma once
+
+#include <algorithm>
+#include <utility>
+#include <vector>
+
+namespace lbm {
+
+#if defined(__HIPCC__)
+#define LBM_PAIR_FN __host__ __device__ __forceinline__
+#else
+#define LBM_PAIR_FN inline
+#endif
+
+// One work-group of the pair kernel: `nz` planes from z0 of a tile in x-y,
+// halo columns included: w x h columns, or, with w == 0, a run of h
+// consecutive positions of rows of X.  `org` is the in-plane linear position
+// of the first column; it may be negative and columns may lie past the plane:
+// positions are linear and wrap at the ends of the domain, as the streaming
+// does.
+struct PairTile {
+    int dom;
+    int org;
+    int z0, nz;
+    int w, h;
+};
+
+// A column of a work-item: its LDS position in the tile (-1: none) and its
+// in-plane linear position.
+struct PairLane {
+    int pos, p;
+};
+
+// LDS positions of one row of a tile
+LBM_PAIR_FN int pair_pitch(const PairTile &P, int X) { return P.w ? P.w : X; }
+
+// The column whose beta work-item t computes: the tile's columns row by row.
+LBM_PAIR_FN PairLane pair_beta_lane(const PairTile &P, int X, int t) {
+    if (P.w == 0) return PairLane{t < P.h ? t : -1, P.org + t};
+    const int ty = t / P.w;
+    return PairLane{ty < P.h ? t : -1, P.org + t - ty * P.w + X * ty};
+}
+
+// The inner column whose alpha work-item t computes.
+LBM_PAIR_FN PairLane pair_alpha_lane(const PairTile &P, int X, int t) {
+    if (P.w == 0) return PairLane{t < P.h - 2 * (X + 1) ? t + X + 1 : -1, P.org + t + X + 1};
+    const int iw = P.w - 2, ty = t / iw, tx = t - ty * iw;
+    return PairLane{ty < P.h - 2 ? (ty + 1) * P.w + tx + 1 : -1, P.org + tx + 1 + X * (ty + 1)};
+}
+
+// Whether a gather of the tile leaves the domain and wraps: those of planes
+// z0-1 .. z0+nz reach planes z0-2 .. z0+nz+1.
+LBM_PAIR_FN bool pair_wraps(const PairTile &P, int X, int XY, int cells) {
+    const int last = P.org + (P.w == 0 ? P.h - 1 : P.w - 1 + X * (P.h - 1));
+    return P.org - 1 - X + XY * (P.z0 - 2) < 0 || last + 1 + X + XY * (P.z0 + P.nz + 1) >= cells;
+}
+
+// How a pair launch is made.
+struct PairLaunch {
+    int threads = 0;
+    int xcd_map = 0;  // see step_kernel
+};
+
+// Shape of a domain's tiles in x-y for work-groups of `threads`.
+struct PairShape {
+    bool run = false;  // runs of consecutive positions (pitch X); else rectangles
+    int tx = 0, ty = 0;  // inner columns per tile: tx positions (run), or tx by ty
+    int nx = 0, ny = 0;  // tiles per plane: nx (run), or nx by ny
+    int tiles() const { return run ? nx : nx * ny; }
+    int beta_waves = 0, alpha_waves = 0;  // of a full tile
+};
+
+// A tile computes beta on its inner columns and a halo of one column around
+// them, so the halo is work done twice (and read twice).  Of all tiles that
+// fit the work-group, the fewest wavefronts of beta and alpha per plane, with
+// a price on narrow rows, whose lines are fetched for single columns at their
+// ends: whole rows as runs of consecutive positions (halo X + 1 positions on
+// each side) suit short rows, rectangles long ones.  FP32 256^3, rows of 32,
+// 64 and 128 inner columns: 367, 342 and 315-330 us a step.
+inline PairShape pair_shape(int X, int Y, int threads) {
+    PairShape best;
+    double best_cost = -1;
+    auto take = [&](PairShape s, int inner, int all) {
+        s.alpha_waves = (inner + 63) / 64;
+        s.beta_waves = (all + 63) / 64;
+        if (all > threads || inner < 1) return;
+        const double cost = (double)s.tiles() * (s.beta_waves + s.alpha_waves) * (s.run ? 1.0 : 1.0 + 25.0 / s.tx);
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = s;
+        }
+    };
+    const long long XY = (long long)X * Y;
+    const int len = threads - 2 * (X + 1);
+    if (len >= 1) {
+        PairShape s;
+        s.run = true;
+        s.nx = (int)((XY + len - 1) / len);
+        s.tx = (int)((XY + s.nx - 1) / s.nx);
+        s.ny = 1;
+        take(s, s.tx, s.tx + 2 * (X + 1));
+    }
+    for (int n = 1; n <= X; ++n) {
+        const int tx = (X + n - 1) / n;
+        if (tx < 6 && n > 1) break;
+        PairShape s;
+        s.nx = (X + tx - 1) / tx;
+        s.tx = tx;
+        const int rows = threads / (tx + 2) - 2;  // the most that fit, evened out over the plane
+        if (rows < 1) continue;
+        s.ny = (Y + rows - 1) / rows;
+        s.ty = (Y + s.ny - 1) / s.ny;
+        take(s, s.tx * s.ty, (s.tx + 2) * (s.ty + 2));
+    }
+    return best;
+}
+
+// Planes per work-group: a work-group walks nz + 2 planes (the two at its
+// ends are halo), so long walks waste least, but `slots` work-groups run at
+// once and the last round of them should be full.
+inline int pair_depth(int Z, long long tiles_per_plane, long long slots) {
+    int best = Z;
+    double best_cost = -1.0;
+    for (int n = 1; n <= Z; ++n) {  // chunks along z
+        const int nz = (Z + n - 1) / n;
+        if (n > 1 && (Z + nz - 1) / nz != n) continue;
+        const long long blocks = tiles_per_plane * n;
+        const long long rounds = (blocks + slots - 1) / slots;
+        const double cost = (double)rounds * (nz + 2.0 + 0.5);
+        if (best_cost < 0.0 || cost < best_cost) {
+            best_cost = cost;
+            best = nz;
+        }
+        if (nz == 1) break;
+    }
+    return best;
+}
+
+// The same for many domains in one launch ((tiles per plane, planes) each):
+// the walks are of all lengths and fill the device one after another, so
+// only their number and the length of the last ones matter.
+inline int pair_depth_of_many(const std::vector<std::pair<long long, int>> &planes, long long slots) {
+    int best = 1;
+    double best_cost = -1.0;
+    for (int nz : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128}) {
+        double work = 0.0;
+        for (const auto &p : planes) work += (double)p.first * (p.second + 2.5 * ((p.second + nz - 1) / nz));
+        const double cost = work / (double)slots + 0.7 * (nz + 2.5);
+        if (best_cost < 0.0 || cost < best_cost) {
+            best_cost = cost;
+            best = nz;
+        }
+    }
+    return best;
+}
+
+// Appends the tiles of domain `dom`, x fastest, then y, then z chunks.
+inline void pair_tiles(int dom, int X, int Y, int Z, const PairShape &s, int nz, std::vector<PairTile> &out) {
+    const int XY = X * Y;
+    for (int z0 = 0; z0 < Z; z0 += nz) {
+        const int dz = std::min(nz, Z - z0);
+        if (s.run) {
+            for (int i = 0; i < s.nx; ++i) {
+                const int p0 = i * s.tx, len = std::min(s.tx, XY - p0);
+                if (len <= 0) break;
+                out.push_back(PairTile{dom, p0 - X - 1, z0, dz, 0, len + 2 * (X + 1)});
+            }
+            continue;
+        }
+        for (int j = 0; j < s.ny; ++j) {
+            const int y0 = j * s.ty, ty = std::min(s.ty, Y - y0);
+            if (ty <= 0) break;
+            for (int i = 0; i < s.nx; ++i) {
+                const int x0 = i * s.tx, tx = std::min(s.tx, X - x0);
+                if (tx <= 0) break;
+                out.push_back(PairTile{dom, x0 - 1 + X * (y0 - 1), z0, dz, tx + 2, ty + 2});
+            }
+        }
+    }
+}
+
+}  // namespace lbm
