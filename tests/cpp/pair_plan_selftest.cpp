@@ -81,6 +81,43 @@ static void check(int X, int Y, int Z, int threads, int nz) {
     for (long long g = 0; g < cells; ++g) CHECK(seen[(size_t)g] == 1, "%dx%dx%d cell %lld stored %d times", X, Y, Z, g, seen[(size_t)g]);
 }
 
+// the boxes of the small-domain kernel
+static void check_box(int X, int Y, int Z, int held, int threads, int resident) {
+    const BoxShape b = box_shape(X, Y, Z, held, threads, resident, 256);
+    CHECK(b.cost > 0, "%dx%dx%d: no boxes", X, Y, Z);
+    if (b.cost <= 0) return;
+    std::vector<PairTile> tiles;
+    box_tiles(0, X, Y, Z, b, tiles);
+    const long long XY = (long long)X * Y, cells = XY * Z;
+    std::vector<unsigned char> seen((size_t)cells, 0);
+    for (const PairTile &P : tiles) {
+        const bool wrap = pair_wraps(P, X, (int)XY, (int)cells);
+        const int w = P.w, wh = P.w * P.h, n = wh * (P.nz + 2);
+        CHECK(n <= held, "%dx%dx%d box of %d cells, %d held", X, Y, Z, n, held);
+        auto cell = [&](int e) {
+            const int tz = e / wh, r = e - tz * wh, ty = r / w;
+            return P.org + r - ty * w + (long long)X * ty + XY * (P.z0 - 1 + tz);
+        };
+        for (int e = 0; e < n; ++e)
+            for (int dz = -1; dz <= 1; ++dz)
+                for (int dy = -1; dy <= 1; ++dy)
+                    for (int dx = -1; dx <= 1; ++dx) {
+                        const long long g = cell(e) + XY * dz + X * dy + dx, v = wrap ? wrap1(g, cells) : g;
+                        CHECK(v >= 0 && v < cells, "%dx%dx%d box gather %lld (wrap %d)", X, Y, Z, g, (int)wrap);
+                    }
+        const int iw = P.w - 2, iwh = iw * (P.h - 2);
+        for (int e = 0; e < iwh * P.nz; ++e) {
+            const int tz = e / iwh, r = e - tz * iwh, ty = r / iw, tx = r - ty * iw;
+            const int pos = (tz + 1) * wh + (ty + 1) * w + tx + 1;
+            const long long g = P.org + tx + 1 + (long long)X * (ty + 1) + XY * (P.z0 + tz);
+            CHECK(pos - (1 + w + wh) >= 0 && pos + 1 + w + wh < n, "box neighbour out of LDS");
+            CHECK(cell(pos) == g && g >= 0 && g < cells, "box store %lld", g);
+            if (g >= 0 && g < cells) seen[(size_t)g]++;
+        }
+    }
+    for (long long g = 0; g < cells; ++g) CHECK(seen[(size_t)g] == 1, "%dx%dx%d box cell %lld stored %d times", X, Y, Z, g, seen[(size_t)g]);
+}
+
 int main() {
     srand(7);
     for (int threads : {256, 512, 1024})
@@ -96,6 +133,17 @@ int main() {
             const int nz = pair_depth(Z, tiles, 512);
             CHECK(nz >= 1 && nz <= Z, "depth %d of %d", nz, Z);
         }
+    for (int held : {704, 1056, 2048})
+        for (int k = 0; k < 40; ++k)
+            check_box(3 + rand() % (k % 4 ? 40 : 200), 3 + rand() % (k % 5 ? 40 : 150), 3 + rand() % (k % 3 ? 30 : 100), held,
+                      held == 704 ? 704 : held / 2, 1 + k % 2);
+    for (int held : {704, 1056, 2048}) {
+        check_box(3, 3, 3, held, 512, 1);
+        check_box(500, 3, 3, held, 512, 1);
+        check_box(3, 500, 3, held, 512, 1);
+        check_box(3, 3, 900, held, 512, 1);
+        check_box(64, 64, 64, held, 512, 1);
+    }
     if (fails) {
         printf("%d failures\n", fails);
         return 1;

@@ -44,7 +44,19 @@ def same(a, b):
     return all(np.array_equal(x, y, equal_nan=isinstance(x, np.ndarray) and x.dtype.kind == "f") for x, y in zip(a, b))
 
 
-# FP32 sequences pair up from 480,000 cells, FP64 from 250,000: rows as runs of
+# Small domains pair up in boxes: one box, single cells over a full box, flat,
+# long and ragged ones.
+BOXES = [
+    ((3, 3, 3), _capi.STORAGE_F32, {}),
+    ((24, 20, 16), _capi.STORAGE_F32, {"outputs": True, "grav": (1e-4, -2e-4, 3e-5)}),
+    ((48, 48, 48), _capi.STORAGE_F32, {"bc": (8, 8, 1, 1, 8, 1)}),
+    ((200, 20, 20), _capi.STORAGE_F32, {"forcing": 1, "grav": (1e-5, 0.0, 0.0), "outputs": True}),
+    ((9, 90, 4), _capi.STORAGE_F32, {"cs": 0.0}),
+    ((3, 4, 151), _capi.STORAGE_F64, {}),
+    ((31, 33, 29), _capi.STORAGE_F64, {"outputs": True}),
+    ((130, 9, 11), _capi.STORAGE_F64, {"cs": 0.0, "bc": (1, 1, 8, 8, 1, 1)}),
+]
+# FP32 sequences walk planes in pairs from 480,000 cells, FP64 from 250,000: rows as runs of
 # positions (short rows), rectangles with one, even and ragged tile columns,
 # domains thinner than a walk, rows longer than a work-group.
 CASES = [
@@ -60,7 +72,7 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("dims,storage,kw", CASES)
+@pytest.mark.parametrize("dims,storage,kw", CASES + BOXES)
 @pytest.mark.parametrize("first,steps", [(0, 4), (0, 7), (1, 12)])
 def test_pairs_equal_single_steps(dims, storage, kw, first, steps):
     print(f"case: {dims} storage {storage} {kw} from {first}, {steps} steps", flush=True)

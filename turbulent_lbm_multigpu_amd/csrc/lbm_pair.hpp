@@ -189,8 +189,8 @@ __device__ __forceinline__ void loads_arrived() { __builtin_amdgcn_s_waitcnt(0x0
 // best launch shape), FP64 563 against 922 (863).
 template <int ST, int NT>
 __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
-    pair_kernel(const DomDev *__restrict__ doms, const PairTile *__restrict__ tiles, int flip, int xcd_map,
-                long long *ctr) {
+    pair_kernel(const DomDev *__restrict__ doms, const PairTile *__restrict__ tiles, void *second, int flip,
+                int xcd_map, long long *ctr) {
     using SP = Storage<ST>;
     using T = typename SP::T;
     using U = typename SP::U;
@@ -228,8 +228,9 @@ __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
     const int alpha_from = (int)scalar_word(__ballot(stores) != 0ull ? 2u : (unsigned)nz + 2u);  // first plane of the walk with an alpha
     if (!stores) LA = pair_alpha_lane(P, X, 0);
     const int pitch = pair_pitch(P, X);
-    gchar *const from = (gchar *)(flip ? D->dd2 : D->dd);
-    const PairBuf dst = pair_buf((gchar *)(flip ? D->dd : D->dd2));
+    void *const two = second ? second : D->dd2;
+    gchar *const from = (gchar *)(flip ? two : D->dd);
+    const PairBuf dst = pair_buf((gchar *)(flip ? D->dd : two));
     const guchar *const flags = (const guchar *)D->flags;
     const bool wrap = pair_wraps(P, X, XY, cells);
     int g = LB.p + XY * (z0 - 1);  // the cell whose populations are loaded next
@@ -345,18 +346,125 @@ __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
     }
 }
 
-// Launch of pair_kernel: beta and alpha of every tile from buffer `flip` (0: dd, 1: dd2) into the other.
+// The two sizes of the small-domain kernel: cells (halo included) its LDS
+// holds, and its work-items.  The small one takes a box in one pass; the large
+// one fills the 160 KB of LDS.
+constexpr int kBoxSmall = 704;
+constexpr int box_large(int storage) { return storage == 1 ? 1056 : 2048; }
+constexpr int box_threads(int storage) { return storage == 1 ? 512 : 1024; }
+
+// The pair of a small domain: a work-group computes the beta of a whole box,
+// halo included, into LDS, and after one barrier the alpha of its inner cells.
+// Small domains are bound by what a launch costs (about 4 us of dispatch,
+// first loads and drain, whatever the kernel does); this halves their number,
+// at the price of the beta on the halo (1.8 to 3 times the inner cells).
+template <int ST, int NT, int CELLS>
+__global__ void __launch_bounds__(NT)
+    pair_box_kernel(const DomDev *__restrict__ doms, const PairTile *__restrict__ tiles, void *second, int flip,
+                    int xcd_map, long long *ctr) {
+    using SP = Storage<ST>;
+    using T = typename SP::T;
+    using U = typename SP::U;
+    extern __shared__ char smem[];
+    U *const lds = (U *)smem;                                     // beta's values: [19][CELLS]
+    uint8_t *const lds_flags = (uint8_t *)smem + 19 * CELLS * sizeof(U);  // and flags: [CELLS]
+    long long h = 0;  // as in pair_kernel
+    if (ctr) {
+        h = ctr[flip];
+        if (blockIdx.x == 0 && threadIdx.x == 0) ctr[flip ^ 1] = h + 2;
+    }
+    const int nb = (int)gridDim.x;
+    const int t = xcd_map < 0 ? xcd_tile((int)blockIdx.x, nb) : (int)blockIdx.x;
+    const PairTile P = tiles[t];
+    const DomDev *D = doms + P.dom;
+    if (h >= D->stop_at) return;  // uniform: before any barrier
+    const PairPhys<T> phys = pair_phys<T>(D);
+    const bool macros = D->store_velocity || D->store_density;
+    const int X = D->nx, XY = D->nx * D->ny, cells = (int)D->cells;
+    void *const two = second ? second : D->dd2;
+    const PairBuf src = pair_buf((gchar *)(flip ? two : D->dd)), dst = pair_buf((gchar *)(flip ? D->dd : two));
+    const guchar *const flags = (const guchar *)D->flags;
+    const bool wrap = pair_wraps(P, X, XY, cells);
+    const int w = P.w, wh = P.w * P.h, n = wh * (P.nz + 2);
+    for (int e = (int)threadIdx.x; e < n; e += NT) {
+        const int tz = e / wh, r = e - tz * wh, ty = r / w;
+        const int g = P.org + r - ty * w + X * ty + XY * (P.z0 - 1 + tz);
+        PairRows rows;
+        pair_plane<SP>(rows, 0, g - XY, X, cells, wrap);
+        pair_plane<SP>(rows, 1, g, X, cells, wrap);
+        pair_plane<SP>(rows, 2, g + XY, X, cells, wrap);
+        U u[19];
+        pair_gather_cell<SP>(src, rows, g, X, XY, cells, wrap, u);
+        const int flag = (int)flags[(unsigned)(wrap ? wrap_idx(g, cells) : g)];
+        T f[19], vx, vy, vz, dens;
+#pragma unroll
+        for (int i = 0; i < 19; ++i) f[i] = kin<SP>(u[i], i);
+        const PairPhys<T> ph = pair_phys_here(phys);
+        const bool bounce = pair_update<T, true, SP::kShifted>(f, flag, ph, false, vx, vy, vz, dens);
+        U *const even = lds + e + (bounce ? CELLS : 0), *const odd = lds + e + (bounce ? 0 : CELLS);
+#pragma unroll
+        for (int i = 0; i < 18; i += 2) {
+            even[i * CELLS] = kout<SP>(f[i], i);
+            odd[i * CELLS] = kout<SP>(f[i + 1], i + 1);
+        }
+        lds[18 * CELLS + e] = kout<SP>(f[18], 18);
+        lds_flags[e] = (uint8_t)flag;
+    }
+    __syncthreads();
+    const int iw = P.w - 2, iwh = iw * (P.h - 2), ni = iwh * P.nz;
+    for (int e = (int)threadIdx.x; e < ni; e += NT) {
+        const int tz = e / iwh, r = e - tz * iwh, ty = r / iw, tx = r - ty * iw;
+        const int pos = (tz + 1) * wh + (ty + 1) * w + tx + 1;
+        T f[19], vx, vy, vz, dens;
+#pragma unroll
+        for (int i = 0; i < 19; ++i) f[i] = kin<SP>(lds[i * CELLS + pos - (ex(i) + w * ey(i) + wh * ez(i))], i);
+        const int flag = lds_flags[pos];
+        const PairPhys<T> ph = pair_phys_here(phys);
+        const bool keep = pair_update<T, false, SP::kShifted>(f, flag, ph, macros, vx, vy, vz, dens);
+        const unsigned gs = (unsigned)(P.org + tx + 1 + X * (ty + 1) + XY * (P.z0 + tz));
+        const unsigned own = cell_base(gs) * SP::kBytes;
+        constexpr unsigned pop = kBlk * SP::kBytes;
+        const unsigned even = own + (keep ? 0u : pop), odd = own + (keep ? pop : 0u);
+#pragma unroll
+        for (int i = 0; i < 18; i += 2) {
+            buf_st<U>(dst, even, (unsigned)i * pop, kout<SP>(f[i], i));
+            buf_st<U>(dst, odd, (unsigned)i * pop, kout<SP>(f[i + 1], i + 1));
+        }
+        buf_st<U>(dst, own, 18u * pop, kout<SP>(f[18], 18));
+        if (macros && flag != kFlagGhost) store_macros<T>(D, gs, cells, vx, vy, vz, dens);
+    }
+}
+
+// Launch of a pair kernel: beta and alpha of every tile from one buffer into
+// the other (flip 0: from dd, 1: back into it).  `second`: the second buffer
+// of a single domain, or null for the one its descriptor names.
 template <int ST>
 hipError_t launch_pair_storage(const PairLaunch &L, int ntiles, const DomDev *descs, const PairTile *tiles,
-                               hipStream_t stream, long long *ctr, int flip) {
-    constexpr int NT = ST == 1 ? 512 : 1024;
-    if (L.threads != NT) return hipErrorInvalidValue;
-    constexpr int lds = 2 * NT * (19 * (int)Storage<ST>::kBytes + 1);
-    static const hipError_t attr = hipFuncSetAttribute((const void *)pair_kernel<ST, NT>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (attr != hipSuccess) return attr;
-    pair_kernel<ST, NT><<<ntiles, NT, lds, stream>>>(descs, tiles, flip, L.xcd_map, ctr);
-    return hipGetLastError();
+                               void *second, hipStream_t stream, long long *ctr, int flip) {
+    constexpr int per_cell = 19 * (int)Storage<ST>::kBytes + 1;
+    auto go = [&](auto *kernel, int threads, int lds, hipError_t attr) -> hipError_t {
+        if (attr != hipSuccess) return attr;
+        if (L.threads != threads) return hipErrorInvalidValue;
+        kernel<<<ntiles, threads, lds, stream>>>(descs, tiles, second, flip, L.xcd_map, ctr);
+        return hipGetLastError();
+    };
+#define LBM_PAIR_GO(kernel, threads, lds)                                                                            \
+    do {                                                                                                              \
+        static const hipError_t attr =                                                                                \
+            hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);               \
+        return go(kernel, threads, lds, attr);                                                                        \
+    } while (0)
+    if (L.box_cells == kBoxSmall) LBM_PAIR_GO((pair_box_kernel<ST, kBoxSmall, kBoxSmall>), kBoxSmall, kBoxSmall * per_cell);
+    if (L.box_cells > 0) {
+        if (L.box_cells != box_large(ST)) return hipErrorInvalidValue;
+        LBM_PAIR_GO((pair_box_kernel<ST, box_threads(ST), box_large(ST)>), box_threads(ST), box_large(ST) * per_cell);
+    }
+    if constexpr (ST < 2) {
+        constexpr int NT = ST == 1 ? 512 : 1024;
+        LBM_PAIR_GO((pair_kernel<ST, NT>), NT, 2 * NT * per_cell);
+    }
+    return hipErrorInvalidValue;
+#undef LBM_PAIR_GO
 }
 
 }  // namespace lbm

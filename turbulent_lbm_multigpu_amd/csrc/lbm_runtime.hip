@@ -364,6 +364,15 @@ struct SharedBlock {
     int refs = 0;
 };
 
+// One device allocation holding the second buffers (fused pairs) of one solver
+// or of the members of a group.
+struct SecondBlock {
+    void *base = nullptr;
+    size_t bytes = 0;
+    int device = 0;
+    int refs = 0;
+};
+
 struct lbm_solver {
     lbm_solver_config cfg{};
     long long cells = 0, padded = 0;  // padded: cells rounded up to whole layout blocks
@@ -387,10 +396,11 @@ struct lbm_solver {
     // second buffer of the fused pairs, allocated by the first run that takes
     // them; another thread may take it away between runs (SecondBuffers)
     std::atomic<void *> dd2{nullptr};
-    void *desc_dd2 = nullptr;    // the one d_desc names
     bool dd2_refused = false;    // there was no memory for it
+    SecondBlock *dd2_block = nullptr;
     PairTile *d_pair = nullptr;  // tiles of the fused pairs of a run on its own
-    int npair = 0;
+    std::vector<PairTile> pair_tiles;  // their copy on the host (the upload reads it)
+    int npair = 0;               // their number; 0: not planned yet, -1: this domain steps in place
     PairLaunch pair_launch{};
     std::atomic<unsigned> version{0};  // bumps when kernel parameters change
     lbm_group *group = nullptr;
@@ -491,21 +501,43 @@ namespace {
 // The second buffers of the solvers that took fused pairs.  They are a use of
 // memory that nothing depends on: where an allocation of this library fails,
 // they are given back and it is tried again.  Launches that use them hold the
-// mutex shared, so none is enqueued while they are taken away.
+// mutex shared, so none is enqueued while they are taken away.  The buffers of
+// the last few destroyed solvers are kept for the next ones (an allocation
+// costs a short run more than it gains): at most kSpares, kSpareBytes in all.
 struct SecondBuffers {
+    static constexpr size_t kSpares = 8, kSpareBytes = (size_t)4 << 30;
     std::shared_mutex mutex;
     std::set<lbm_solver *> held;
+    std::vector<SecondBlock *> spares;  // oldest first
+    size_t spare_bytes = 0;
 };
 SecondBuffers &second_buffers() {
     static SecondBuffers *b = new SecondBuffers();  // outlives every solver
     return *b;
 }
 
-// mutex held exclusively
+// The following hold the mutex exclusively.
+void free_spares(SecondBuffers &sb, size_t keep_bytes, size_t keep) {
+    while (!sb.spares.empty() && (sb.spare_bytes > keep_bytes || sb.spares.size() > keep)) {
+        SecondBlock *b = sb.spares.front();
+        (void)hipFree(b->base);
+        sb.spare_bytes -= b->bytes;
+        sb.spares.erase(sb.spares.begin());
+        delete b;
+    }
+}
 void drop_second(lbm_solver *s) {
-    (void)hipFree(s->dd2.exchange(nullptr));
+    SecondBuffers &sb = second_buffers();
+    if (!s->dd2) return;
+    s->dd2 = nullptr;
     s->version++;
-    second_buffers().held.erase(s);
+    sb.held.erase(s);
+    SecondBlock *b = s->dd2_block;
+    s->dd2_block = nullptr;
+    if (--b->refs > 0) return;
+    sb.spares.push_back(b);
+    sb.spare_bytes += b->bytes;
+    free_spares(sb, SecondBuffers::kSpareBytes, SecondBuffers::kSpares);
 }
 
 int fail(lbm_solver *s, int code, const std::string &msg) { return record(s ? &s->err : nullptr, code, msg); }
@@ -564,7 +596,6 @@ int upload_desc(lbm_solver *s) {
     fill_desc(s);
     SCHK(hipMemcpyAsync(s->d_desc, &s->host_desc, sizeof(DomDev), hipMemcpyHostToDevice, s->stream));
     SCHK(hipStreamSynchronize(s->stream));
-    s->desc_dd2 = s->host_desc.dd2;
     s->version++;
     return LBM_OK;
 }
@@ -589,9 +620,9 @@ hipError_t launch_step_kernel(int storage, bool beta, int variant, int lds, int 
 }
 
 hipError_t launch_pair_kernel(int storage, const PairLaunch &L, int ntiles, const DomDev *descs, const PairTile *tiles,
-                              hipStream_t stream, long long *ctr, int flip) {
-    return storage == LBM_STORAGE_F32 ? launch_pair_storage<0>(L, ntiles, descs, tiles, stream, ctr, flip)
-                                      : launch_pair_storage<1>(L, ntiles, descs, tiles, stream, ctr, flip);
+                              void *second, hipStream_t stream, long long *ctr, int flip) {
+    return storage == LBM_STORAGE_F32 ? launch_pair_storage<0>(L, ntiles, descs, tiles, second, stream, ctr, flip)
+                                      : launch_pair_storage<1>(L, ntiles, descs, tiles, second, stream, ctr, flip);
 }
 
 // Tiles and launch of the fused pairs over a set of domains of one storage.
@@ -603,8 +634,60 @@ struct PairPlan {
 // Work-groups of the pair kernel that run at once: the LDS of one takes a compute unit.
 constexpr long long kPairSlots = 256;
 
+long long cells_of(const std::vector<lbm_solver *> &doms) {
+    long long n = 0;
+    for (const lbm_solver *m : doms) n += m->cells;
+    return n;
+}
+
+// Whether pair_kernel's walks are the better way through a step sequence of
+// these domains.  In place against walks, us a step of a cube: FP32 LES 64^3
+// 8.7 / 10.3, 72^3 10.4 / 10.8, 80^3 14.3 / 13.2, 96^3 23.2 / 17.0, 160^3
+// 100.5 / 78.2, 256^3 464 / 336; FP64 LES 48^3 7.7 / 10.0, 64^3 14.1 / 12.9,
+// 96^3 40.7 / 31.6, 160^3 231 / 147, 256^3 922 / 563.  Small domains have too
+// few columns to hide a walk's latency.  The two-byte storages move half the
+// bytes with as many instructions, and are bound by those already.
+bool walks_pay(const std::vector<lbm_solver *> &doms, int storage) {
+    return elem_size(storage) >= 4 && cells_of(doms) >= (storage == LBM_STORAGE_F64 ? 250000 : 480000);
+}
+
+// The boxes of a domain too small for walks, and whether they beat the
+// half-step launches: both sides as fitted to measurements of cubes from 16^3
+// to 72^3 and of flat and long domains, us a pair of a run on its own.  In
+// place / boxes: FP32 LES 16^3 8.8 / 6.0, 32^3 9.2 / 7.5, 48^3 11.8 / 10.4,
+// 64^3 17.2 / 16.1, 33x50x97 14.4 / 14.8; FP64 16^3 10.6 / 6.6, 32^3 11.6 /
+// 8.6, 48^3 15.6 / 15.0, 56^3 19.6 / 24.  Above the cell limits runs of several
+// solvers side by side fill the device, and the halo's share decides: three
+// 64^3 BGK runs at once, 6.06 us a step each in place, 6.44 in boxes.
+bool boxes_pay(const lbm_solver *m, int storage, BoxShape *shape, PairLaunch *launch) {
+    const int *d = m->cfg.dims;
+    const bool f64 = storage == LBM_STORAGE_F64;
+    if (elem_size(storage) == 2 || m->cells > (f64 ? 70000 : 120000)) return false;
+    const int large = box_large(f64), threads = box_threads(f64);
+    const BoxShape a = box_shape(d[0], d[1], d[2], kBoxSmall, kBoxSmall, f64 ? 1 : 2, kPairSlots);
+    const BoxShape b = box_shape(d[0], d[1], d[2], large, threads, 1, kPairSlots);
+    const bool small = b.cost < 0.0 || (a.cost >= 0.0 && a.cost <= b.cost);
+    *shape = small ? a : b;
+    launch->box_cells = small ? kBoxSmall : large;
+    launch->threads = small ? kBoxSmall : threads;
+    launch->xcd_map = -1;
+    if (shape->cost < 0.0) return false;
+    const double boxes = f64 ? 3.5 + 0.30 * shape->cost : 3.0 + 0.21 * shape->cost;
+    const double in_place = f64 ? 9.0 + 6.8e-5 * (double)m->cells : 8.2 + 3.4e-5 * (double)m->cells;
+    return boxes < 0.96 * in_place;
+}
+
+// Tiles and launch of fused pairs over the domains; none: they step in place.
 PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage) {
     PairPlan P;
+    if (!walks_pay(doms, storage)) {
+        BoxShape shape;
+        if (doms.size() == 1 && boxes_pay(doms[0], storage, &shape, &P.launch)) {
+            const int *d = doms[0]->cfg.dims;
+            box_tiles(0, d[0], d[1], d[2], shape, P.tiles);
+        }
+        return P;
+    }
     // The most work-items whose two LDS planes fit a compute unit (160 KB): the
     // larger the tile, the smaller its halo's share.  FP32 256^3 in tiles of
     // 1024 against 512: 336 and 343-375 us a step.
@@ -633,69 +716,93 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage) {
     return P;
 }
 
-// Whether a step sequence of these domains is better off in pairs.  In place
-// against pairs, us a step of a cube: FP32 LES 64^3 8.7 / 10.3, 72^3 10.4 /
-// 10.8, 80^3 14.3 / 13.2, 96^3 23.2 / 17.0, 160^3 100.5 / 78.2, 256^3 464 /
-// 336; FP64 LES 48^3 7.7 / 10.0, 64^3 14.1 / 12.9, 96^3 40.7 / 31.6, 160^3 231
-// / 147, 256^3 922 / 563.  Small domains have too few columns to hide a walk's
-// latency.  The two-byte storages move half the bytes with as many
-// instructions, and are bound by those already.
-bool pairs_pay(const std::vector<lbm_solver *> &doms, int storage) {
-    if (elem_size(storage) == 2) return false;
-    long long cells = 0;
-    for (const lbm_solver *m : doms) {
-        if (m->external) return false;  // no memory beyond the caller's
-        cells += m->cells;
+// The device made current for a scope (a run does not need it current, an allocation does).
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int device) {
+        int now = 0;
+        if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) before = now;
     }
-    return cells >= (storage == LBM_STORAGE_F64 ? 250000 : 480000);
-}
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
 
-// Gives a solver its second buffer; false if it has to do without.  Half of
-// the device's memory is left to others.
-bool take_second(lbm_solver *s) {
+// Gives the solvers (of one device) their second buffers, those without one
+// in a block together; false if they have to do without.  Half of the device's
+// memory is left to others.
+bool take_seconds(const std::vector<lbm_solver *> &solvers) {
     SecondBuffers &sb = second_buffers();
     std::unique_lock<std::shared_mutex> lock(sb.mutex);
-    if (s->dd2) return true;
-    if (s->dd2_refused) return false;
-    const size_t bytes = (size_t)19 * s->padded * elem_size(s->cfg.storage);
-    size_t free_b = 0, total_b = 0;
-    void *p = nullptr;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < bytes + total_b / 2 ||
-        hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        s->dd2_refused = true;
-        return false;
+    auto size_of = [](const lbm_solver *s) {
+        return ((size_t)19 * s->padded * elem_size(s->cfg.storage) + 255) & ~(size_t)255;
+    };
+    std::vector<lbm_solver *> without;
+    size_t bytes = 0;
+    for (lbm_solver *s : solvers) {
+        if (s->dd2) continue;
+        if (s->dd2_refused) return false;
+        without.push_back(s);
+        bytes += size_of(s);
     }
-    s->dd2 = p;
-    sb.held.insert(s);
-    s->version++;
+    if (without.empty()) return true;
+    const int device = without[0]->cfg.device;
+    const OnDevice on(device);
+    SecondBlock *b = nullptr;
+    for (auto it = sb.spares.rbegin(); it != sb.spares.rend(); ++it) {
+        if ((*it)->device != device || (*it)->bytes < bytes || (*it)->bytes > 2 * bytes) continue;
+        b = *it;
+        sb.spare_bytes -= b->bytes;
+        sb.spares.erase(std::next(it).base());
+        break;
+    }
+    if (!b) {
+        size_t free_b = 0, total_b = 0;
+        void *p = nullptr;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < bytes + total_b / 2 ||
+            hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            for (lbm_solver *s : without) s->dd2_refused = true;
+            return false;
+        }
+        b = new SecondBlock{p, bytes, device, 0};
+    }
+    size_t off = 0;
+    for (lbm_solver *s : without) {
+        s->dd2_block = b;
+        b->refs++;
+        s->dd2 = (char *)b->base + off;
+        off += size_of(s);
+        sb.held.insert(s);
+        s->version++;
+    }
     return true;
 }
 
 // Second buffer and tile table of a solver stepped on its own; false: the run
 // steps in place.
 bool solver_pairs_ready(lbm_solver *s) {
-    const std::vector<lbm_solver *> one = {s};
-    if (!pairs_pay(one, s->cfg.storage)) return false;
-    if (!take_second(s)) return false;
+    if (s->external || s->npair < 0) return false;  // no memory beyond the caller's
     if (!s->d_pair) {
-        const PairPlan P = plan_pairs(one, s->cfg.storage);
+        PairPlan P = plan_pairs({s}, s->cfg.storage);
+        s->npair = P.tiles.empty() ? -1 : (int)P.tiles.size();
+        if (s->npair < 0) return false;
+        const OnDevice on(s->cfg.device);
         if (hipMalloc((void **)&s->d_pair, sizeof(PairTile) * P.tiles.size()) != hipSuccess) {
             (void)hipGetLastError();
             s->d_pair = nullptr;
             return false;
         }
-        if (hipMemcpyAsync(s->d_pair, P.tiles.data(), sizeof(PairTile) * P.tiles.size(), hipMemcpyHostToDevice,
-                           s->stream) != hipSuccess ||
-            hipStreamSynchronize(s->stream) != hipSuccess) {
+        s->pair_tiles.swap(P.tiles);
+        if (hipMemcpyAsync(s->d_pair, s->pair_tiles.data(), sizeof(PairTile) * s->pair_tiles.size(),
+                           hipMemcpyHostToDevice, s->stream) != hipSuccess) {
             (void)hipFree(s->d_pair);
             s->d_pair = nullptr;
             return false;
         }
-        s->npair = (int)P.tiles.size();
         s->pair_launch = P.launch;
     }
-    return s->desc_dd2 == s->dd2 || upload_desc(s) == LBM_OK;
+    return take_seconds({s});
 }
 
 int launch_step(lbm_solver *s, bool beta) {
@@ -756,9 +863,10 @@ hipError_t lbm_device_malloc(void **p, size_t bytes) {
         std::vector<lbm_solver *> here;
         for (lbm_solver *s : sb.held)
             if (s->cfg.device == device) here.push_back(s);
-        if (here.empty()) return e;
+        if (here.empty() && sb.spares.empty()) return e;
         (void)hipDeviceSynchronize();  // launches that still use them
         for (lbm_solver *s : here) drop_second(s);
+        free_spares(sb, 0, 0);
     }
     e = hipMalloc(p, bytes);
     if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
@@ -1135,9 +1243,9 @@ extern "C" int lbm_solver_run(lbm_solver *s, int steps) {
     if (steps - i >= 4 && (s->step_counter & 1) == 0 && solver_pairs_ready(s)) {
         std::shared_lock<std::shared_mutex> lock(second_buffers().mutex);
         // two pairs at a time: into the second buffer and back
-        for (; s->dd2 && s->dd2 == s->desc_dd2 && steps - i >= 4; i += 4) {
+        for (void *two = s->dd2; two && steps - i >= 4; i += 4) {
             for (int flip = 0; flip < 2; ++flip)
-                SCHK(launch_pair_kernel(s->cfg.storage, s->pair_launch, s->npair, s->d_desc, s->d_pair, s->stream,
+                SCHK(launch_pair_kernel(s->cfg.storage, s->pair_launch, s->npair, s->d_desc, s->d_pair, two, s->stream,
                                         nullptr, flip));
             s->step_counter += 4;
         }
@@ -2277,11 +2385,12 @@ static void group_advance_counters(lbm_group *g, long long before, long long don
 // buffer).  Brings the pair tiles and descriptors up to date.
 static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
     *ready = false;
-    if (steps < 4 || g->timing || !g->comms.empty() || !pairs_pay(g->members, g->storage)) return LBM_OK;
+    if (steps < 4 || g->timing || !g->comms.empty() || !walks_pay(g->members, g->storage)) return LBM_OK;
+    for (const lbm_solver *m : g->members)
+        if (m->external) return LBM_OK;
     for (const lbm_solver *m : g->members)
         if (m->stop_at > g->step_counter && m->stop_at < g->step_counter + steps) return LBM_OK;
-    for (lbm_solver *m : g->members)
-        if (!take_second(m)) return LBM_OK;
+    if (!take_seconds(g->members)) return LBM_OK;
     if (!g->npair) {
         const PairPlan P = plan_pairs(g->members, g->storage);
         GCHK(grow_table(g->d_pair, g->pair_cap, P.tiles.size()));
@@ -2300,8 +2409,8 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
 // Two beta+alpha pairs of every member: into the second buffers and back.
 static int group_launch_two_pairs(lbm_group *g) {
     for (int flip = 0; flip < 2; ++flip)
-        GCHK(launch_pair_kernel(g->storage, g->pair_launch, g->npair, g->lt[0].d_descs, g->d_pair, g->stream, g->d_ctr,
-                                flip));
+        GCHK(launch_pair_kernel(g->storage, g->pair_launch, g->npair, g->lt[0].d_descs, g->d_pair, nullptr, g->stream,
+                                g->d_ctr, flip));
     return LBM_OK;
 }
 

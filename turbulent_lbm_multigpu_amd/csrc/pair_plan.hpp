@@ -60,6 +60,7 @@ LBM_PAIR_FN bool pair_wraps(const PairTile &P, int X, int XY, int cells) {
 // How a pair launch is made.
 struct PairLaunch {
     int threads = 0;
+    int box_cells = 0;  // > 0: tiles are boxes of at most this many columns x planes (pair_box_kernel)
     int xcd_map = 0;  // see step_kernel
 };
 
@@ -179,6 +180,56 @@ inline void pair_tiles(int dom, int X, int Y, int Z, const PairShape &s, int nz,
             }
         }
     }
+}
+
+// Boxes of the small-domain pair kernel: a work-group holds the beta values of
+// a whole box, halo included, in LDS.  `cells`: what its LDS holds, `threads`
+// its work-items, `resident` how many of it a compute unit runs at once.
+struct BoxShape {
+    int bx = 0, by = 0, bz = 0;  // inner cells per box and axis
+    double cost = -1.0;
+};
+
+// Small domains leave compute units idle or repeat much of beta on the halo;
+// this picks the boxes whose rounds of work-groups take least: the wavefronts
+// of beta and alpha that share a compute unit, plus a load latency for each
+// pass over the box.  Units: a wavefront's collision.
+inline BoxShape box_shape(int X, int Y, int Z, int cells, int threads, int resident, long long units) {
+    // even splits of an axis into boxes of at least `least` cells, at most 32
+    auto splits = [](int n, int least) {
+        std::vector<int> v;
+        for (int k = 1; k <= n; ++k) {
+            const int b = (n + k - 1) / k;
+            if (b < least && k > 1) break;
+            if (b <= 32 && (v.empty() || v.back() != b)) v.push_back(b);
+        }
+        return v;
+    };
+    const std::vector<int> sx = splits(X, 6), sy = splits(Y, 4), sz = splits(Z, 1);
+    BoxShape best;
+    for (int bx : sx)
+        for (int by : sy)
+            for (int bz : sz) {
+                const int ext = (bx + 2) * (by + 2) * (bz + 2);
+                if (ext > cells) continue;
+                const int in = bx * by * bz;
+                const long long blocks = (long long)((X + bx - 1) / bx) * ((Y + by - 1) / by) * ((Z + bz - 1) / bz);
+                const long long per = (blocks + units - 1) / units;  // work-groups a compute unit runs in all
+                const long long rounds = (per + resident - 1) / resident;
+                const double waves = (double)((ext + 63) / 64 + (in + 63) / 64);
+                const double passes = (double)((ext + threads - 1) / threads + (in + threads - 1) / threads);
+                const double cost = (double)per * waves + (double)rounds * 6.0 * passes;
+                if (best.cost < 0.0 || cost < best.cost) best = BoxShape{bx, by, bz, cost};
+            }
+    return best;
+}
+
+inline void box_tiles(int dom, int X, int Y, int Z, const BoxShape &b, std::vector<PairTile> &out) {
+    for (int z0 = 0; z0 < Z; z0 += b.bz)
+        for (int y0 = 0; y0 < Y; y0 += b.by)
+            for (int x0 = 0; x0 < X; x0 += b.bx)
+                out.push_back(PairTile{dom, x0 - 1 + X * (y0 - 1), z0, std::min(b.bz, Z - z0),
+                                       std::min(b.bx, X - x0) + 2, std::min(b.by, Y - y0) + 2});
 }
 
 }  // namespace lbm
