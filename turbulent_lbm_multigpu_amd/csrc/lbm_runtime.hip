@@ -22,6 +22,7 @@
 #include "../../include/lbm_capi.h"
 #include "device_memory.hpp"
 #include "exchange_plan.hpp"
+#include "host_lanes.hpp"
 #include "launch_shape.hpp"
 #include "lbm_device.hpp"
 #include "lbm_pair.hpp"
@@ -122,16 +123,16 @@ __device__ __forceinline__ long long box_cell(const DomDev &D, const Box &b, lon
     return (long long)(b.o[0] + bx) + (long long)D.nx * ((b.o[1] + by) + (long long)D.ny * (b.o[2] + bz));
 }
 
-// Region -> dense [component][box] buffer (copy_buffer_rect,
-// src/cl_programs/copy_buffer_rect.cl:12-52, all components in one launch).
+// `n` cells of a region from its cell `first` -> dense [component][n] buffer
+// (copy_buffer_rect, src/cl_programs/copy_buffer_rect.cl:12-52, all components
+// in one launch).
 template <int ST>
-__global__ void pack_kernel(DomDev D, int field, Box b, void *out) {
+__global__ void pack_kernel(DomDev D, int field, Box b, long long first, long long n, void *out) {
     using SP = Storage<ST>;
     using T = typename SP::T;
-    const long long n = (long long)b.s[0] * b.s[1] * b.s[2];
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const long long g = box_cell(D, b, e);
+    const long long g = box_cell(D, b, first + e);
     if (field == LBM_FIELD_DD_RAW) {  // stored bit patterns, no conversion
         using U = typename SP::U;
         U *o = (U *)out;
@@ -152,15 +153,15 @@ __global__ void pack_kernel(DomDev D, int field, Box b, void *out) {
     }
 }
 
-// Dense buffer -> region; for distributions only populations in `mask`.
+// Dense buffer -> `n` cells of a region from its cell `first`; for
+// distributions only populations in `mask`.
 template <int ST>
-__global__ void unpack_kernel(DomDev D, int field, Box b, const void *in, uint32_t mask) {
+__global__ void unpack_kernel(DomDev D, int field, Box b, long long first, long long n, const void *in, uint32_t mask) {
     using SP = Storage<ST>;
     using T = typename SP::T;
-    const long long n = (long long)b.s[0] * b.s[1] * b.s[2];
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const long long g = box_cell(D, b, e);
+    const long long g = box_cell(D, b, first + e);
     if (field == LBM_FIELD_DD_RAW) {
         using U = typename SP::U;
         const U *s = (const U *)in;
@@ -256,20 +257,20 @@ __device__ __forceinline__ void cell_moments(const DomDev &D, long long g, bool 
     }
 }
 
-template <int ST>
-__global__ void moments_kernel(DomDev D, Box b, int swapped, void *rho_out, void *j_out) {
+// rho and j of `n` cells of a region from its cell `first`, as [4][n] of O
+// (the compute type, or float from any storage).
+template <int ST, typename O>
+__global__ void moments_kernel(DomDev D, Box b, long long first, long long n, int swapped, O *out) {
     using T = typename Storage<ST>::T;
-    const long long n = (long long)b.s[0] * b.s[1] * b.s[2];
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const long long g = box_cell(D, b, e);
+    const long long g = box_cell(D, b, first + e);
     double r, a, bb, c;
     cell_moments<ST>(D, g, swapped != 0, r, a, bb, c);
-    ((T *)rho_out)[e] = (T)r;
-    T *j = (T *)j_out;
-    j[e] = (T)a;
-    j[n + e] = (T)bb;
-    j[2 * n + e] = (T)c;
+    out[e] = (O)(T)r;
+    out[n + e] = (O)(T)a;
+    out[2 * n + e] = (O)(T)bb;
+    out[3 * n + e] = (O)(T)c;
 }
 
 // FP64 mass and kinetic energy over FLUID cells, first pass: one partial
@@ -389,8 +390,7 @@ struct lbm_solver {
     DomDev *d_desc = nullptr;  // single-domain launch descriptor
     int *d_tile = nullptr;
     int ntiles = 0;
-    void *staging = nullptr;
-    size_t staging_bytes = 0;
+    size_t staging_bytes = 0;  // largest transfer of a solver in caller-provided memory
     double *d_partials = nullptr;
     size_t partial_count = 0;
     // second buffer of the fused pairs, allocated by the first run that takes
@@ -811,20 +811,24 @@ int launch_step(lbm_solver *s, bool beta) {
     return LBM_OK;
 }
 
-int ensure_staging(lbm_solver *s, size_t bytes) {
-    if (s->staging_bytes >= bytes) return LBM_OK;
-    if (s->external)
-        return fail(s, LBM_ERR_CAPACITY,
-                    "a solver in caller-provided memory has " + std::to_string(s->staging_bytes) +
-                        " staging bytes; this transfer needs " + std::to_string(bytes) + ": transfer it in regions");
-    if (s->staging) SCHK(hipFree(s->staging));
-    s->staging = nullptr;
-    s->staging_bytes = 0;
-    if (lbm_device_malloc(&s->staging, bytes) != hipSuccess)
-        return fail(s, LBM_ERR_OUT_OF_MEMORY, "staging buffer allocation of " + std::to_string(bytes) + " bytes failed");
-    s->staging_bytes = bytes;
-    return LBM_OK;
+// Transfers go through pinned lanes and need no device memory, but a solver in
+// caller-provided memory keeps to the size of its staging area, as documented.
+int check_staging(lbm_solver *s, size_t bytes) {
+    if (!s->external || s->staging_bytes >= bytes) return LBM_OK;
+    return fail(s, LBM_ERR_CAPACITY,
+                "a solver in caller-provided memory has " + std::to_string(s->staging_bytes) +
+                    " staging bytes; this transfer needs " + std::to_string(bytes) + ": transfer it in regions");
 }
+
+// What move_fields returned, as a status of the solver.
+int moved(lbm_solver *s, hipError_t e, const char *what) {
+    if (e == hipSuccess) return LBM_OK;
+    if (e == hipErrorOutOfMemory)
+        return fail(s, LBM_ERR_OUT_OF_MEMORY, std::string(what) + ": no pinned host memory for the transfer");
+    return fail(s, LBM_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
+}
+
+unsigned blocks_of(long long n) { return (unsigned)((n + 255) / 256); }
 
 int check_box(lbm_solver *s, const int *origin, const int *size, Box &b) {
     for (int a = 0; a < 3; ++a) {
@@ -837,6 +841,16 @@ int check_box(lbm_solver *s, const int *origin, const int *size, Box &b) {
     }
     return LBM_OK;
 }
+
+// The host arrays of a field's components, one after the other.
+struct FieldArrays {
+    int comps;
+    size_t elem;
+    char *at[19];
+    FieldArrays(void *base, long long n, int comps_, size_t elem_) : comps(comps_), elem(elem_) {
+        for (int i = 0; i < comps; ++i) at[i] = (char *)base + (size_t)i * (size_t)n * elem;
+    }
+};
 
 int field_components(int field) {
     return (field == LBM_FIELD_DD || field == LBM_FIELD_DD_RAW) ? 19 : field == LBM_FIELD_VELOCITY ? 3 : 1;
@@ -1027,7 +1041,6 @@ static int create_solver(const lbm_solver_config *cfg, void *memory, size_t memo
         s->dens = c.store_density ? base + L.dens : nullptr;
         s->d_desc = (DomDev *)(base + L.desc);
         s->d_tile = (int *)(base + L.tile);
-        s->staging = base + L.staging;
         s->staging_bytes = L.staging_bytes;
     } else {
         const size_t es = elem_size(c.storage), cs = compute_size(c.storage);
@@ -1080,7 +1093,6 @@ extern "C" int lbm_solver_destroy(lbm_solver *s) {
     if (s->group) return fail(s, LBM_ERR_STATE, "destroy the group before its member solvers");
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     if (s->block) {
-        (void)hipFree(s->staging);  // allocated on its own when a transfer needed it
         if (--s->block->refs == 0) {
             (void)hipFree(s->block->base);
             delete s->block;
@@ -1092,7 +1104,6 @@ extern "C" int lbm_solver_destroy(lbm_solver *s) {
         (void)hipFree(s->dens);
         (void)hipFree(s->d_desc);
         (void)hipFree(s->d_tile);
-        (void)hipFree(s->staging);
     }
     if (s->d_partials) (void)hipFree(s->d_partials);
     if (s->dd2) {
@@ -1303,18 +1314,19 @@ extern "C" int lbm_solver_store(lbm_solver *s, int field, const int origin[3], c
     if (rc) return rc;
     const long long n = (long long)b.s[0] * b.s[1] * b.s[2];
     const size_t bytes = (size_t)n * field_components(field) * field_elem_bytes(s, field);
-    rc = ensure_staging(s, bytes);
+    rc = check_staging(s, bytes);
     if (rc) return rc;
-    rc = dispatch_storage(s->cfg.storage, [&](auto st) -> int {
+    return dispatch_storage(s->cfg.storage, [&](auto st) -> int {
         constexpr int ST = decltype(st)::value;
-        pack_kernel<ST><<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->host_desc, field, b, s->staging);
-        SCHK(hipGetLastError());
-        return LBM_OK;
+        const FieldArrays host(host_dst, n, field_components(field), field_elem_bytes(s, field));
+        return moved(s, move_fields<true>(s->cfg.device, s->stream, n, host.comps, host.elem, host.at,
+                                          [&](long long first, long long count, void *pinned) {
+                                              pack_kernel<ST><<<blocks_of(count), 256, 0, s->stream>>>(
+                                                  s->host_desc, field, b, first, count, pinned);
+                                              return hipGetLastError();
+                                          }),
+                     "store");
     });
-    if (rc) return rc;
-    SCHK(hipMemcpyAsync(host_dst, s->staging, bytes, hipMemcpyDeviceToHost, s->stream));
-    SCHK(hipStreamSynchronize(s->stream));
-    return LBM_OK;
 }
 
 extern "C" int lbm_solver_set(lbm_solver *s, int field, const int origin[3], const int size[3], const void *host_src,
@@ -1333,24 +1345,25 @@ extern "C" int lbm_solver_set(lbm_solver *s, int field, const int origin[3], con
     const long long n = (long long)b.s[0] * b.s[1] * b.s[2];
     if (field == LBM_FIELD_FLAGS) {
         const int32_t *fl = (const int32_t *)host_src;
-        for (long long i = 0; i < n; ++i)
-            if (fl[i] < 0 || fl[i] > 255)
-                return fail(s, LBM_ERR_INVALID_ARGUMENT, "flag values must be in [0, 255]");
+        unsigned over = 0;
+        for (long long i = 0; i < n; ++i) over |= (unsigned)fl[i] & ~255u;
+        if (over) return fail(s, LBM_ERR_INVALID_ARGUMENT, "flag values must be in [0, 255]");
     }
     const size_t bytes = (size_t)n * field_components(field) * field_elem_bytes(s, field);
-    rc = ensure_staging(s, bytes);
+    rc = check_staging(s, bytes);
     if (rc) return rc;
-    SCHK(hipMemcpyAsync(s->staging, host_src, bytes, hipMemcpyHostToDevice, s->stream));
     const uint32_t mask = norm_mask(norm);
-    rc = dispatch_storage(s->cfg.storage, [&](auto st) -> int {
+    return dispatch_storage(s->cfg.storage, [&](auto st) -> int {
         constexpr int ST = decltype(st)::value;
-        unpack_kernel<ST><<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->host_desc, field, b, s->staging, mask);
-        SCHK(hipGetLastError());
-        return LBM_OK;
+        const FieldArrays host((void *)host_src, n, field_components(field), field_elem_bytes(s, field));
+        return moved(s, move_fields<false>(s->cfg.device, s->stream, n, host.comps, host.elem, host.at,
+                                           [&](long long first, long long count, void *pinned) {
+                                               unpack_kernel<ST><<<blocks_of(count), 256, 0, s->stream>>>(
+                                                   s->host_desc, field, b, first, count, pinned, mask);
+                                               return hipGetLastError();
+                                           }),
+                     "set");
     });
-    if (rc) return rc;
-    SCHK(hipStreamSynchronize(s->stream));
-    return LBM_OK;
 }
 
 extern "C" int lbm_solver_velocity_checksum(lbm_solver *s, float *out) {
@@ -1470,6 +1483,23 @@ extern "C" int lbm_solver_mass_energy_noalloc(lbm_solver *s, double *mass, doubl
     return mass_energy_passes(s, ptr, (int)blocks, mass, ke);
 }
 
+namespace {
+
+// rho and the components of j of a region into four host arrays of O
+template <int ST, typename O>
+int moments_out(lbm_solver *s, const Box &b, long long n, char *const *host) {
+    const int swapped = (s->step_counter % 2) == 0;
+    return moved(s, move_fields<true>(s->cfg.device, s->stream, n, 4, sizeof(O), host,
+                                      [&](long long first, long long count, void *pinned) {
+                                          moments_kernel<ST, O><<<blocks_of(count), 256, 0, s->stream>>>(
+                                              s->host_desc, b, first, count, swapped, (O *)pinned);
+                                          return hipGetLastError();
+                                      }),
+                 "moments");
+}
+
+}  // namespace
+
 extern "C" int lbm_solver_moments(lbm_solver *s, const int origin[3], const int size[3], void *host_rho, void *host_j) {
     if (!s || !host_rho || !host_j || (origin && !size)) return record(nullptr, LBM_ERR_INVALID_ARGUMENT, "null argument");
     Box b;
@@ -1477,22 +1507,24 @@ extern "C" int lbm_solver_moments(lbm_solver *s, const int origin[3], const int 
     if (rc) return rc;
     const long long n = (long long)b.s[0] * b.s[1] * b.s[2];
     const size_t cs = compute_size(s->cfg.storage);
-    rc = ensure_staging(s, (size_t)n * 4 * cs);
+    rc = check_staging(s, (size_t)n * 4 * cs);
     if (rc) return rc;
-    const int swapped = (s->step_counter % 2) == 0;
-    char *base = (char *)s->staging;
-    rc = dispatch_storage(s->cfg.storage, [&](auto st) -> int {
-        constexpr int ST = decltype(st)::value;
-        moments_kernel<ST><<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->host_desc, b, swapped, base,
-                                                                                 base + (size_t)n * cs);
-        SCHK(hipGetLastError());
-        return LBM_OK;
+    char *const host[4] = {(char *)host_rho, (char *)host_j, (char *)host_j + (size_t)n * cs,
+                           (char *)host_j + 2 * (size_t)n * cs};
+    return dispatch_storage(s->cfg.storage, [&](auto st) -> int {
+        return moments_out<decltype(st)::value, typename Storage<decltype(st)::value>::T>(s, b, n, host);
     });
+}
+
+int lbm_solver_moments_float(lbm_solver *s, float *rho, float *j) {
+    Box b;
+    const int rc = check_box(s, nullptr, nullptr, b);
     if (rc) return rc;
-    SCHK(hipMemcpyAsync(host_rho, base, (size_t)n * cs, hipMemcpyDeviceToHost, s->stream));
-    SCHK(hipMemcpyAsync(host_j, base + (size_t)n * cs, (size_t)n * 3 * cs, hipMemcpyDeviceToHost, s->stream));
-    SCHK(hipStreamSynchronize(s->stream));
-    return LBM_OK;
+    const long long n = s->cells;
+    char *const host[4] = {(char *)rho, (char *)j, (char *)(j + n), (char *)(j + 2 * n)};
+    return dispatch_storage(s->cfg.storage, [&](auto st) -> int {
+        return moments_out<decltype(st)::value, float>(s, b, n, host);
+    });
 }
 
 extern "C" int lbm_solver_device_pointers(lbm_solver *s, void **dd, void **flags, long long *block_cells) {
@@ -1585,11 +1617,10 @@ double host_unit(uint64_t seed, uint64_t key) {
     return (double)(host_mix64(seed ^ host_mix64(key)) >> 11) * (1.0 / 9007199254740992.0);
 }
 
-__global__ void mark_obstacles_kernel(DomDev D, const uint8_t *solid, Box b) {
-    const long long n = (long long)b.s[0] * b.s[1] * b.s[2];
+__global__ void mark_obstacles_kernel(DomDev D, const uint8_t *solid, Box b, long long first, long long n) {
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n || !solid[e]) return;
-    const long long g = box_cell(D, b, e);
+    const long long g = box_cell(D, b, first + e);
     const uint8_t f = D.flags[g];
     if (f == kFlagFluid) D.flags[g] = (uint8_t)kFlagObstacle;
 }
@@ -1653,13 +1684,16 @@ extern "C" int lbm_solver_place_spheres(lbm_solver *s, uint64_t seed, double fil
             for (int x = 0; x < s->cfg.dims[0]; ++x)
                 local[(size_t)(x + (long long)s->cfg.dims[0] * (y + (long long)s->cfg.dims[1] * z))] =
                     solid[(size_t)((ko[0] + x) + KX * ((ko[1] + y) + KY * (long long)(ko[2] + z)))];
-    int rc = ensure_staging(s, (size_t)n);
+    int rc = check_staging(s, (size_t)n);
     if (rc) return rc;
-    SCHK(hipMemcpyAsync(s->staging, local.data(), (size_t)n, hipMemcpyHostToDevice, s->stream));
-    mark_obstacles_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->host_desc, (const uint8_t *)s->staging, b);
-    SCHK(hipGetLastError());
-    SCHK(hipStreamSynchronize(s->stream));
-    return LBM_OK;
+    char *const host[1] = {(char *)local.data()};
+    return moved(s, move_fields<false>(s->cfg.device, s->stream, n, 1, 1, host,
+                                       [&](long long first, long long count, void *pinned) {
+                                           mark_obstacles_kernel<<<blocks_of(count), 256, 0, s->stream>>>(
+                                               s->host_desc, (const uint8_t *)pinned, b, first, count);
+                                           return hipGetLastError();
+                                       }),
+                 "place_spheres");
 }
 
 // ---- device copy bandwidth (calibration of the roofline) --------------------

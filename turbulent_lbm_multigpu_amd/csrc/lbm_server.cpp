@@ -20,7 +20,9 @@
 #include <deque>
 #include <map>
 #include <memory>
+#include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/lbm_capi.h"
@@ -81,7 +83,8 @@ struct Case {
     long long steps_done = 0;
     long long cells = 0;
     double submit_s = 0, admit_s = 0, done_s = 0;
-    std::vector<float> rho, j;
+    std::unique_ptr<float[]> fields;  // rho[cells], j[3][cells]
+    size_t fields_floats = 0;         // its size
     std::string error;  // why a FAILED case failed
 };
 
@@ -146,6 +149,8 @@ struct lbm_server {
     std::deque<Case *> queue;
     std::vector<Case *> ready;   // initialised, joining at the next chunk boundary
     std::vector<Case *> retiring;
+    std::vector<std::pair<std::unique_ptr<float[]>, size_t>> spare_results;  // oldest first
+    size_t spare_floats = 0;
     std::deque<long long> done_order;
     bool inflight = false;
     long long next_id = 1;
@@ -164,6 +169,8 @@ struct lbm_server {
 };
 
 namespace {
+
+constexpr size_t kSpareResults = 64, kSpareFloats = (size_t)64 << 20;  // 256 MB
 
 int active_count(const lbm_server *s) {
     int n = 0;
@@ -310,38 +317,52 @@ int pool_join(lbm_server *s, Case *c, bool *stuck) {
     return LBM_OK;
 }
 
-// rho and j of the whole case, z-slab by z-slab through the solver's staging
-// area (one face of 19 values holds the 4 moment values of >= 4 planes).
-int case_readback(lbm_server *s, Case *c) {
-    const int X = c->c.dims[0], Y = c->c.dims[1], Z = c->c.dims[2];
-    const size_t plane = (size_t)X * Y;
-    const bool f64 = c->c.storage == LBM_STORAGE_F64;
-    c->rho.resize((size_t)c->cells);
-    c->j.resize((size_t)c->cells * 3);
-    const int slab = 4;
-    std::vector<double> rb, jb;
-    std::vector<float> rf, jf;
-    for (int z0 = 0; z0 < Z; z0 += slab) {
-        const int nz = std::min(slab, Z - z0);
-        const int o[3] = {0, 0, z0}, sz[3] = {X, Y, nz};
-        const size_t n = plane * nz;
-        int rc;
-        if (f64) {
-            rb.resize(n);
-            jb.resize(3 * n);
-            rc = lbm_solver_moments(c->solver, o, sz, rb.data(), jb.data());
-        } else {
-            rf.resize(n);
-            jf.resize(3 * n);
-            rc = lbm_solver_moments(c->solver, o, sz, rf.data(), jf.data());
-        }
-        if (rc) return s->fail_lib(rc, "readback", lbm_solver_error(c->solver));
-        const size_t at = plane * z0;
-        for (size_t i = 0; i < n; ++i) c->rho[at + i] = f64 ? (float)rb[i] : rf[i];
-        for (int a = 0; a < 3; ++a)
-            for (size_t i = 0; i < n; ++i)
-                c->j[(size_t)a * c->cells + at + i] = f64 ? (float)jb[a * n + i] : jf[a * n + i];
+// Room for a case's results: the smallest kept block that holds them (touching
+// fresh pages costs more than the copy), else a new one.
+void results_take(lbm_server *s, Case *c) {
+    const size_t want = (size_t)c->cells * 4;
+    auto best = s->spare_results.end();
+    for (auto it = s->spare_results.begin(); it != s->spare_results.end(); ++it)
+        if (it->second >= want && it->second <= 4 * want &&
+            (best == s->spare_results.end() || it->second < best->second))
+            best = it;
+    if (best != s->spare_results.end()) {
+        c->fields = std::move(best->first);
+        c->fields_floats = best->second;
+        s->spare_floats -= best->second;
+        s->spare_results.erase(best);
+        return;
     }
+    c->fields.reset(new float[want]);
+    c->fields_floats = want;
+}
+
+// A fetched case's block is kept for the next results, at most kSpareResults
+// and kSpareFloats in all.
+void results_give(lbm_server *s, Case *c) {
+    if (!c->fields || c->fields_floats > kSpareFloats) return;
+    try {
+        s->spare_results.reserve(kSpareResults + 1);
+    } catch (const std::bad_alloc &) {
+        return;
+    }
+    s->spare_floats += c->fields_floats;
+    s->spare_results.emplace_back(std::move(c->fields), c->fields_floats);
+    while (s->spare_results.size() > kSpareResults || s->spare_floats > kSpareFloats) {
+        s->spare_floats -= s->spare_results.front().second;
+        s->spare_results.erase(s->spare_results.begin());
+    }
+}
+
+// rho and j of the whole case to the host.
+int case_readback(lbm_server *s, Case *c) {
+    try {
+        results_take(s, c);
+    } catch (const std::bad_alloc &) {
+        return s->fail(LBM_ERR_OUT_OF_MEMORY, "readback: no host memory for the results");
+    }
+    const int rc = lbm_solver_moments_float(c->solver, c->fields.get(), c->fields.get() + c->cells);
+    if (rc) return s->fail_lib(rc, "readback", lbm_solver_error(c->solver));
     if (!case_release(s, c)) return s->fail(LBM_ERR_STATE, "readback: the case's solver cannot be released");
     c->state = LBM_CASE_DONE;
     c->done_s = s->now();
@@ -637,8 +658,10 @@ extern "C" int lbm_server_fetch(lbm_server *s, long long id, float *rho, float *
         return s->fail(LBM_ERR_STATE, why);
     }
     if (c->state != LBM_CASE_DONE) return s->fail(LBM_ERR_STATE, "case not completed");
-    if (rho) std::copy(c->rho.begin(), c->rho.end(), rho);
-    if (j) std::copy(c->j.begin(), c->j.end(), j);
+    const float *f = c->fields.get();
+    if (rho) std::copy(f, f + c->cells, rho);
+    if (j) std::copy(f + c->cells, f + 4 * c->cells, j);
+    results_give(s, c);
     s->cases.erase(it);
     return LBM_OK;
 }
