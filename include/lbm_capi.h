@@ -306,9 +306,9 @@ int lbm_group_get_stream(const lbm_group *g, void **stream);
 /* ---- server: continuous batching of independent cases (new) ------------- */
 /* Cases (cavities, periodic channels) are admitted against a device-memory
  * budget into one arena, stepped together per storage type as members of a
- * group (one fused launch per half-step, graph-replayed chunks), frozen at
- * their own step count and read back while the next chunk runs.  Requests
- * that arrive while others run join at the next chunk boundary.  A case's
+ * group (one fused launch per half-step), frozen at their own step count and
+ * read back while the next chunk runs.  Requests that arrive while others run
+ * join at the next chunk boundary.  A case's
  * result does not depend on what it was batched with: the per-cell
  * arithmetic is the same in every launch shape and membership. */
 typedef struct lbm_server lbm_server;

@@ -5,8 +5,8 @@
 // Resident state lives in one device arena sized by the memory budget, so
 // admitting and retiring cases never allocates or frees device memory (a
 // free would wait for the whole device).  Cases of one storage type are the
-// members of one group: a chunk of K steps is one graph-replayed sequence of
-// fused launches over all of them, and every member carries its own stop, so
+// members of one group: a chunk of K steps is one sequence of fused launches
+// over all of them, and every member carries its own stop, so
 // it freezes at exactly its step count inside the chunk.  Between chunks the
 // frozen members leave the group and newly admitted ones join; while a chunk
 // runs, retired cases are read back and queued cases are initialised on an
@@ -195,10 +195,12 @@ int pool_open(lbm_server *s, int slot) {
     rc = lbm_group_set_exchange_mode(p.g, 1);
     // periodic channel seams inside the step kernel for FP32/FP64, copy launch for FP16/BF16
     if (!rc) rc = lbm_group_set_fused_x(p.g, LBM_FUSED_X_AUTO);
-    // membership changes at most chunk boundaries, and a changed membership
-    // needs new graphs: one captured pair, replayed K/2 times, keeps the
-    // capture cost per chunk small
-    if (!rc) rc = lbm_group_set_graph_pairs(p.g, 1);
+    // Membership changes at most chunk boundaries, and a changed membership
+    // would need new graphs.  Replays of one captured pair leave 8 us between
+    // pairs where launches leave 4, and their captures stand in line with the
+    // host's other work: eight cases of 39^3 to 90^3 took 17.4 ms, launched
+    // eagerly 15.0.
+    if (!rc) rc = lbm_group_set_graph(p.g, 0);
     if (rc) return s->fail_lib(rc, "exchange mode", lbm_group_error(p.g));
     void *st = nullptr;
     lbm_group_get_stream(p.g, &st);
@@ -578,7 +580,7 @@ extern "C" int lbm_server_progress(lbm_server *s, int *completed) {
         }
         case_fail(s, c);
     }
-    // 4. the next chunk, one graph-replayed step sequence per storage
+    // 4. the next chunk, one step sequence per storage
     for (Pool &p : s->pools) {
         if (p.members.empty()) continue;
         if (s->cfg.autotune && !p.tuned) {

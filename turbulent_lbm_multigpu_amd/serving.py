@@ -2,7 +2,7 @@
 
 ``Server`` wraps the native scheduler of the C-ABI (lbm_server_*): cases are
 admitted against a device-memory budget into one arena, stepped per storage
-type as one fused, graph-replayed launch sequence, frozen at their own step
+type as one fused launch sequence, frozen at their own step
 count and read back while the next chunk runs; requests that arrive while
 others are on the device join at the next chunk boundary.
 
