@@ -111,11 +111,19 @@ inline ChainShape chain_shape(int M, int X, int wg) {
 // left partner, then rings.  A chain that does not fit (chain_shape with its
 // members' X) is left out and its members' joins are cleared.
 // A periodic ring of one member in a kernel of packed pairs (two-byte storage,
-// two cells per work-item) keeps its seam inside one wavefront per row
-// (seam_pairs in lbm_device.hpp): rows of an even length of at least 128 cells.
+// two cells per work-item) keeps the seam of each row inside one wavefront
+// (seam_pairs in lbm_device.hpp): rows of an even length of at least 128 cells,
+// so that no wavefront meets two.
 inline bool seam_ring_ok(bool pairs, int X) { return pairs && X % 2 == 0 && X >= 128; }
-// wavefronts per row of such a member: the seam wavefront, then runs of 64 pairs
-inline int seam_waves_per_row(int X) { return 1 + (X / 2 - 64 + 63) / 64; }
+// The order in which such a member's work-items take the NP pairs of a row: as
+// they lie, but with pair 0 right before pair NP - 1, at an even place among all
+// pairs of the domain, so that no wavefront ends between the two.  Place `seam`
+// (NP - 2, or NP - 3 where that is odd) and place 0 change their pairs; with
+// NP - 3, so do the last two places.
+constexpr int seam_place(int row, int NP) { return NP - 2 - ((row * NP + NP) & 1); }
+constexpr int seam_pair_at(int place, int seam, int NP) {
+    return place == 0 ? seam : place == seam ? 0 : seam == NP - 3 && place >= NP - 2 ? 2 * NP - 3 - place : place;
+}
 
 inline std::vector<std::vector<int>> find_chains(std::vector<XJoin> &j, const std::vector<int> &X, int wg,
                                                  bool pairs = false) {

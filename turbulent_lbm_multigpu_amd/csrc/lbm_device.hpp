@@ -248,7 +248,7 @@ struct DomDev {
     double inv_tau, tau0, les_coeff, gx, gy, gz, lid;
     long long stop_at;  // launch half-step index from which this domain stays frozen
     unsigned xmask_a[2];  // slots this domain's x- / x+ ghost layer takes after alpha in a chain tile
-    int seam_wpr;         // > 0: periodic x seam inside the pair kernel, wavefronts per row (seam_pairs)
+    int x_seam;           // periodic x seam inside the pair kernel (seam_pairs)
 };
 
 // ---- fused x chains ----------------------------------------------------------
@@ -896,8 +896,7 @@ __device__ __forceinline__ void cells_vector(gchar *const *pl, unsigned g0, int 
 // block (at any 2-byte alignment: gfx950 serves unaligned dword accesses),
 // two element accesses at a block's last cell.
 typedef __attribute__((address_space(1))) unsigned __attribute__((aligned(2))) gpair;
-__device__ __forceinline__ unsigned pair_ld(const gchar *p, unsigned s) {
-    if ((s & (kBlk - 1u)) != kBlk - 1u) return *(const gpair *)(p + cell_base(s) * 2u);
+__device__ __forceinline__ unsigned pair_ld_split(const gchar *p, unsigned s) {
     return (unsigned)raw_ld<false, unsigned short>(p, cell_base(s) * 2u) |
            ((unsigned)raw_ld<false, unsigned short>(p, cell_base(s + 1u) * 2u) << 16);
 }
@@ -915,53 +914,61 @@ __device__ __forceinline__ void pair_st(gchar *p, unsigned s, unsigned v) {
     raw_st<NT, unsigned short>(p, cell_base(s + 1u) * 2u, (unsigned short)(v >> 16));
 }
 
-// pair_ld / pair_st through the linear wrap W where the run nears a domain end
-__device__ __forceinline__ unsigned pair_ld_w(const gchar *p, int s, int cells, bool wrap) {
-    if (!wrap) return pair_ld(p, (unsigned)s);
+// a pair through the linear wrap W, where the cells near a domain end
+__device__ __forceinline__ unsigned pair_ld_wrap(const gchar *p, int s, int cells) {
     return (unsigned)raw_ld<false, unsigned short>(p, cell_base((unsigned)wrap_idx(s, cells)) * 2u) |
            ((unsigned)raw_ld<false, unsigned short>(p, cell_base((unsigned)wrap_idx(s + 1, cells)) * 2u) << 16);
 }
-__device__ __forceinline__ void pair_st_w(gchar *p, int s, int cells, bool wrap, bool nt, unsigned v) {
-    if (!wrap) {
-        if (nt) pair_st<true>(p, (unsigned)s, v);
-        else pair_st<false>(p, (unsigned)s, v);
-        return;
-    }
+__device__ __forceinline__ void pair_st_wrap(gchar *p, int s, int cells, unsigned v) {
     raw_st<false, unsigned short>(p, cell_base((unsigned)wrap_idx(s, cells)) * 2u, (unsigned short)v);
     raw_st<false, unsigned short>(p, cell_base((unsigned)wrap_idx(s + 1, cells)) * 2u, (unsigned short)(v >> 16));
 }
 
-// Pair runs: a wavefront whose 64 lanes hold the packed pairs of the
-// consecutive cells c0 .. c0+127 (c0 uniform).  Where a shifted run
-// c0 - d_i (gather) or c0 + d_i (scatter) lies in one layout block, lane l's
-// pair of it is the run's wavefront-uniform base plus 4 l bytes: the address
-// costs scalar instructions only, where the per-lane form spends about six
-// vector instructions per access (index, block split, straddle check), for
-// each of beta's 36 shifted accesses.  The two-byte kernels issue vector
-// instructions near the SIMDs' limit, so these count.
-__device__ __forceinline__ bool pair_run_in_block(unsigned c0) { return (c0 & (kBlk - 1u)) <= kBlk - 128u; }
+// Shifted runs: the packed pairs of a wavefront lie in the cells c0 .. c0 +
+// span - 1 (uniform).  Where such a run shifted by -d_i (gather) or d_i
+// (scatter) lies in one layout block, a lane's pair of it is the run's uniform
+// base plus lo = 2 (g - c0) bytes: the address costs scalar instructions only,
+// where the per-lane form spends about six vector instructions per access
+// (index, block split, straddle check), for each of beta's 36 shifted accesses.
+// The two-byte kernels issue vector instructions near the SIMDs' limit, so
+// these count.  Chosen per access: a wavefront with one run across a block's
+// end keeps the others' (384x192x192 FP16 channel: beta 236 -> 214 us).
+struct PairRun {
+    unsigned c0, span, lo;
+};
+__device__ __forceinline__ bool in_one_block(unsigned s0, unsigned span) { return (s0 & (kBlk - 1u)) + span <= kBlk; }
 
-// every gather run (ld) / every scatter run (st) of the wavefront in one block
-__device__ __forceinline__ void pair_runs(unsigned c0, const int *d, bool &ld, bool &st) {
-    ld = st = true;
+// beta's 18 gathered pairs (slot opp(i) at g - d_i) and the own slot 18.  Away
+// from the domain ends every pair is loaded by one instruction; a pair that
+// straddles two blocks, which reads a neighbouring population's first cell
+// there, is loaded again by halves.
+__device__ __forceinline__ void pair_gather(gchar *const *pl, unsigned g, const PairRun &r, const int *d, int cells,
+                                            bool wrap, unsigned *P) {
+    if (wrap) {
 #pragma unroll
-    for (int i = 0; i < 18; ++i) {
-        ld = ld && pair_run_in_block(c0 - (unsigned)d[i]);
-        st = st && pair_run_in_block(c0 + (unsigned)d[i]);
-    }
-}
-
-// beta's 18 gathered pairs (slot opp(i) at g - d_i) and the own slot 18, per
-// lane (pair_ld) or, with `run`, from the runs' uniform bases (lo = 4 l)
-__device__ __forceinline__ void pair_gather(gchar *const *pl, unsigned g, unsigned c0, unsigned lo, bool run,
-                                            const int *d, int cells, bool wrap, unsigned *P) {
-    if (run) {
-#pragma unroll
-        for (int i = 0; i < 18; ++i)
-            P[i] = *(const gpair *)(pl[opp(i)] + (size_t)cell_base(c0 - (unsigned)d[i]) * 2u + lo);
+        for (int i = 0; i < 18; ++i) P[i] = pair_ld_wrap(pl[opp(i)], (int)g - d[i], cells);
     } else {
+        unsigned split = 0;  // gathers that leave a block, uniform
 #pragma unroll
-        for (int i = 0; i < 18; ++i) P[i] = pair_ld_w(pl[opp(i)], (int)g - d[i], cells, wrap);
+        for (int i = 0; i < 18; ++i) {
+            const unsigned s0 = r.c0 - (unsigned)d[i];
+            size_t base = (size_t)cell_base(s0) * 2u;
+            unsigned off = r.lo;
+            if (!in_one_block(s0, r.span)) {
+                base = 0;
+                off = cell_base(g - (unsigned)d[i]) * 2u;
+                split |= 1u << i;
+            }
+            P[i] = *(const gpair *)(pl[opp(i)] + base + off);
+        }
+        if (split) {
+#pragma unroll
+            for (int i = 0; i < 18; ++i)
+                if (split >> i & 1u) {
+                    const unsigned s = g - (unsigned)d[i];
+                    if ((s & (kBlk - 1u)) == kBlk - 1u) P[i] = pair_ld_split(pl[opp(i)], s);
+                }
+        }
     }
     P[18] = raw_ld<false, unsigned>(pl[18], cell_base(g) * 2u);
 }
@@ -969,19 +976,24 @@ __device__ __forceinline__ void pair_gather(gchar *const *pl, unsigned g, unsign
 // beta's 18 scattered pairs (slot q at g + d_q) and the own slot 18; the
 // non-temporal policy only for the e.x = 0 slots at 4-byte alignment
 template <bool NTS>
-__device__ __forceinline__ void pair_scatter(gchar *const *pl, unsigned g, unsigned c0, unsigned lo, bool run,
-                                             const int *d, int cells, bool wrap, const unsigned *P) {
-    if (run) {
+__device__ __forceinline__ void pair_scatter(gchar *const *pl, unsigned g, const PairRun &r, const int *d, int cells,
+                                             bool wrap, const unsigned *P) {
+    if (wrap) {
 #pragma unroll
-        for (int q = 0; q < 18; ++q) {
-            const unsigned s0 = c0 + (unsigned)d[q];
-            gchar *b = pl[q] + (size_t)cell_base(s0) * 2u;
-            if (NTS && ex(q) == 0 && (s0 & 1u) == 0u) raw_st<true, unsigned>(b, lo, P[q]);  // uniform
-            else *(gpair *)(b + lo) = P[q];
-        }
+        for (int q = 0; q < 18; ++q) pair_st_wrap(pl[q], (int)g + d[q], cells, P[q]);
     } else {
 #pragma unroll
-        for (int q = 0; q < 18; ++q) pair_st_w(pl[q], (int)g + d[q], cells, wrap, NTS && ex(q) == 0, P[q]);
+        for (int q = 0; q < 18; ++q) {
+            const unsigned s0 = r.c0 + (unsigned)d[q];
+            if (in_one_block(s0, r.span)) {
+                gchar *b = pl[q] + (size_t)cell_base(s0) * 2u;
+                if (NTS && ex(q) == 0 && (s0 & 1u) == 0u) raw_st<true, unsigned>(b, r.lo, P[q]);  // uniform
+                else *(gpair *)(b + r.lo) = P[q];
+            } else {
+                if (NTS && ex(q) == 0) pair_st<true>(pl[q], g + (unsigned)d[q], P[q]);
+                else pair_st<false>(pl[q], g + (unsigned)d[q], P[q]);
+            }
+        }
     }
     raw_st<NTS, unsigned>(pl[18], cell_base(g) * 2u, P[18]);
 }
@@ -999,15 +1011,11 @@ __device__ __forceinline__ void cells_pair2(gchar *const *pl, unsigned g0, int c
     using T = typename SP::T;
     const unsigned fl = raw_ld<false, unsigned short>((const gchar *)D->flags, g0);
     unsigned P[19];
-    // beta: pair runs when all 64 lanes are here (consecutive pairs from the
-    // lane-0 cell c0; lanes at the domain end take another path)
-    unsigned c0 = g0, lo = 0u;
-    bool rl = false, rs = false;
+    PairRun run{0u, 128u, 0u};
     if (BETA) {
-        c0 = __builtin_amdgcn_readfirstlane(g0);
-        lo = (g0 - c0) * 2u;
-        if (__ballot(1) == ~0ull) pair_runs(c0, d, rl, rs);
-        pair_gather(pl, g0, c0, lo, rl, d, cells, false, P);
+        run.c0 = __builtin_amdgcn_readfirstlane(g0);
+        run.lo = (g0 - run.c0) * 2u;
+        pair_gather(pl, g0, run, d, cells, false, P);
     } else {
         const unsigned own = cell_base(g0) * 2u;
 #pragma unroll
@@ -1038,7 +1046,7 @@ __device__ __forceinline__ void cells_pair2(gchar *const *pl, unsigned g0, int c
     unsigned gs = g0;
     asm volatile("" : "+v"(gs));
     if (BETA) {
-        pair_scatter<NTS>(pl, gs, c0, lo, rs, d, cells, false, P);
+        pair_scatter<NTS>(pl, gs, run, d, cells, false, P);
     } else {
         const unsigned own_st = cell_base(gs) * 2u;
 #pragma unroll
@@ -1211,27 +1219,65 @@ __device__ __forceinline__ void chain_tile(const DomDev *__restrict__ doms, cons
 
 // ---- periodic x seam of one domain, packed pairs ---------------------------
 // A two-byte domain whose x faces are each other's neighbours (a periodic
-// ring of one), stepped with two cells per work-item: every row is split into
-// `seam_wpr` wavefronts, the first holding pairs 0..31 and the row's last 32
-// pairs (cells 0..63 and X-64..X-1), the others the pairs in between.  The
-// x = 0 ghost cell (lane 0, low half) and its sender x = X-2 (lane 63, low
-// half), and the x = X-1 ghost (lane 63, high half) and its sender x = 1
-// (lane 0, high half), are then in one wavefront: the face values move by
-// lane reads, with no LDS, no barrier and no copy launch.  The ghost cells
-// take what the copy exchange would give them: after alpha the slots of
+// ring of one), stepped with two cells per work-item.  The pairs 0 and NP - 1
+// of each row are lanes of one wavefront: the x = 0 ghost cell and its sender
+// x = X-2, and the x = X-1 ghost and its sender x = 1, exchange their face
+// values by lane reads, with no LDS, no barrier and no copy launch.  The ghost
+// cells take what the copy exchange would give them: after alpha the slots of
 // their receiver masks, in beta the populations they scatter into the inner
 // layer (e.x = +1 at x = 0, e.x = -1 at x = X-1).
-template <class SP, bool BETA, bool NTS, bool NTL>
+//
+// Bound by memory, so by whether a wavefront's accesses are whole cache lines:
+//  * SPLIT, rows of a multiple of 128 cells: a row's first wavefront holds its
+//    first and its last 32 pairs (128 bytes each at either end), the others
+//    the runs of 64 in between.  Every line belongs to one wavefront.
+//  * otherwise the wavefronts take the pairs as they lie in memory, over the
+//    ends of rows, except that a row's pair 0 comes right before its last one
+//    (seam_pair_at).  Lines with such a pair are touched by two wavefronts,
+//    which a non-temporal access would send to memory in pieces: the launch's
+//    non-temporal policies don't hold here (200x95x73: alpha 26.8 -> 23.6 us).
+// Split rows of another length leave lanes idle and tear lines: FP16
+// half-steps of 200x95x73 took 32.4 us and take 23.8, 264x192x192 180 -> 143,
+// 140x95x73 25.7 -> 18.7; taken in memory order, 384x192x192 took 200 us,
+// split it takes 172.
+template <class SP, bool BETA, bool NTS, bool NTL, bool SPLIT>
 __device__ __forceinline__ void seam_pairs(const DomDev *__restrict__ D, int tile) {
     using T = typename SP::T;
-    const int X = D->nx, NP = X >> 1, wpr = D->seam_wpr;
+    const int X = D->nx, NP = X >> 1, rows = D->ny * D->nz;
     const int cells = (int)D->cells;
-    const int gw = tile * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6);  // wavefront of the domain
-    const int row = gw / wpr, k = gw - row * wpr;
-    if (row >= D->ny * D->nz) return;  // uniform per wavefront
+    // the wavefront's first place: its row and the place there, uniform
+    const int q0 = 64 * (int)__builtin_amdgcn_readfirstlane(
+                            (unsigned)(tile * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6)));
+    const int row0 = q0 / NP, s0 = q0 - row0 * NP;
+    if (row0 >= rows) return;
     const int l = (int)(threadIdx.x & 63);
-    const int p = k == 0 ? (l < 32 ? l : NP - 64 + l) : 32 + 64 * (k - 1) + l;
-    if (k != 0 && p >= NP - 32) return;  // past the row's interior pairs (never in the first wavefront)
+    int row = row0, p = s0 + l;
+    int first, end;   // the cells that hold its pairs, uniform
+    int lz, le;       // the lanes of pair 0 and of pair NP - 1
+    bool seam;        // ... which it holds
+    if (SPLIT) {
+        p = s0 != 0 ? s0 - 32 + l : l < 32 ? l : NP - 64 + l;
+        seam = s0 == 0;
+        lz = 0;
+        le = 63;
+        first = row0 * X + (s0 != 0 ? 2 * s0 - 64 : 0);
+        end = s0 != 0 ? first + 128 : first + X;
+    } else {
+        if (p >= NP) {  // NP > 64: not past the next row
+            p -= NP;
+            row += 1;
+        }
+        if (row >= rows) return;  // past the last pair
+        const int seam0 = seam_place(row0, NP), seam1 = seam_place(row0 + 1, NP);
+        p = seam_pair_at(p, row == row0 ? seam0 : seam1, NP);
+        const bool own = seam0 >= s0;
+        lz = (own ? seam0 : NP + seam1) - s0;
+        le = lz + 1;
+        seam = lz < 63 && (own || row0 + 1 < rows);
+        // a whole row on the side where a pair is away from its place
+        first = row0 * X + (own && lz < 64 ? 0 : s0 < NP - 1 ? 2 * s0 : X - 4);
+        end = row0 * X + (s0 + 63 >= NP ? X + X : s0 == 0 || s0 + 63 == NP - 2 ? X : 2 * (s0 + 64));
+    }
     const int g = row * X + 2 * p;
     gchar *pl[19];
     {
@@ -1246,7 +1292,7 @@ __device__ __forceinline__ void seam_pairs(const DomDev *__restrict__ D, int til
 #pragma unroll
         for (int i = 0; i < 19; ++i) d[i] = ex(i) + X * ey(i) + XY * ez(i);
         const int dmax = 1 + X + XY;
-        wrap = row * X < dmax || row * X + X + dmax > cells;
+        wrap = row0 * X < dmax || (row0 + 2) * X + dmax > cells;
     } else {
 #pragma unroll
         for (int i = 0; i < 19; ++i) d[i] = 0;
@@ -1254,15 +1300,12 @@ __device__ __forceinline__ void seam_pairs(const DomDev *__restrict__ D, int til
     // the pair's loads and collisions (as cells_pair2, with the linear wrap per half)
     const unsigned fl = raw_ld<false, unsigned short>((const gchar *)D->flags, (unsigned)g);
     unsigned P[19];
-    // beta: pair runs for the wavefronts of consecutive pairs (not the split
-    // first one), all 64 lanes present, away from the domain ends
-    unsigned c0 = (unsigned)g, lo = 0u;
-    bool rl = false, rs = false;
+    PairRun run{0u, 0u, 0u};
     if (BETA) {
-        c0 = __builtin_amdgcn_readfirstlane((unsigned)g);
-        lo = ((unsigned)g - c0) * 2u;
-        if (k != 0 && !wrap && __ballot(1) == ~0ull) pair_runs(c0, d, rl, rs);
-        pair_gather(pl, (unsigned)g, c0, lo, rl, d, cells, wrap, P);
+        run.c0 = (unsigned)first;
+        run.span = (unsigned)(end - first);
+        run.lo = ((unsigned)g - run.c0) * 2u;
+        pair_gather(pl, (unsigned)g, run, d, cells, wrap, P);
     } else {
         const unsigned own = cell_base((unsigned)g) * 2u;
 #pragma unroll
@@ -1284,22 +1327,22 @@ __device__ __forceinline__ void seam_pairs(const DomDev *__restrict__ D, int til
         }
         if (flag != kFlagGhost) store_macros<T>(D, (unsigned)(g + j), cells, vx, vy, vz, dn);
     }
-    if (k == 0) {  // the seam: lane 0 holds cells 0, 1 and lane 63 cells X-2, X-1
+    if (seam) {  // lane lz holds cells 0 and 1, lane le cells X-2 and X-1
         const unsigned m0 = D->xmask_a[0], m1 = D->xmask_a[1];
 #pragma unroll
         for (int q = 0; q < 19; ++q) {
-            const unsigned last = __builtin_amdgcn_readlane(P[q], 63), first = __builtin_amdgcn_readlane(P[q], 0);
             const bool take0 = BETA ? ex(q) == 1 : ((m0 >> q) & 1u) != 0;
             const bool take1 = BETA ? ex(q) == -1 : ((m1 >> q) & 1u) != 0;
-            if (l == 0 && take0) P[q] = (P[q] & 0xffff0000u) | (last & 0xffffu);
-            if (l == 63 && take1) P[q] = (P[q] & 0xffffu) | (first & 0xffff0000u);
+            const unsigned low = __builtin_amdgcn_readlane(P[q], lz), high = __builtin_amdgcn_readlane(P[q], le);
+            if (l == lz && take0) P[q] = (P[q] & 0xffff0000u) | (high & 0xffffu);
+            if (l == le && take1) P[q] = (P[q] & 0xffffu) | (low & 0xffff0000u);
         }
     }
     // store addresses from a fresh copy of the cell index (see cells_pair2)
     int gs = g;
     asm volatile("" : "+v"(gs));
     if (BETA) {
-        pair_scatter<NTS>(pl, (unsigned)gs, c0, lo, rs, d, cells, wrap, P);
+        pair_scatter<NTS>(pl, (unsigned)gs, run, d, cells, wrap, P);
     } else {
         const unsigned own_st = cell_base((unsigned)gs) * 2u;
 #pragma unroll
@@ -1341,8 +1384,9 @@ __global__ void __launch_bounds__(512) step_kernel(const DomDev *__restrict__ do
     const DomDev *D = doms + td;
     if (h >= D->stop_at) return;  // a finished member of a continuous batch keeps its state
     if constexpr (N == 2 && SP::kBytes == 2) {
-        if (D->seam_wpr > 0) {  // uniform per work-group
-            seam_pairs<SP, BETA, NTS, NTL>(D, t - D->tile_begin);
+        if (D->x_seam) {  // uniform per work-group
+            if ((D->nx & 127) == 0) seam_pairs<SP, BETA, NTS, NTL, true>(D, t - D->tile_begin);
+            else seam_pairs<SP, BETA, false, false, false>(D, t - D->tile_begin);
             return;
         }
     }

@@ -589,7 +589,7 @@ void fill_desc(lbm_solver *s) {
     d.gz = s->cfg.gravitation[2];
     d.lid = s->cfg.lid_velocity;
     d.stop_at = s->group ? s->stop_at : std::numeric_limits<long long>::max();
-    d.seam_wpr = 0;
+    d.x_seam = 0;
 }
 
 int upload_desc(lbm_solver *s) {
@@ -1854,16 +1854,14 @@ static int build_tables(lbm_group *g, int wg, LaunchTables &T) {
         if (pos[i] != 0) continue;  // a chain's tiles go with its first member
         if (g->chains[c].size() == 1 && g->xfuse[i].nb[0] == (int)i &&
             seam_ring_ok(group_pairs(g), g->members[i]->cfg.dims[0])) {
-            // a periodic ring of one in packed pairs: its seam stays in one
-            // wavefront per row (seam_pairs), tiles of whole wavefronts
-            const int X = g->members[i]->cfg.dims[0];
-            const long long pw = (long long)seam_waves_per_row(X) * g->members[i]->cfg.dims[1];
-            note_plane(pw % (wg / 64) == 0 ? pw / (wg / 64) : 0);
-            const long long waves = pw * g->members[i]->cfg.dims[2];
-            const int nt = (int)((waves + wg / 64 - 1) / (wg / 64));
+            // a periodic ring of one in packed pairs: the seam of each row stays
+            // in one wavefront (seam_pairs), the tiles are those of its cells
+            const long long pc = (long long)g->members[i]->cfg.dims[0] * g->members[i]->cfg.dims[1];
+            note_plane(pc % per_tile == 0 ? pc / per_tile : 0);
+            const int nt = (int)((g->members[i]->cells + per_tile - 1) / per_tile);
             descs[i].tile_begin = (int)tiles.size();
             descs[i].ntiles = nt;
-            descs[i].seam_wpr = seam_waves_per_row(X);
+            descs[i].x_seam = 1;
             tiles.insert(tiles.end(), (size_t)nt, (int)i);
             continue;
         }
