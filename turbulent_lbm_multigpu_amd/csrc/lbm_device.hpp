@@ -249,6 +249,13 @@ struct DomDev {
     long long stop_at;  // launch half-step index from which this domain stays frozen
     unsigned xmask_a[2];  // slots this domain's x- / x+ ghost layer takes after alpha in a chain tile
     int x_seam;           // periodic x seam inside the pair kernel (seam_pairs)
+    unsigned layers;      // faces exchanged between beta and alpha (in_layers), for pair_kernel
+    // x faces that pair_kernel exchanges itself (SeamRows): what comes in over
+    // them, all domains' in one buffer, per side its place there and the domain
+    // beyond, and whether a ghost cell takes all slots (or those that move to it)
+    void *seam;
+    unsigned seam_bytes, seam_at[2];
+    int seam_nb[2], seam_all;
 };
 
 // ---- fused x chains ----------------------------------------------------------

@@ -187,7 +187,7 @@ __device__ __forceinline__ void loads_arrived() { __builtin_amdgcn_s_waitcnt(0x0
 // HBM carries about 3.0 GB a pair at 256^3 where two half-step launches move
 // 5.1 GB.  256^3 LES: FP32 336 us a step against 464 in place (419 with the
 // best launch shape), FP64 563 against 922 (863).
-template <int ST, int NT>
+template <int ST, int NT, bool LAYERS>
 __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
     pair_kernel(const DomDev *__restrict__ doms, const PairTile *__restrict__ tiles, void *second, int flip,
                 int xcd_map, long long *ctr) {
@@ -228,6 +228,28 @@ __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
     const int alpha_from = (int)scalar_word(__ballot(stores) != 0ull ? 2u : (unsigned)nz + 2u);  // first plane of the walk with an alpha
     if (!stores) LA = pair_alpha_lane(P, X, 0);
     const int pitch = pair_pitch(P, X);
+    // Cells whose alpha has to wait for an exchange keep beta's values.  Over an
+    // x face, the inner cell's alpha takes what comes in from `seam` and goes to
+    // the ghost cell beyond the face, whose own lane leaves those slots out.
+    bool waits = false, inner[2] = {false, false}, ghost[2] = {false, false};
+    unsigned seam_at = 1u << 31;  // past the buffer: nothing is fetched
+    gchar *beyond = nullptr;
+    const SeamRows SR(D->layers, D->ny, D->nz);
+    if constexpr (LAYERS) {
+        const int y = LA.p / X, x = LA.p - y * X, side = x >= 2;
+        const bool face = in_layers(D->layers, 0, x, X), rim = in_layers(D->layers, 1, y, D->ny);
+        waits = rim || (face && !D->seam);
+        if (face && !waits) {
+            const bool out = x == (side ? X - 1 : 0);
+            inner[side] = !out;
+            ghost[side] = out;
+            if (!out) {
+                const DomDev *N = doms + D->seam_nb[side];
+                beyond = (gchar *)(flip ? N->dd : N->dd2);
+                seam_at = D->seam_at[side] + (unsigned)(y - SR.y0) * SP::kBytes;
+            }
+        }
+    }
     void *const two = second ? second : D->dd2;
     gchar *const from = (gchar *)(flip ? two : D->dd);
     const PairBuf dst = pair_buf((gchar *)(flip ? D->dd : two));
@@ -314,6 +336,15 @@ __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
         take_plane(k);
     }
     for (; k < nz + 2; ++k) {
+        const int z = z0 + k - 2;
+        const bool rows_z = z >= SR.z0 && z < SR.z0 + SR.nz;
+        U in[kSeamPops];
+        if constexpr (LAYERS) {
+            const PairBuf sb = pair_buf((gchar *)D->seam, scalar_word(rows_z && D->seam ? D->seam_bytes : 0u));
+            const unsigned at_row = seam_at + (unsigned)((z - SR.z0) * SR.ny) * SP::kBytes;
+#pragma unroll
+            for (int q = 0; q < kSeamPops; ++q) in[q] = buf_ld<U>(sb, at_row, (unsigned)(q * SR.count()) * SP::kBytes);
+        }
         beta_plane(k);
         T f[19], vx, vy, vz, dens;
         int q0 = 0, qu = 0;
@@ -325,24 +356,152 @@ __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
             f[i] = kin<SP>(v, i);
         }
         const PairPhys<T> ph = pair_phys_here(phys);
-        const bool keep = pair_update<T, false, SP::kShifted>(f, flag_mid, ph, macros, vx, vy, vz, dens);
+        int flag = flag_mid;
+        if constexpr (LAYERS) {
+            if (waits || !rows_z) flag = kFlagGhost;  // a ghost cell's values pass
+            int q = 0;
+#pragma unroll
+            for (int i = 0; i < 18; i += 2) {  // ex(i) = 1 comes with ex(i + 1) = -1
+                if (ex(i) == 0) continue;
+                const T v = kin<SP>(in[q], i);
+                f[i] = inner[0] && rows_z ? v : f[i];
+                f[i + 1] = inner[1] && rows_z ? v : f[i + 1];
+                ++q;
+            }
+        }
+        const bool keep = pair_update<T, false, SP::kShifted>(f, flag, ph, macros, vx, vy, vz, dens);
         // The next plane's loads are waited for before the stores: at the top
         // of the next plane the wait would cover the stores as well.
         loads_arrived();
         if (stores) {
-            const unsigned gs = (unsigned)(LA.p + XY * (z0 + k - 2));
+            const unsigned gs = (unsigned)(LA.p + XY * z);
             const unsigned own = cell_base(gs) * SP::kBytes;
             constexpr unsigned pop = kBlk * SP::kBytes;
             const unsigned even = own + (keep ? 0u : pop), odd = own + (keep ? pop : 0u);
+            auto put = [&](bool along_x, bool evens, bool odds) {
 #pragma unroll
-            for (int i = 0; i < 18; i += 2) {
-                buf_st<U>(dst, even, (unsigned)i * pop, kout<SP>(f[i], i));
-                buf_st<U>(dst, odd, (unsigned)i * pop, kout<SP>(f[i + 1], i + 1));
+                for (int i = 0; i < 18; i += 2) {
+                    if ((ex(i) != 0) != along_x) continue;
+                    if (evens) buf_st<U>(dst, even, (unsigned)i * pop, kout<SP>(f[i], i));
+                    if (odds) buf_st<U>(dst, odd, (unsigned)i * pop, kout<SP>(f[i + 1], i + 1));
+                }
+            };
+            if constexpr (LAYERS) {
+                const bool low = ghost[0] && rows_z, high = ghost[1] && rows_z;
+                if (!((low || high) && D->seam_all)) {
+                    put(false, true, true);
+                    buf_st<U>(dst, own, 18u * pop, kout<SP>(f[18], 18));
+                    // the low ghost cell leaves the slots with ex = -1 out, the high one those with ex = 1
+                    if (!(keep ? high : low)) put(true, true, false);
+                    if (!(keep ? low : high)) put(true, false, true);
+                }
+                if ((inner[0] || inner[1]) && rows_z) {
+                    const int to = inner[0] ? X - 2 : 2 - X;
+                    gchar *const n = beyond + (size_t)(cell_base(gs + (unsigned)to) * SP::kBytes);
+                    const bool all = D->seam_all;
+#pragma unroll
+                    for (int i = 0; i < 18; i += 2) {
+                        const U a = kout<SP>(keep ? f[i] : f[i + 1], i), b = kout<SP>(keep ? f[i + 1] : f[i], i + 1);
+                        if (all || (ex(i) != 0 && inner[0])) raw_st<false, U>(n + (size_t)i * pop, 0u, a);
+                        if (all || (ex(i) != 0 && inner[1])) raw_st<false, U>(n + (size_t)(i + 1) * pop, 0u, b);
+                    }
+                    if (all) raw_st<false, U>(n + (size_t)18 * pop, 0u, kout<SP>(f[18], 18));
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 18; i += 2) {
+                    buf_st<U>(dst, even, (unsigned)i * pop, kout<SP>(f[i], i));
+                    buf_st<U>(dst, odd, (unsigned)i * pop, kout<SP>(f[i + 1], i + 1));
+                }
+                buf_st<U>(dst, own, 18u * pop, kout<SP>(f[18], 18));
             }
-            buf_st<U>(dst, own, 18u * pop, kout<SP>(f[18], 18));
-            if (macros && flag_mid != kFlagGhost) store_macros<T>(D, gs, cells, vx, vy, vz, dens);
+            if (macros && flag != kFlagGhost) store_macros<T>(D, gs, cells, vx, vy, vz, dens);
         }
         take_plane(k);
+    }
+}
+
+// Alpha of the layers that pair_kernel left at beta's values, after their
+// exchange: `boxes` and, per block, the box it belongs to.  Bound by memory, as
+// alpha of a whole domain: 262,144 cells of y and z layers, FP32, in 13 us.
+template <int ST>
+__global__ void __launch_bounds__(256)
+    layer_alpha_kernel(const DomDev *__restrict__ doms, const LayerBox *__restrict__ boxes,
+                       const int *__restrict__ block_box, int flip) {
+    using SP = Storage<ST>;
+    using T = typename SP::T;
+    using U = typename SP::U;
+    const LayerBox &B = boxes[block_box[blockIdx.x]];
+    const DomDev *D = doms + B.dom;
+    const int e = ((int)blockIdx.x - B.block_begin) * 256 + (int)threadIdx.x;
+    if (e >= B.s[0] * B.s[1] * B.s[2]) return;
+    const int r = e / B.s[0], bz = r / B.s[1];
+    const int x = B.o[0] + e - r * B.s[0], y = B.o[1] + r - bz * B.s[1], z = B.o[2] + bz;
+    if (B.axis < 2 && in_layers(D->layers, 2, z, D->nz)) return;
+    if (B.axis < 1 && in_layers(D->layers, 1, y, D->ny)) return;
+    const unsigned g = (unsigned)(x + D->nx * (y + D->ny * z));
+    const int flag = (int)((const guchar *)D->flags)[g];
+    if (flag == kFlagGhost) return;
+    gchar *const own = (gchar *)(flip ? D->dd : D->dd2) + (size_t)cell_base(g) * SP::kBytes;
+    constexpr size_t pop = (size_t)kBlk * SP::kBytes;
+    T f[19], vx, vy, vz, dens;
+#pragma unroll
+    for (int i = 0; i < 19; ++i) f[i] = kin<SP>(raw_ld<false, U>(own + i * pop, 0u), i);
+    if (cell_update<T, false, SP::kShifted>(f, flag, D, vx, vy, vz, dens)) {
+#pragma unroll
+        for (int k = 0; k < 19; ++k) raw_st<false, U>(own + k * pop, 0u, kout<SP>(f[opp(k)], k));
+    }
+    store_macros<T>(D, g, (int)D->cells, vx, vy, vz, dens);
+}
+
+// What beta of the domain beyond an x face moves over it, into the seam buffer
+// for the pair of this domain: beta of the column next to its ghost layer, from
+// the buffer the pair starts in.  Bound by cache lines, 19 for a cell: 131,072
+// cells, FP32, in 89 us (3.6 TB/s of lines).  The alternative, pair_kernel
+// leaving both layers of a face by rows and a kernel after it doing their alpha
+// and exchange, stores single columns twice: 52 us more in pair_kernel, 82 in
+// that kernel.
+template <int ST>
+__global__ void __launch_bounds__(256)
+    seam_beta_kernel(const DomDev *__restrict__ doms, const SeamFace *__restrict__ faces,
+                     const int *__restrict__ block_face, int flip) {
+    using SP = Storage<ST>;
+    using T = typename SP::T;
+    using U = typename SP::U;
+    const SeamFace F = faces[block_face[blockIdx.x]];
+    const DomDev *N = doms + F.nb;
+    const int X = N->nx, XY = X * N->ny, cells = (int)N->cells;
+    const SeamRows SR(N->layers, N->ny, N->nz);  // those of both sides
+    // the rows whose populations reach such a row; past the ends by the linear wrap
+    const int wy = SR.ny + 2, e = ((int)blockIdx.x - F.block_begin) * 256 + (int)threadIdx.x;
+    if (e >= wy * (SR.nz + 2)) return;
+    const int rz = e / wy, y = SR.y0 - 1 + e - rz * wy, z = SR.z0 - 1 + rz;
+    const int g = (F.side ? 1 : X - 2) + X * y + XY * z;
+    PairRows rows;
+    pair_plane<SP>(rows, 0, g - XY, X, cells, true);
+    pair_plane<SP>(rows, 1, g, X, cells, true);
+    pair_plane<SP>(rows, 2, g + XY, X, cells, true);
+    U u[19];
+    pair_gather_cell<SP>(pair_buf((gchar *)(flip ? N->dd2 : N->dd)), rows, g, X, XY, cells, true, u);
+    const int flag = (int)((const guchar *)N->flags)[(unsigned)wrap_idx(g, cells)];
+    T f[19], vx, vy, vz, dens;
+#pragma unroll
+    for (int i = 0; i < 19; ++i) f[i] = kin<SP>(u[i], i);
+    const PairPhys<T> ph = pair_phys_here(pair_phys<T>(N));
+    const bool bounce = pair_update<T, true, SP::kShifted>(f, flag, ph, false, vx, vy, vz, dens);
+    gchar *const to = (gchar *)N->seam + doms[F.dom].seam_at[F.side];
+    int q = 0;
+#pragma unroll
+    for (int i = 0; i < 18; i += 2) {
+        if (ex(i) == 0) continue;
+        // the one of the two that moves to this domain: ex = 1 over its low face
+        const bool first = F.side == 0;
+        const int ty = y + (first ? ey(i) : ey(i + 1)), tz = z + (first ? ez(i) : ez(i + 1));
+        const T v = first != bounce ? f[i] : f[i + 1];
+        if (SR.has(ty, tz))
+            raw_st<false, U>(to + ((size_t)q * SR.count() + (ty - SR.y0) + (size_t)(tz - SR.z0) * SR.ny) * SP::kBytes,
+                             0u, kout<SP>(v, i));
+        ++q;
     }
 }
 
@@ -461,7 +620,8 @@ hipError_t launch_pair_storage(const PairLaunch &L, int ntiles, const DomDev *de
     }
     if constexpr (ST < 2) {
         constexpr int NT = ST == 1 ? 512 : 1024;
-        LBM_PAIR_GO((pair_kernel<ST, NT>), NT, 2 * NT * per_cell);
+        if (L.layers) LBM_PAIR_GO((pair_kernel<ST, NT, true>), NT, 2 * NT * per_cell);
+        LBM_PAIR_GO((pair_kernel<ST, NT, false>), NT, 2 * NT * per_cell);
     }
     return hipErrorInvalidValue;
 #undef LBM_PAIR_GO

@@ -455,6 +455,28 @@ struct lbm_group {
     size_t pair_cap = 0;
     int npair = 0;               // 0: not planned for the present members
     PairLaunch pair_launch{};
+    // Fused pairs of members that exchange faces: per member the faces
+    // (DomDev::layers), the boxes of the layers and, per block, its box, and
+    // the copies after beta ([1]) and alpha ([0]) in the buffer that a pair
+    // ends in ([flip]), with the second buffers they were made for.
+    bool faces_planned = false, faces_pair = false;
+    std::vector<unsigned> layers;
+    LayerBox *d_layers = nullptr;
+    size_t layers_cap = 0;
+    int nlayers = 0, layer_blocks = 0;
+    bool seams = false;  // x faces inside pair_kernel: seam_beta_kernel's faces and, per block, its face, and its results
+    SeamFace *d_seams = nullptr;
+    size_t seams_cap = 0;
+    int nseams = 0, seam_blocks = 0;
+    char *d_seam_slots = nullptr;
+    size_t seam_slots_cap = 0, seam_bytes = 0;
+    std::vector<size_t> seam_at;  // per member and side, where its part of them starts
+    std::vector<int> seam_nb;     // and the member beyond
+    CopyOp *d_face_ops[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+    size_t face_cap[2][2] = {{0, 0}, {0, 0}};
+    int nface[2] = {0, 0}, face_blocks[2] = {0, 0};
+    std::vector<HOp> face_hops[2];
+    std::vector<void *> face_seconds;
     std::vector<unsigned> seen_versions;
     std::vector<GroupComm> comms;
     bool plan_built = false;
@@ -590,6 +612,8 @@ void fill_desc(lbm_solver *s) {
     d.lid = s->cfg.lid_velocity;
     d.stop_at = s->group ? s->stop_at : std::numeric_limits<long long>::max();
     d.x_seam = 0;
+    d.layers = 0;
+    d.seam = nullptr;
 }
 
 int upload_desc(lbm_solver *s) {
@@ -649,6 +673,21 @@ long long cells_of(const std::vector<lbm_solver *> &doms) {
 // bytes with as many instructions, and are bound by those already.
 bool walks_pay(const std::vector<lbm_solver *> &doms, int storage) {
     return elem_size(storage) >= 4 && cells_of(doms) >= (storage == LBM_STORAGE_F64 ? 250000 : 480000);
+}
+
+// Whether fused pairs pay for domains that exchange faces (plan_faces), whose
+// pair takes five launches, or two with x faces only, and some of the work
+// again.  In place and its copies against pairs, us a half-step of a group.
+// In place, a state that stays in the last-level cache (256 MB) is moved
+// faster than one that does not: FP32 8 x 64^3 57 / 65, 8 x 72^3 128 / 91, 8 x
+// 96^3 194 / 164, 8 x 128^3 423 / 364, 4 of 120x90x90 in y and z 103 / 103;
+// FP64 8 x 52^3 62 / 74, 8 x 64^3 151 / 122, 8 x 80^3 315 / 203.  Joined in x
+// only, FP32: 2 of 100x100x50 34 / 36, 3 of 40x100x100 47 / 43, 2 of 100^3 57 /
+// 56; with x faces in the step kernel 39 / 36, 51 / 40, 68 / 54.  FP64 2 x 80^3
+// 57 / 68.
+bool face_pairs_pay(const std::vector<lbm_solver *> &doms, int storage, bool x_only) {
+    const long long bytes = 19ll * (long long)elem_size(storage) * cells_of(doms);
+    return bytes >= (x_only && storage == LBM_STORAGE_F32 ? 84000000ll : 240000000ll);
 }
 
 // The boxes of a domain too small for walks, and whether they beat the
@@ -1780,6 +1819,21 @@ static void group_drop_graph(lbm_group *g) {
 }
 
 static void group_free_plan(lbm_group *g) {
+    (void)hipFree(g->d_layers);
+    (void)hipFree(g->d_seams);
+    (void)hipFree(g->d_seam_slots);
+    g->d_layers = nullptr;
+    g->d_seams = nullptr;
+    g->d_seam_slots = nullptr;
+    g->layers_cap = g->seams_cap = g->seam_slots_cap = 0;
+    for (int f = 0; f < 2; ++f)
+        for (int k = 0; k < 2; ++k) {
+            (void)hipFree(g->d_face_ops[f][k]);
+            g->d_face_ops[f][k] = nullptr;
+            g->face_cap[f][k] = 0;
+        }
+    g->face_seconds.clear();
+    g->faces_planned = false;
     for (int k = 0; k < 2; ++k)
         for (int p = 0; p < 4; ++p) {
             if (g->d_ops[k][p]) (void)hipFree(g->d_ops[k][p]);
@@ -1837,6 +1891,18 @@ static int build_tables(lbm_group *g, int wg, LaunchTables &T) {
         descs[i] = m->host_desc;
         if (i < g->xfuse.size())
             for (int side = 0; side < 2; ++side) descs[i].xmask_a[side] = g->xfuse[i].mask[side];
+        if (i < g->layers.size()) {
+            descs[i].layers = g->layers[i];
+            if (g->seams) {
+                descs[i].seam = g->d_seam_slots;
+                descs[i].seam_bytes = (unsigned)g->seam_bytes;
+                descs[i].seam_all = g->exchange_mode != 1;
+                for (int side = 0; side < 2; ++side) {
+                    descs[i].seam_at[side] = (unsigned)g->seam_at[2 * i + side];
+                    descs[i].seam_nb[side] = g->seam_nb[2 * i + side];
+                }
+            }
+        }
     }
     long long plane = -1;  // tiles per z plane, shared by every member so far (0: not shared or not whole)
     auto note_plane = [&plane](long long p) { plane = (plane < 0 || plane == p) ? p : 0; };
@@ -2223,6 +2289,53 @@ static void plan_chains(lbm_group *g, const std::vector<char> &fuse) {
     }
 }
 
+// The counterpart of a comm: its partner's comm across the same face.
+static const GroupComm *partner_of(const lbm_group *g, const GroupComm &c) {
+    for (const GroupComm &q : g->comms)
+        if (q.member == c.dst && q.dst == c.member && q.normal[0] == -c.normal[0] && q.normal[1] == -c.normal[1] &&
+            q.normal[2] == -c.normal[2])
+            return &q;
+    return nullptr;
+}
+
+// The two copies of a comm and its counterpart: [0] after alpha, [1] after beta.
+static void comm_copies(const lbm_group *g, const GroupComm &c, const GroupComm &p, HOp *h) {
+    h[0] = HOp{c.dst, c.member, {}, {}, {}, alpha_mask(g, c)};
+    // after beta: neighbour's ghost layer -> my inner layer, n.e > 0 only (src/CController.hpp:322-383)
+    h[1] = HOp{c.dst, c.member, {}, {}, {}, norm_mask(c.normal)};
+    for (int ax = 0; ax < 3; ++ax) {
+        h[0].so[ax] = p.send_origin[ax];
+        h[0].dof[ax] = c.recv_origin[ax];
+        h[1].so[ax] = p.recv_origin[ax];
+        h[1].dof[ax] = c.send_origin[ax];
+        h[0].sz[ax] = h[1].sz[ax] = c.size[ax];
+    }
+}
+
+// A table of copies on the device: the ops, then the op index of every block
+// (exchange_kernel).  The host vectors are read until the stream is waited for.
+static int upload_ops(lbm_group *g, std::vector<CopyOp> &ops, std::vector<int> &block_op, CopyOp *&d_ops, size_t &cap,
+                      int &nops, int &nblocks) {
+    int blocks = 0;
+    block_op.clear();
+    for (size_t i = 0; i < ops.size(); ++i) {
+        CopyOp &op = ops[i];
+        op.block_begin = blocks;
+        const int nb = (op.cells / op.vec * op.npop + 255) / 256;
+        block_op.insert(block_op.end(), (size_t)nb, (int)i);
+        blocks += nb;
+    }
+    nops = (int)ops.size();
+    nblocks = blocks;
+    if (ops.empty()) return LBM_OK;
+    const size_t n = ops.size();
+    const size_t extra = (sizeof(int) * (size_t)blocks + sizeof(CopyOp) - 1) / sizeof(CopyOp);
+    GCHK(grow_table(d_ops, cap, n + extra));
+    GCHK(hipMemcpyAsync(d_ops, ops.data(), sizeof(CopyOp) * n, hipMemcpyHostToDevice, g->stream));
+    GCHK(hipMemcpyAsync(d_ops + n, block_op.data(), sizeof(int) * (size_t)blocks, hipMemcpyHostToDevice, g->stream));
+    return LBM_OK;
+}
+
 static int build_plan(lbm_group *g) {
     std::vector<CopyOp> ops[2][4];
     std::vector<HOp> hops[2][4];
@@ -2230,12 +2343,7 @@ static int build_plan(lbm_group *g) {
     std::vector<char> fuse(g->comms.size(), 0);
     for (size_t ci = 0; ci < g->comms.size(); ++ci) {
         const GroupComm &c = g->comms[ci];
-        for (const GroupComm &q : g->comms)
-            if (q.member == c.dst && q.dst == c.member && q.normal[0] == -c.normal[0] && q.normal[1] == -c.normal[1] &&
-                q.normal[2] == -c.normal[2]) {
-                partner[ci] = &q;
-                break;
-            }
+        partner[ci] = partner_of(g, c);
         if (!partner[ci])
             return gfail(g, LBM_ERR_STATE,
                          "comm of member " + std::to_string(c.member) + " toward " + std::to_string(c.dst) +
@@ -2249,19 +2357,11 @@ static int build_plan(lbm_group *g) {
         const int axis = c.normal[0] ? 0 : c.normal[1] ? 1 : 2;
         lbm_solver *me = g->members[c.member], *nb = g->members[c.dst];
         std::string why;
-        const uint32_t amask = alpha_mask(g, c);
         const bool fused = fuse[ci] && g->xfuse[c.member].nb[c.normal[0] == 1 ? 0 : 1] == c.dst;
         const int slot = fused ? 3 : axis;
-        HOp a{c.dst, c.member, {}, {}, {}, amask};
-        // after beta: neighbour's ghost layer -> my inner layer, n.e > 0 only (src/CController.hpp:322-383)
-        HOp b{c.dst, c.member, {}, {}, {}, norm_mask(c.normal)};
-        for (int ax = 0; ax < 3; ++ax) {
-            a.so[ax] = p->send_origin[ax];
-            a.dof[ax] = c.recv_origin[ax];
-            b.so[ax] = p->recv_origin[ax];
-            b.dof[ax] = c.send_origin[ax];
-            a.sz[ax] = b.sz[ax] = c.size[ax];
-        }
+        HOp copies[2];
+        comm_copies(g, c, *p, copies);
+        const HOp &a = copies[0], &b = copies[1];
         // each box is checked against both subdomains before any merging
         CopyOp chk;
         int rc = fill_op(nb, a.so, me, a.dof, a.sz, a.mask, chk, why);
@@ -2292,31 +2392,18 @@ static int build_plan(lbm_group *g) {
                 if (rc) return gfail(g, rc, why);
                 ops[k][q].push_back(op);
             }
-    // each table: the ops, then the op index of every block (exchange_kernel)
     std::vector<int> block_op[2][4];
     for (int k = 0; k < 2; ++k)
         for (int p = 0; p < 4; ++p) {
-            int blocks = 0;
-            for (size_t i = 0; i < ops[k][p].size(); ++i) {
-                CopyOp &op = ops[k][p][i];
-                op.block_begin = blocks;
-                const int nb = (op.cells / op.vec * op.npop + 255) / 256;
-                block_op[k][p].insert(block_op[k][p].end(), (size_t)nb, (int)i);
-                blocks += nb;
-            }
-            g->nops[k][p] = (int)ops[k][p].size();
-            g->nblocks[k][p] = blocks;
-            if (ops[k][p].empty()) continue;
-            const size_t n = ops[k][p].size();
-            const size_t extra = (sizeof(int) * (size_t)blocks + sizeof(CopyOp) - 1) / sizeof(CopyOp);
-            GCHK(grow_table(g->d_ops[k][p], g->ops_cap[k][p], n + extra));
-            GCHK(hipMemcpyAsync(g->d_ops[k][p], ops[k][p].data(), sizeof(CopyOp) * n, hipMemcpyHostToDevice,
-                                g->stream));
-            GCHK(hipMemcpyAsync(g->d_ops[k][p] + n, block_op[k][p].data(), sizeof(int) * (size_t)blocks,
-                                hipMemcpyHostToDevice, g->stream));
+            const int rc = upload_ops(g, ops[k][p], block_op[k][p], g->d_ops[k][p], g->ops_cap[k][p], g->nops[k][p],
+                                      g->nblocks[k][p]);
+            if (rc) return rc;
         }
     GCHK(hipStreamSynchronize(g->stream));
     g->plan_built = true;
+    g->faces_planned = false;
+    g->face_seconds.clear();
+    g->layers.clear();
     g->descs_dirty = true;  // the descriptors carry the fused faces
     return LBM_OK;
 }
@@ -2341,7 +2428,14 @@ static int group_prepare(lbm_group *g) {
 // at replay time and may change in place).
 static std::vector<long long> group_shape(const lbm_group *g) {
     std::vector<long long> v = {g->wg, g->wg_alpha, g->variant, g->lds, (long long)(uintptr_t)g->d_ctr,
-                                g->npair, (long long)(uintptr_t)g->d_pair};
+                                g->npair, (long long)(uintptr_t)g->d_pair, g->nlayers, g->layer_blocks,
+                                (long long)(uintptr_t)g->d_layers, g->nseams, g->seam_blocks,
+                                (long long)(uintptr_t)g->d_seams};
+    for (int k = 0; k < 2; ++k) {
+        v.push_back(g->nface[k]);
+        v.push_back(g->face_blocks[k]);
+        for (int f = 0; f < 2; ++f) v.push_back((long long)(uintptr_t)g->d_face_ops[f][k]);
+    }
     for (const LaunchTables &T : g->lt) {
         v.push_back(T.ntiles);
         v.push_back((long long)(uintptr_t)T.d_descs);
@@ -2410,19 +2504,192 @@ static void group_advance_counters(lbm_group *g, long long before, long long don
     g->step_counter = before + done;
 }
 
+// Whether members that exchange faces can run as fused pairs: every comm joins
+// a whole face, ghost layer and the one next to it, with its counterpart, no
+// member stops, and the copies of the three axes resolve to one set.  In such
+// a pair the cells of the layers, whose alpha needs the exchange after beta,
+// keep beta's values in the new buffer; there follow the copies after beta,
+// alpha of the layers (layer_alpha_kernel) and the copies after alpha.  x faces
+// are pair_kernel's own (SeamRows).  256^3 FP32 in 2x2x2: pair_kernel 620 us,
+// before it seam_beta_kernel 89, after it 12 + 13 + 9, where beta, alpha and
+// two copies in place took 858.
+static void plan_faces(lbm_group *g) {
+    g->faces_planned = true;
+    g->faces_pair = false;
+    g->layers.assign(g->members.size(), 0u);
+    std::vector<HOp> phase[2][3];
+    for (const lbm_solver *m : g->members)
+        if (m->stop_at != std::numeric_limits<long long>::max()) return;
+    for (const GroupComm &c : g->comms) {
+        const GroupComm *p = partner_of(g, c);
+        const int a = c.normal[0] ? 0 : c.normal[1] ? 1 : 2, side = c.normal[a] == 1 ? 0 : 1;
+        for (const GroupComm *q : {&c, p}) {
+            const int *d = g->members[q->member]->cfg.dims;
+            const bool low = q->normal[a] == 1;
+            for (int ax = 0; ax < 3; ++ax) {
+                if (q->normal[ax] != (ax == a ? (low ? 1 : -1) : 0)) return;
+                if (q->size[ax] != (ax == a ? 1 : d[ax])) return;
+                if (q->send_origin[ax] != (ax != a ? 0 : low ? 1 : d[a] - 2)) return;
+                if (q->recv_origin[ax] != (ax != a ? 0 : low ? 0 : d[a] - 1)) return;
+            }
+            if (d[a] < 4) return;
+        }
+        g->layers[(size_t)c.member] |= 1u << (2 * a + side);
+        HOp h[2];
+        comm_copies(g, c, *p, h);
+        for (int k = 0; k < 2; ++k) phase[k][a].push_back(h[k]);
+    }
+    for (int k = 0; k < 2; ++k) {
+        g->face_hops[k].clear();
+        if (!merge_phases(phase[k], g->face_hops[k])) return;
+    }
+    // The columns of x faces lie a row apart, each in a cache line of its own, so
+    // going through them again costs far more than their cells (with copies and
+    // layer_alpha_kernel for them too, those took 194 us of the above pair, not
+    // 34): pair_kernel exchanges them itself, in the rows that both sides of
+    // every x face step this way.
+    g->seams = true;
+    for (const GroupComm &c : g->comms) {
+        if (!c.normal[0]) continue;
+        const lbm_solver *m = g->members[c.member], *n = g->members[c.dst];
+        for (int ax = 0; ax < 3; ++ax) g->seams = g->seams && m->cfg.dims[ax] == n->cfg.dims[ax];
+        g->seams = g->seams && (g->layers[(size_t)c.member] >> 2) == (g->layers[(size_t)c.dst] >> 2);
+    }
+    g->seam_at.assign(2 * g->members.size(), 0);
+    g->seam_nb.assign(2 * g->members.size(), 0);
+    for (const GroupComm &c : g->comms)
+        if (c.normal[0]) g->seam_nb[2 * (size_t)c.member + (c.normal[0] == 1 ? 0 : 1)] = c.dst;
+    g->seam_bytes = 0;
+    for (size_t i = 0; i < g->members.size(); ++i)
+        for (int side = 0; side < 2; ++side) {
+            if (!(g->layers[i] >> side & 1u)) continue;
+            const int *d = g->members[i]->cfg.dims;
+            g->seam_at[2 * i + side] = g->seam_bytes;
+            const int n = SeamRows(g->layers[i], d[1], d[2]).count();
+            if (n <= 0 || SeamRows(g->layers[i], d[1], d[2]).ny <= 0) g->seams = false;
+            g->seam_bytes += (size_t)kSeamPops * std::max(n, 0) * elem_size(g->storage);
+        }
+    if (g->seam_bytes == 0 || g->seam_bytes >= (size_t)1 << 31) g->seams = false;
+    // the copies in those rows are that kernel's
+    for (int k = 0; k < 2 && g->seams; ++k) {
+        std::vector<HOp> kept;
+        for (const HOp &h : g->face_hops[k]) {
+            const int *d = g->members[(size_t)h.dm]->cfg.dims;
+            const SeamRows R(g->layers[(size_t)h.dm], d[1], d[2]);
+            const int o[3] = {0, R.y0, R.z0}, sz[3] = {d[0], R.ny, R.nz};
+            int io[3], is[3];
+            if (!box_isect(h.dof, h.sz, o, sz, io, is)) {
+                kept.push_back(h);
+                continue;
+            }
+            std::vector<std::array<int, 6>> rest;
+            box_minus(h.dof, h.sz, io, is, rest);
+            for (const auto &b : rest) kept.push_back(op_at_dst(h, &b[0], &b[3]));
+        }
+        g->face_hops[k].swap(kept);
+    }
+    g->faces_pair = true;
+    g->descs_dirty = true;  // the descriptors carry the layers
+}
+
+// The tables of plan_faces on the device, for the present second buffers.
+static int upload_faces(lbm_group *g) {
+    std::vector<void *> seconds;
+    for (const lbm_solver *m : g->members) seconds.push_back(m->dd2);
+    if (seconds == g->face_seconds) return LBM_OK;
+    std::vector<LayerBox> boxes;
+    std::vector<int> block_box;
+    for (size_t i = 0; i < g->members.size(); ++i) layer_boxes((int)i, g->layers[i], g->members[i]->cfg.dims, g->seams, boxes);
+    for (size_t i = 0; i < boxes.size(); ++i) {
+        boxes[i].block_begin = (int)block_box.size();
+        const long long n = (long long)boxes[i].s[0] * boxes[i].s[1] * boxes[i].s[2];
+        block_box.insert(block_box.end(), (size_t)((n + 255) / 256), (int)i);
+    }
+    const size_t extra = (sizeof(int) * block_box.size() + sizeof(LayerBox) - 1) / sizeof(LayerBox);
+    GCHK(grow_table(g->d_layers, g->layers_cap, boxes.size() + extra));
+    if (!boxes.empty()) {
+        GCHK(hipMemcpyAsync(g->d_layers, boxes.data(), sizeof(LayerBox) * boxes.size(), hipMemcpyHostToDevice,
+                            g->stream));
+        GCHK(hipMemcpyAsync(g->d_layers + boxes.size(), block_box.data(), sizeof(int) * block_box.size(),
+                            hipMemcpyHostToDevice, g->stream));
+    }
+    g->nlayers = (int)boxes.size();
+    g->layer_blocks = (int)block_box.size();
+    std::vector<SeamFace> faces;
+    std::vector<int> block_face;
+    for (const GroupComm &c : g->comms) {
+        if (!g->seams || !c.normal[0]) continue;
+        const int *d = g->members[(size_t)c.member]->cfg.dims;
+        const SeamRows R(g->layers[(size_t)c.member], d[1], d[2]);
+        const int n = (R.ny + 2) * (R.nz + 2);
+        faces.push_back(SeamFace{c.member, c.normal[0] == 1 ? 0 : 1, c.dst, (int)block_face.size()});
+        block_face.insert(block_face.end(), (size_t)((n + 255) / 256), (int)faces.size() - 1);
+    }
+    const size_t face_extra = (sizeof(int) * block_face.size() + sizeof(SeamFace) - 1) / sizeof(SeamFace);
+    GCHK(grow_table(g->d_seams, g->seams_cap, faces.size() + face_extra));
+    void *const slots = g->d_seam_slots;
+    GCHK(grow_table(g->d_seam_slots, g->seam_slots_cap, g->seams ? g->seam_bytes : 1));
+    if (slots != g->d_seam_slots) g->descs_dirty = true;
+    g->nseams = (int)faces.size();
+    g->seam_blocks = (int)block_face.size();
+    if (!faces.empty()) {
+        GCHK(hipMemcpyAsync(g->d_seams, faces.data(), sizeof(SeamFace) * faces.size(), hipMemcpyHostToDevice,
+                            g->stream));
+        GCHK(hipMemcpyAsync(g->d_seams + faces.size(), block_face.data(), sizeof(int) * block_face.size(),
+                            hipMemcpyHostToDevice, g->stream));
+    }
+    std::vector<CopyOp> ops[2][2];
+    std::vector<int> block_op[2][2];
+    for (int f = 0; f < 2; ++f)
+        for (int k = 0; k < 2; ++k) {
+            for (const HOp &h : g->face_hops[k]) {
+                if (!h.mask) continue;
+                CopyOp op;
+                std::string why;
+                lbm_solver *from = g->members[h.sm], *to = g->members[h.dm];
+                const int rc = fill_op(from, h.so, to, h.dof, h.sz, h.mask, op, why);
+                if (rc) return gfail(g, rc, why);
+                if (!f) {
+                    op.src = from->dd2;
+                    op.dst = to->dd2;
+                }
+                ops[f][k].push_back(op);
+            }
+            const int rc = upload_ops(g, ops[f][k], block_op[f][k], g->d_face_ops[f][k], g->face_cap[f][k],
+                                      g->nface[k], g->face_blocks[k]);
+            if (rc) return rc;
+        }
+    GCHK(hipStreamSynchronize(g->stream));
+    g->face_seconds = seconds;
+    return LBM_OK;
+}
+
 // Whether the next `steps` half-steps (from a beta step) may run as fused
-// pairs: no exchange between the half-steps, second buffers for every member,
-// and no member that freezes on the way (a member frozen already keeps its
-// state; one that freezes between two pairs would keep it in the wrong
-// buffer).  Brings the pair tiles and descriptors up to date.
+// pairs: second buffers for every member, faces that are exchanged in a way
+// plan_faces knows, and no member that freezes on the way (a member frozen
+// already keeps its state; one that freezes between two pairs would keep it in
+// the wrong buffer).  Brings the pair tiles and descriptors up to date.
 static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
     *ready = false;
-    if (steps < 4 || g->timing || !g->comms.empty() || !walks_pay(g->members, g->storage)) return LBM_OK;
+    if (steps < 4 || g->timing || !walks_pay(g->members, g->storage)) return LBM_OK;
     for (const lbm_solver *m : g->members)
         if (m->external) return LBM_OK;
     for (const lbm_solver *m : g->members)
         if (m->stop_at > g->step_counter && m->stop_at < g->step_counter + steps) return LBM_OK;
+    if (!g->comms.empty()) {
+        bool x_only = true;
+        for (const GroupComm &c : g->comms) x_only = x_only && c.normal[0] != 0;
+        if (!face_pairs_pay(g->members, g->storage, x_only)) return LBM_OK;
+        int rc = group_prepare(g);  // refuses comms without a counterpart
+        if (rc) return rc;
+        if (!g->faces_planned) plan_faces(g);
+        if (!g->faces_pair) return LBM_OK;
+    }
     if (!take_seconds(g->members)) return LBM_OK;
+    if (!g->comms.empty()) {
+        int rc = upload_faces(g);
+        if (rc) return rc;
+    }
     if (!g->npair) {
         const PairPlan P = plan_pairs(g->members, g->storage);
         GCHK(grow_table(g->d_pair, g->pair_cap, P.tiles.size()));
@@ -2432,6 +2699,7 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
         g->npair = (int)P.tiles.size();
         g->pair_launch = P.launch;
     }
+    g->pair_launch.layers = !g->comms.empty();
     int rc = group_prepare(g);  // the descriptors carry the second buffers
     if (rc) return rc;
     *ready = true;
@@ -2440,9 +2708,37 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
 
 // Two beta+alpha pairs of every member: into the second buffers and back.
 static int group_launch_two_pairs(lbm_group *g) {
-    for (int flip = 0; flip < 2; ++flip)
-        GCHK(launch_pair_kernel(g->storage, g->pair_launch, g->npair, g->lt[0].d_descs, g->d_pair, nullptr, g->stream,
-                                g->d_ctr, flip));
+    const DomDev *descs = g->lt[0].d_descs;
+    auto seam_betas = [&](auto st, int flip) -> hipError_t {
+        if (g->seam_blocks)
+            seam_beta_kernel<decltype(st)::value><<<g->seam_blocks, 256, 0, g->stream>>>(
+                descs, g->d_seams, (const int *)(g->d_seams + g->nseams), flip);
+        return hipGetLastError();
+    };
+    auto layer_alphas = [&](auto st, int flip) -> hipError_t {
+        if (g->layer_blocks)
+            layer_alpha_kernel<decltype(st)::value><<<g->layer_blocks, 256, 0, g->stream>>>(
+                descs, g->d_layers, (const int *)(g->d_layers + g->nlayers), flip);
+        return hipGetLastError();
+    };
+    auto of_storage = [&](auto fn, int flip) -> hipError_t {
+        return g->storage == LBM_STORAGE_F32 ? fn(std::integral_constant<int, 0>{}, flip)
+                                             : fn(std::integral_constant<int, 1>{}, flip);
+    };
+    auto copies = [&](int k, int flip) -> hipError_t {
+        if (!g->nface[k]) return hipSuccess;
+        return exchange_launch(g->storage, g->d_face_ops[flip][k], g->nface[k], g->face_blocks[k], g->stream);
+    };
+    const bool faces = g->pair_launch.layers;
+    for (int flip = 0; flip < 2; ++flip) {
+        if (faces) GCHK(of_storage(seam_betas, flip));
+        GCHK(launch_pair_kernel(g->storage, g->pair_launch, g->npair, descs, g->d_pair, nullptr, g->stream, g->d_ctr,
+                                flip));
+        if (!faces) continue;
+        GCHK(copies(1, flip));
+        GCHK(of_storage(layer_alphas, flip));
+        GCHK(copies(0, flip));
+    }
     return LBM_OK;
 }
 

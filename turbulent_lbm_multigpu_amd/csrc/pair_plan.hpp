@@ -57,9 +57,59 @@ LBM_PAIR_FN bool pair_wraps(const PairTile &P, int X, int XY, int cells) {
     return P.org - 1 - X + XY * (P.z0 - 2) < 0 || last + 1 + X + XY * (P.z0 + P.nz + 1) >= cells;
 }
 
+// A domain that exchanges faces: bit 2a (2a + 1) of `layers` is set where the
+// low (high) end of axis a has a neighbour.  Whether coordinate c of that axis
+// (extent n) is in the ghost layer there or in the layer next to it.
+LBM_PAIR_FN bool in_layers(unsigned layers, int a, int c, int n) {
+    return ((layers >> (2 * a) & 1u) != 0 && c < 2) || ((layers >> (2 * a + 1) & 1u) != 0 && c >= n - 2);
+}
+
+// The rows (y, z) of a domain that are in no layer of y or z, by y, then z: in
+// those pair_kernel exchanges x faces itself.  What comes in over a face are
+// the kSeamPops populations that beta moves over it, by population (in their
+// order) and row.
+constexpr int kSeamPops = 5;
+struct SeamRows {
+    int y0, z0, ny, nz;
+    LBM_PAIR_FN SeamRows(unsigned layers, int Y, int Z)
+        : y0(layers >> 2 & 1u ? 2 : 0), z0(layers >> 4 & 1u ? 2 : 0), ny(Y - y0 - (layers >> 3 & 1u ? 2 : 0)),
+          nz(Z - z0 - (layers >> 5 & 1u ? 2 : 0)) {}
+    LBM_PAIR_FN int count() const { return ny * nz; }
+    LBM_PAIR_FN bool has(int y, int z) const { return y >= y0 && y < y0 + ny && z >= z0 && z < z0 + nz; }
+};
+
+// An x face of domain `dom`, beyond it `nb`, as a range of blocks of
+// seam_beta_kernel.
+struct SeamFace {
+    int dom, side, nb;
+    int block_begin;
+};
+
+// Planes of a domain at an exchanged face, a range of blocks of
+// layer_alpha_kernel.
+struct LayerBox {
+    int dom, axis;
+    int o[3], s[3];
+    int block_begin;
+};
+
+// The boxes of a domain, those of x faces unless `seams`; a cell of several
+// belongs to the one of the last axis.
+inline void layer_boxes(int dom, unsigned layers, const int *dims, bool seams, std::vector<LayerBox> &out) {
+    for (int a = seams ? 1 : 0; a < 3; ++a)
+        for (int side = 0; side < 2; ++side) {
+            if (!(layers >> (2 * a + side) & 1u)) continue;
+            LayerBox b{dom, a, {0, 0, 0}, {dims[0], dims[1], dims[2]}, 0};
+            b.o[a] = side ? dims[a] - 2 : 0;
+            b.s[a] = 2;
+            out.push_back(b);
+        }
+}
+
 // How a pair launch is made.
 struct PairLaunch {
     int threads = 0;
+    bool layers = false;  // the domains exchange faces between beta and alpha (DomDev::layers)
     int box_cells = 0;  // > 0: tiles are boxes of at most this many columns x planes (pair_box_kernel)
     int xcd_map = 0;  // see step_kernel
 };
