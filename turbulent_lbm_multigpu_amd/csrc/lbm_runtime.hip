@@ -2427,10 +2427,11 @@ static int group_prepare(lbm_group *g) {
 // tables' addresses (a table that grew was reallocated; its contents are read
 // at replay time and may change in place).
 static std::vector<long long> group_shape(const lbm_group *g) {
-    std::vector<long long> v = {g->wg, g->wg_alpha, g->variant, g->lds, (long long)(uintptr_t)g->d_ctr,
-                                g->npair, (long long)(uintptr_t)g->d_pair, g->nlayers, g->layer_blocks,
-                                (long long)(uintptr_t)g->d_layers, g->nseams, g->seam_blocks,
-                                (long long)(uintptr_t)g->d_seams};
+    std::vector<long long> v;
+    v.reserve(64);  // made for every step call
+    v = {g->wg, g->wg_alpha, g->variant, g->lds, (long long)(uintptr_t)g->d_ctr, g->npair,
+         (long long)(uintptr_t)g->d_pair, g->nlayers, g->layer_blocks, (long long)(uintptr_t)g->d_layers, g->nseams,
+         g->seam_blocks, (long long)(uintptr_t)g->d_seams};
     for (int k = 0; k < 2; ++k) {
         v.push_back(g->nface[k]);
         v.push_back(g->face_blocks[k]);
