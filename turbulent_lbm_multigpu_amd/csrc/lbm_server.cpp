@@ -13,6 +13,8 @@
 // auxiliary stream.  Built only on the C-ABI of lbm_capi.h plus HIP streams
 // and events.
 #include <hip/hip_runtime.h>
+#include <stdlib.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <chrono>
@@ -73,6 +75,22 @@ class Arena {
     std::map<size_t, size_t> free_;
 };
 
+// A block of floats, uninitialised, in large pages where the system has them:
+// a result's pages are touched for the first time by its readback (eight cases
+// of 39^3 to 90^3 in a new server: 23.3 -> 19.5 ms).
+struct FreeBlock {
+    void operator()(float *p) const { free(p); }
+};
+typedef std::unique_ptr<float[], FreeBlock> FloatBlock;
+FloatBlock new_block(size_t floats) {
+    constexpr size_t kPage = (size_t)2 << 20;
+    const size_t bytes = floats * sizeof(float);
+    if (bytes < kPage) return FloatBlock((float *)malloc(bytes));
+    void *p = aligned_alloc(kPage, (bytes + kPage - 1) / kPage * kPage);
+    if (p) (void)madvise(p, bytes, MADV_HUGEPAGE);  // else it is made of small ones
+    return FloatBlock((float *)p);
+}
+
 struct Case {
     long long id = 0;
     lbm_case c{};
@@ -83,8 +101,8 @@ struct Case {
     long long steps_done = 0;
     long long cells = 0;
     double submit_s = 0, admit_s = 0, done_s = 0;
-    std::unique_ptr<float[]> fields;  // rho[cells], j[3][cells]
-    size_t fields_floats = 0;         // its size
+    FloatBlock fields;         // rho[cells], j[3][cells]
+    size_t fields_floats = 0;  // its size
     std::string error;  // why a FAILED case failed
 };
 
@@ -149,7 +167,7 @@ struct lbm_server {
     std::deque<Case *> queue;
     std::vector<Case *> ready;   // initialised, joining at the next chunk boundary
     std::vector<Case *> retiring;
-    std::vector<std::pair<std::unique_ptr<float[]>, size_t>> spare_results;  // oldest first
+    std::vector<std::pair<FloatBlock, size_t>> spare_results;  // oldest first
     size_t spare_floats = 0;
     std::deque<long long> done_order;
     bool inflight = false;
@@ -321,7 +339,7 @@ int pool_join(lbm_server *s, Case *c, bool *stuck) {
 
 // Room for a case's results: the smallest kept block that holds them (touching
 // fresh pages costs more than the copy), else a new one.
-void results_take(lbm_server *s, Case *c) {
+bool results_take(lbm_server *s, Case *c) {
     const size_t want = (size_t)c->cells * 4;
     auto best = s->spare_results.end();
     for (auto it = s->spare_results.begin(); it != s->spare_results.end(); ++it)
@@ -333,10 +351,11 @@ void results_take(lbm_server *s, Case *c) {
         c->fields_floats = best->second;
         s->spare_floats -= best->second;
         s->spare_results.erase(best);
-        return;
+        return true;
     }
-    c->fields.reset(new float[want]);
+    c->fields = new_block(want);
     c->fields_floats = want;
+    return c->fields != nullptr;
 }
 
 // A fetched case's block is kept for the next results, at most kSpareResults
@@ -358,11 +377,7 @@ void results_give(lbm_server *s, Case *c) {
 
 // rho and j of the whole case to the host.
 int case_readback(lbm_server *s, Case *c) {
-    try {
-        results_take(s, c);
-    } catch (const std::bad_alloc &) {
-        return s->fail(LBM_ERR_OUT_OF_MEMORY, "readback: no host memory for the results");
-    }
+    if (!results_take(s, c)) return s->fail(LBM_ERR_OUT_OF_MEMORY, "readback: no host memory for the results");
     const int rc = lbm_solver_moments_float(c->solver, c->fields.get(), c->fields.get() + c->cells);
     if (rc) return s->fail_lib(rc, "readback", lbm_solver_error(c->solver));
     if (!case_release(s, c)) return s->fail(LBM_ERR_STATE, "readback: the case's solver cannot be released");
