@@ -148,6 +148,10 @@ int lbm_solver_init_perturbed(lbm_solver *s, double amplitude, uint64_t seed, ui
 int lbm_solver_simulation_step(lbm_solver *s);
 int lbm_solver_simulation_step_alpha(lbm_solver *s);
 int lbm_solver_simulation_step_beta(lbm_solver *s);
+/* a sequence of at least 4 half-steps in FP32 or FP64 may go through a second
+ * buffer of the distributions that the solver then keeps, as may
+ * lbm_group_step's (same results; taken only while half the device's memory
+ * stays free, given up when an allocation of this library fails) */
 int lbm_solver_run(lbm_solver *s, int steps);
 /* wait(): clFinish (src/CLbmSolver.hpp:681-683) */
 int lbm_solver_wait(lbm_solver *s);
@@ -223,13 +227,13 @@ int lbm_group_set_exchange_mode(lbm_group *g, int mode);
  * launch disappears (the x faces are the strided ones: one element per cache
  * line).  A periodic ring of one member in a two-byte storage launched with
  * packed pairs (kernel variants 8, 11) and rows of an even length >= 128
- * instead keeps each row's seam in one wavefront (cells 0..63 and X-64..X-1)
- * and moves the face values by lane reads.  Every slot of every member is
+ * instead keeps each row's seam in one wavefront and moves the face values by
+ * lane reads.  Every slot of every member is
  * identical to the copy-based exchange.  Chains whose rows (or, for wide
  * rows, whose 64-cell face runs) do not fit the work-group keep their
  * copies.  lbm_group_sync still copies.  `mode`: 0 = copy launch, 1 = inside
  * the step kernel, LBM_FUSED_X_AUTO = inside the step kernel for FP32/FP64
- * storage; for FP16/BF16 only the seam wavefronts, other x faces by the copy
+ * storage; for FP16/BF16 only those seams, other x faces by the copy
  * launch (measured: the two-byte kernels lose more to the handoff tiles than
  * the copy launch costs). */
 #define LBM_FUSED_X_AUTO 2

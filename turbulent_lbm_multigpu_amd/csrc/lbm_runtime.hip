@@ -451,7 +451,7 @@ struct lbm_group {
     std::string err;
     LaunchTables lt[2];        // [0]: at wg (beta, and alpha unless wg_alpha is set), [1]: alpha at wg_alpha
     long long *d_ctr = nullptr;  // device half-step counter (two slots, see step_kernel)
-    PairTile *d_pair = nullptr;  // tiles of the fused pairs (groups without exchange)
+    PairTile *d_pair = nullptr;  // tiles of the fused pairs
     size_t pair_cap = 0;
     int npair = 0;               // 0: not planned for the present members
     PairLaunch pair_launch{};
