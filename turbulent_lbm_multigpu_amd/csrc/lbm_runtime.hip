@@ -2675,6 +2675,9 @@ static int upload_faces(lbm_group *g) {
             if (rc) return rc;
         }
     GCHK(hipStreamSynchronize(g->stream));
+    // the tables' own allocation may have had to take second buffers away
+    for (size_t i = 0; i < seconds.size(); ++i)
+        if (g->members[i]->dd2 != seconds[i]) return LBM_OK;
     g->face_seconds = seconds;
     return LBM_OK;
 }
