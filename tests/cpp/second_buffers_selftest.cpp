@@ -1,0 +1,125 @@
+// Checks the bookkeeping of the second buffers with host memory in the
+// device's place.
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <memory>
+#include <thread>
+
+#include "second_buffers.hpp"
+
+using namespace lbm;
+
+static int fails = 0;
+#define CHECK(c)                                               \
+    do {                                                       \
+        if (!(c)) {                                            \
+            if (++fails < 20) printf("FAIL %d: %s\n", __LINE__, #c); \
+        }                                                      \
+    } while (0)
+
+struct HostMemory : SecondMemory {
+    std::atomic<int> blocks{0}, drains{0}, asked{0};
+    bool full = false;
+    void *allocate(int, size_t bytes) override {
+        ++asked;
+        if (full) return nullptr;
+        ++blocks;
+        return malloc(bytes);
+    }
+    void release(void *p) override {
+        --blocks;
+        free(p);
+    }
+    void drain(int) override { ++drains; }
+};
+
+struct Solver {
+    std::atomic<unsigned> version{0};
+    SecondBuffer second;
+    explicit Solver(size_t bytes, int device = 0) {
+        second.version = &version;
+        second.bytes = bytes;
+        second.device = device;
+    }
+};
+
+// A solver goes away on its own thread while another thread's failed allocation
+// takes its buffer: after give() nothing of it may be written any more.
+static void destroyed_while_taken_away() {
+    HostMemory mem;
+    SecondBuffers sb(mem);
+    std::atomic<bool> stop{false};
+    std::thread short_of_memory([&] {
+        while (!stop) sb.give_all(0);
+    });
+    SecondBlock *const other = (SecondBlock *)0x10;
+    for (int k = 0; k < 3000 && !fails; ++k) {
+        Solver *s = new Solver(1000);
+        CHECK(sb.take({&s->second}));
+        while (s->second.at) {
+        }
+        sb.give(s->second);
+        s->second.block = other;  // the solver's memory is someone else's now
+        const unsigned v = s->version;
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(20);
+        while (std::chrono::steady_clock::now() < until) {
+        }
+        CHECK(s->second.block == other && s->version == v);
+        delete s;
+    }
+    stop = true;
+    short_of_memory.join();
+}
+
+static void blocks_and_spares() {
+    HostMemory mem;
+    SecondBuffers sb(mem);
+    {
+        Solver a(1000), b(200), c(500, 1);
+        CHECK(sb.take({&a.second, &b.second}));
+        CHECK(mem.blocks == 1 && (char *)b.second.at.load() - (char *)a.second.at.load() == 1024);
+        CHECK(a.version == 1 && b.version == 1);
+        CHECK(sb.take({&a.second, &b.second}) && mem.blocks == 1 && a.version == 1);
+        CHECK(sb.take({&c.second}) && mem.blocks == 2);
+        CHECK(sb.give_all(0) && mem.drains == 1);
+        CHECK(!a.second.at && !b.second.at && c.second.at && a.version == 2 && mem.blocks == 1);
+        CHECK(sb.take({&a.second}) && mem.blocks == 2);
+        sb.give(a.second);
+        CHECK(mem.blocks == 2);  // kept for the next solver
+        CHECK(sb.take({&b.second}) && mem.blocks == 3);  // far too large for this one
+        sb.give(b.second);
+        sb.give(c.second);
+        sb.give(c.second);
+    }
+    Solver d(900);
+    CHECK(sb.take({&d.second}) && mem.blocks == 3);
+    sb.give(d.second);
+    {
+        std::vector<std::unique_ptr<Solver>> many;
+        for (int k = 0; k < 30; ++k) {
+            many.emplace_back(new Solver(5000 + 4000 * (size_t)k));
+            CHECK(sb.take({&many.back()->second}));
+        }
+        for (auto &s : many) sb.give(s->second);
+        CHECK(mem.blocks == (int)SecondBuffers::kSpares);
+    }
+    sb.give_all(0);
+    CHECK(mem.blocks == 0 && !sb.give_all(0));
+    mem.full = true;
+    Solver e(100);
+    CHECK(!sb.take({&e.second}) && !e.second.at);
+    sb.give(e.second);
+}
+
+int main() {
+    blocks_and_spares();
+    destroyed_while_taken_away();
+    if (fails) {
+        printf("%d failures\n", fails);
+        return 1;
+    }
+    printf("second buffers: ok\n");
+    return 0;
+}

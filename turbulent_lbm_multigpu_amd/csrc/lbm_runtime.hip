@@ -14,8 +14,6 @@
 #include <cstring>
 #include <limits>
 #include <mutex>
-#include <set>
-#include <shared_mutex>
 #include <string>
 #include <vector>
 
@@ -26,6 +24,7 @@
 #include "launch_shape.hpp"
 #include "lbm_device.hpp"
 #include "lbm_pair.hpp"
+#include "second_buffers.hpp"
 
 using namespace lbm;
 
@@ -365,15 +364,6 @@ struct SharedBlock {
     int refs = 0;
 };
 
-// One device allocation holding the second buffers (fused pairs) of one solver
-// or of the members of a group.
-struct SecondBlock {
-    void *base = nullptr;
-    size_t bytes = 0;
-    int device = 0;
-    int refs = 0;
-};
-
 struct lbm_solver {
     lbm_solver_config cfg{};
     long long cells = 0, padded = 0;  // padded: cells rounded up to whole layout blocks
@@ -393,11 +383,7 @@ struct lbm_solver {
     size_t staging_bytes = 0;  // largest transfer of a solver in caller-provided memory
     double *d_partials = nullptr;
     size_t partial_count = 0;
-    // second buffer of the fused pairs, allocated by the first run that takes
-    // them; another thread may take it away between runs (SecondBuffers)
-    std::atomic<void *> dd2{nullptr};
-    bool dd2_refused = false;    // there was no memory for it
-    SecondBlock *dd2_block = nullptr;
+    SecondBuffer second;         // of the fused pairs, taken by the first run that uses them
     PairTile *d_pair = nullptr;  // tiles of the fused pairs of a run on its own
     std::vector<PairTile> pair_tiles;  // their copy on the host (the upload reads it)
     int npair = 0;               // their number; 0: not planned yet, -1: this domain steps in place
@@ -520,46 +506,39 @@ struct lbm_group {
 
 namespace {
 
-// The second buffers of the solvers that took fused pairs.  They are a use of
-// memory that nothing depends on: where an allocation of this library fails,
-// they are given back and it is tried again.  Launches that use them hold the
-// mutex shared, so none is enqueued while they are taken away.  The buffers of
-// the last few destroyed solvers are kept for the next ones (an allocation
-// costs a short run more than it gains): at most kSpares, kSpareBytes in all.
-struct SecondBuffers {
-    static constexpr size_t kSpares = 8, kSpareBytes = (size_t)4 << 30;
-    std::shared_mutex mutex;
-    std::set<lbm_solver *> held;
-    std::vector<SecondBlock *> spares;  // oldest first
-    size_t spare_bytes = 0;
+// The device made current for a scope (a run does not need it current, an allocation does).
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int device) {
+        int now = 0;
+        if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) before = now;
+    }
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+
+struct DeviceMemory : SecondMemory {
+    // half of the device's memory is left to others
+    void *allocate(int device, size_t bytes) override {
+        const OnDevice on(device);
+        size_t free_b = 0, total_b = 0;
+        void *p = nullptr;
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b >= bytes + total_b / 2 &&
+            hipMalloc(&p, bytes) == hipSuccess)
+            return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    void release(void *base) override { (void)hipFree(base); }
+    void drain(int device) override {
+        const OnDevice on(device);
+        (void)hipDeviceSynchronize();
+    }
 };
 SecondBuffers &second_buffers() {
-    static SecondBuffers *b = new SecondBuffers();  // outlives every solver
+    static SecondBuffers *b = new SecondBuffers(*new DeviceMemory());  // outlives every solver
     return *b;
-}
-
-// The following hold the mutex exclusively.
-void free_spares(SecondBuffers &sb, size_t keep_bytes, size_t keep) {
-    while (!sb.spares.empty() && (sb.spare_bytes > keep_bytes || sb.spares.size() > keep)) {
-        SecondBlock *b = sb.spares.front();
-        (void)hipFree(b->base);
-        sb.spare_bytes -= b->bytes;
-        sb.spares.erase(sb.spares.begin());
-        delete b;
-    }
-}
-void drop_second(lbm_solver *s) {
-    SecondBuffers &sb = second_buffers();
-    if (!s->dd2) return;
-    s->dd2 = nullptr;
-    s->version++;
-    sb.held.erase(s);
-    SecondBlock *b = s->dd2_block;
-    s->dd2_block = nullptr;
-    if (--b->refs > 0) return;
-    sb.spares.push_back(b);
-    sb.spare_bytes += b->bytes;
-    free_spares(sb, SecondBuffers::kSpareBytes, SecondBuffers::kSpares);
 }
 
 int fail(lbm_solver *s, int code, const std::string &msg) { return record(s ? &s->err : nullptr, code, msg); }
@@ -589,7 +568,7 @@ int dispatch_storage(int storage, F &&f) {
 void fill_desc(lbm_solver *s) {
     DomDev &d = s->host_desc;
     d.dd = s->dd;
-    d.dd2 = s->dd2;
+    d.dd2 = s->second.at;
     d.flags = s->flags;
     d.vel = s->vel;
     d.dens = s->dens;
@@ -755,67 +734,11 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage) {
     return P;
 }
 
-// The device made current for a scope (a run does not need it current, an allocation does).
-struct OnDevice {
-    int before = -1;
-    explicit OnDevice(int device) {
-        int now = 0;
-        if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) before = now;
-    }
-    ~OnDevice() {
-        if (before >= 0) (void)hipSetDevice(before);
-    }
-};
-
-// Gives the solvers (of one device) their second buffers, those without one
-// in a block together; false if they have to do without.  Half of the device's
-// memory is left to others.
+// Second buffers for all of them; false: they have to do without.
 bool take_seconds(const std::vector<lbm_solver *> &solvers) {
-    SecondBuffers &sb = second_buffers();
-    std::unique_lock<std::shared_mutex> lock(sb.mutex);
-    auto size_of = [](const lbm_solver *s) {
-        return ((size_t)19 * s->padded * elem_size(s->cfg.storage) + 255) & ~(size_t)255;
-    };
-    std::vector<lbm_solver *> without;
-    size_t bytes = 0;
-    for (lbm_solver *s : solvers) {
-        if (s->dd2) continue;
-        if (s->dd2_refused) return false;
-        without.push_back(s);
-        bytes += size_of(s);
-    }
-    if (without.empty()) return true;
-    const int device = without[0]->cfg.device;
-    const OnDevice on(device);
-    SecondBlock *b = nullptr;
-    for (auto it = sb.spares.rbegin(); it != sb.spares.rend(); ++it) {
-        if ((*it)->device != device || (*it)->bytes < bytes || (*it)->bytes > 2 * bytes) continue;
-        b = *it;
-        sb.spare_bytes -= b->bytes;
-        sb.spares.erase(std::next(it).base());
-        break;
-    }
-    if (!b) {
-        size_t free_b = 0, total_b = 0;
-        void *p = nullptr;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < bytes + total_b / 2 ||
-            hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            for (lbm_solver *s : without) s->dd2_refused = true;
-            return false;
-        }
-        b = new SecondBlock{p, bytes, device, 0};
-    }
-    size_t off = 0;
-    for (lbm_solver *s : without) {
-        s->dd2_block = b;
-        b->refs++;
-        s->dd2 = (char *)b->base + off;
-        off += size_of(s);
-        sb.held.insert(s);
-        s->version++;
-    }
-    return true;
+    std::vector<SecondBuffer *> all;
+    for (lbm_solver *s : solvers) all.push_back(&s->second);
+    return second_buffers().take(all);
 }
 
 // Second buffer and tile table of a solver stepped on its own; false: the run
@@ -910,17 +833,7 @@ hipError_t lbm_device_malloc(void **p, size_t bytes) {
     (void)hipGetLastError();
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return e;
-    {
-        SecondBuffers &sb = second_buffers();
-        std::unique_lock<std::shared_mutex> lock(sb.mutex);
-        std::vector<lbm_solver *> here;
-        for (lbm_solver *s : sb.held)
-            if (s->cfg.device == device) here.push_back(s);
-        if (here.empty() && sb.spares.empty()) return e;
-        (void)hipDeviceSynchronize();  // launches that still use them
-        for (lbm_solver *s : here) drop_second(s);
-        free_spares(sb, 0, 0);
-    }
+    if (!second_buffers().give_all(device)) return e;
     e = hipMalloc(p, bytes);
     if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
     return e;
@@ -1058,6 +971,9 @@ static int create_solver(const lbm_solver_config *cfg, void *memory, size_t memo
     s->cells = cells;
     s->padded = padded;
     s->ntiles = ntiles;
+    s->second.version = &s->version;
+    s->second.bytes = (size_t)19 * padded * elem_size(c.storage);
+    s->second.device = c.device;
     s->external = memory != nullptr;
     auto bail = [&](int code, const std::string &m) {
         record(nullptr, code, m);
@@ -1145,10 +1061,7 @@ extern "C" int lbm_solver_destroy(lbm_solver *s) {
         (void)hipFree(s->d_tile);
     }
     if (s->d_partials) (void)hipFree(s->d_partials);
-    if (s->dd2) {
-        std::unique_lock<std::shared_mutex> lock(second_buffers().mutex);
-        drop_second(s);
-    }
+    second_buffers().give(s->second);
     if (s->d_pair) (void)hipFree(s->d_pair);
     if (s->own_stream) (void)hipStreamDestroy(s->own_stream);
     delete s;
@@ -1291,9 +1204,9 @@ extern "C" int lbm_solver_run(lbm_solver *s, int steps) {
         ++i;
     }
     if (steps - i >= 4 && (s->step_counter & 1) == 0 && solver_pairs_ready(s)) {
-        std::shared_lock<std::shared_mutex> lock(second_buffers().mutex);
+        const auto lock = second_buffers().in_use();
         // two pairs at a time: into the second buffer and back
-        for (void *two = s->dd2; two && steps - i >= 4; i += 4) {
+        for (void *two = s->second.at; two && steps - i >= 4; i += 4) {
             for (int flip = 0; flip < 2; ++flip)
                 SCHK(launch_pair_kernel(s->cfg.storage, s->pair_launch, s->npair, s->d_desc, s->d_pair, two, s->stream,
                                         nullptr, flip));
@@ -2610,7 +2523,7 @@ static void plan_faces(lbm_group *g) {
 // The tables of plan_faces on the device, for the present second buffers.
 static int upload_faces(lbm_group *g) {
     std::vector<void *> seconds;
-    for (const lbm_solver *m : g->members) seconds.push_back(m->dd2);
+    for (const lbm_solver *m : g->members) seconds.push_back(m->second.at);
     if (seconds == g->face_seconds) return LBM_OK;
     std::vector<LayerBox> boxes;
     std::vector<int> block_box;
@@ -2665,8 +2578,8 @@ static int upload_faces(lbm_group *g) {
                 const int rc = fill_op(from, h.so, to, h.dof, h.sz, h.mask, op, why);
                 if (rc) return gfail(g, rc, why);
                 if (!f) {
-                    op.src = from->dd2;
-                    op.dst = to->dd2;
+                    op.src = from->second.at;
+                    op.dst = to->second.at;
                 }
                 ops[f][k].push_back(op);
             }
@@ -2677,7 +2590,7 @@ static int upload_faces(lbm_group *g) {
     GCHK(hipStreamSynchronize(g->stream));
     // the tables' own allocation may have had to take second buffers away
     for (size_t i = 0; i < seconds.size(); ++i)
-        if (g->members[i]->dd2 != seconds[i]) return LBM_OK;
+        if (g->members[i]->second.at != seconds[i]) return LBM_OK;
     g->face_seconds = seconds;
     return LBM_OK;
 }
@@ -2862,8 +2775,8 @@ static int group_advance(lbm_group *g, int steps, bool run, int *done) {
     int rc = group_pairs_ready(g, steps, &fused);
     if (rc) return rc;
     if (!fused) return group_walk(g, steps, run, false, done);
-    std::shared_lock<std::shared_mutex> lock(second_buffers().mutex);
-    for (const lbm_solver *m : g->members) fused = fused && m->dd2;
+    const auto lock = second_buffers().in_use();
+    for (const lbm_solver *m : g->members) fused = fused && m->second.at;
     return group_walk(g, steps, run, fused, done);
 }
 

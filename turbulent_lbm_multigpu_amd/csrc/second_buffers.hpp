@@ -1,0 +1,151 @@
+// second_buffers.hpp -- the second buffers of the solvers that took fused pairs
+// (pair_kernel).  Plain C++: device memory comes in as SecondMemory, so the
+// bookkeeping, which threads with a solver each share, is checked on the CPU.
+#pragma once
+
+#include <stddef.h>
+
+#include <atomic>
+#include <iterator>
+#include <mutex>
+#include <set>
+#include <shared_mutex>
+#include <vector>
+
+namespace lbm {
+
+// One device allocation holding the second buffers of one solver or of the
+// members of a group.
+struct SecondBlock {
+    void *base = nullptr;
+    size_t bytes = 0;
+    int device = 0;
+    int refs = 0;
+};
+
+// A solver's second buffer.  `at` is read by the solver's own thread; another
+// thread may take it away between launches (give_all).
+struct SecondBuffer {
+    std::atomic<void *> at{nullptr};
+    std::atomic<unsigned> *version = nullptr;  // bumped when `at` changes
+    size_t bytes = 0;                          // what the solver needs
+    int device = 0;
+    bool refused = false;                      // there was no memory for it
+    SecondBlock *block = nullptr;
+};
+
+struct SecondMemory {
+    virtual ~SecondMemory() = default;
+    virtual void *allocate(int device, size_t bytes) = 0;  // null: not to be had
+    virtual void release(void *base) = 0;
+    virtual void drain(int device) = 0;  // waits for the launches that still use them
+};
+
+// They are a use of memory that nothing depends on: where an allocation of
+// this library fails, they are given back and it is tried again.  Launches
+// that use them hold in_use(), so none is enqueued while they are taken away.
+// The blocks of the last few destroyed solvers are kept for the next ones (an
+// allocation costs a short run more than it gains): at most kSpares,
+// kSpareBytes in all.
+class SecondBuffers {
+  public:
+    static constexpr size_t kSpares = 8, kSpareBytes = (size_t)4 << 30;
+    explicit SecondBuffers(SecondMemory &memory) : memory_(memory) {}
+
+    // Gives these (of one device) their second buffers, those without one in a
+    // block together; false if they have to do without.
+    bool take(const std::vector<SecondBuffer *> &all) {
+        std::unique_lock<std::shared_mutex> lock(mutex_);
+        std::vector<SecondBuffer *> without;
+        size_t bytes = 0;
+        for (SecondBuffer *s : all) {
+            if (s->at) continue;
+            if (s->refused) return false;
+            without.push_back(s);
+            bytes += aligned(s->bytes);
+        }
+        if (without.empty()) return true;
+        const int device = without[0]->device;
+        SecondBlock *b = nullptr;
+        for (auto it = spares_.rbegin(); it != spares_.rend(); ++it) {
+            if ((*it)->device != device || (*it)->bytes < bytes || (*it)->bytes > 2 * bytes) continue;
+            b = *it;
+            spare_bytes_ -= b->bytes;
+            spares_.erase(std::next(it).base());
+            break;
+        }
+        if (!b) {
+            void *const p = memory_.allocate(device, bytes);
+            if (!p) {
+                for (SecondBuffer *s : without) s->refused = true;
+                return false;
+            }
+            b = new SecondBlock{p, bytes, device, 0};
+        }
+        size_t off = 0;
+        for (SecondBuffer *s : without) {
+            s->block = b;
+            b->refs++;
+            s->at = (char *)b->base + off;
+            off += aligned(s->bytes);
+            held_.insert(s);
+            (*s->version)++;
+        }
+        return true;
+    }
+
+    // A solver's last call.  The lock is taken before `at` is looked at: while
+    // give_all is at work on this buffer, `at` may be null already with other
+    // members still to be written, and the solver is freed when this returns.
+    void give(SecondBuffer &s) {
+        std::unique_lock<std::shared_mutex> lock(mutex_);
+        drop(s);
+    }
+
+    // Takes away every second buffer and spare of the device; whether there were any.
+    bool give_all(int device) {
+        std::unique_lock<std::shared_mutex> lock(mutex_);
+        std::vector<SecondBuffer *> here;
+        for (SecondBuffer *s : held_)
+            if (s->device == device) here.push_back(s);
+        if (here.empty() && spares_.empty()) return false;
+        memory_.drain(device);
+        for (SecondBuffer *s : here) drop(*s);
+        free_spares(0, 0);
+        return true;
+    }
+
+    std::shared_lock<std::shared_mutex> in_use() { return std::shared_lock<std::shared_mutex>(mutex_); }
+
+  private:
+    static size_t aligned(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+    void free_spares(size_t keep_bytes, size_t keep) {
+        while (!spares_.empty() && (spare_bytes_ > keep_bytes || spares_.size() > keep)) {
+            SecondBlock *b = spares_.front();
+            memory_.release(b->base);
+            spare_bytes_ -= b->bytes;
+            spares_.erase(spares_.begin());
+            delete b;
+        }
+    }
+    void drop(SecondBuffer &s) {
+        if (!s.at) return;
+        s.at = nullptr;
+        (*s.version)++;
+        held_.erase(&s);
+        SecondBlock *b = s.block;
+        s.block = nullptr;
+        if (--b->refs > 0) return;
+        spares_.push_back(b);
+        spare_bytes_ += b->bytes;
+        free_spares(kSpareBytes, kSpares);
+    }
+
+    SecondMemory &memory_;
+    std::shared_mutex mutex_;
+    std::set<SecondBuffer *> held_;
+    std::vector<SecondBlock *> spares_;  // oldest first
+    size_t spare_bytes_ = 0;
+};
+
+}  // namespace lbm
