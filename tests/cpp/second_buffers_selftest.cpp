@@ -73,6 +73,63 @@ static void destroyed_while_taken_away() {
     short_of_memory.join();
 }
 
+// While one thread enqueues a long sequence, another takes and gives back
+// buffers without waiting for it; taking them away waits for the sequence, and
+// does not wait for sequences that begin later.
+static void launches_keep_nobody_waiting() {
+    HostMemory mem;
+    SecondBuffers sb(mem);
+    auto within = [](std::atomic<bool> &done) {
+        for (int k = 0; k < 5000 && !done; ++k) std::this_thread::sleep_for(std::chrono::milliseconds(1));
+        return done.load();
+    };
+    Solver a(1000);
+    CHECK(sb.take({&a.second}));
+    std::atomic<bool> stepped{false}, taken{false}, stop{false};
+    std::thread second, short_of_memory;
+    {
+        const auto enqueuing = sb.in_use();
+        second = std::thread([&] {
+            Solver b(1000);
+            for (int k = 0; k < 2; ++k) {
+                CHECK(sb.take({&b.second}));
+                const auto lock = sb.in_use();
+                CHECK(b.second.at);
+            }
+            sb.give(b.second);
+            stepped = true;
+        });
+        CHECK(within(stepped));
+        short_of_memory = std::thread([&] {
+            sb.give_all(0);
+            taken = true;
+        });
+        std::this_thread::sleep_for(std::chrono::milliseconds(50));
+        CHECK(!taken && a.second.at);
+    }
+    second.join();
+    std::vector<std::thread> busy;  // sequences that overlap without end
+    for (int t = 0; t < 2; ++t)
+        busy.emplace_back([&] {
+            while (!stop) {
+                const auto lock = sb.in_use();
+                std::this_thread::sleep_for(std::chrono::milliseconds(2));
+            }
+        });
+    CHECK(within(taken) && !a.second.at);
+    taken = false;
+    std::thread again([&] {
+        Solver c(100);
+        CHECK(sb.take({&c.second}) && sb.give_all(0));
+        taken = true;
+    });
+    CHECK(within(taken));
+    stop = true;
+    for (std::thread &t : busy) t.join();
+    short_of_memory.join();
+    again.join();
+}
+
 static void blocks_and_spares() {
     HostMemory mem;
     SecondBuffers sb(mem);
@@ -115,6 +172,7 @@ static void blocks_and_spares() {
 
 int main() {
     blocks_and_spares();
+    launches_keep_nobody_waiting();
     destroyed_while_taken_away();
     if (fails) {
         printf("%d failures\n", fails);

@@ -43,7 +43,9 @@ struct SecondMemory {
 
 // They are a use of memory that nothing depends on: where an allocation of
 // this library fails, they are given back and it is tried again.  Launches
-// that use them hold in_use(), so none is enqueued while they are taken away.
+// that use them hold in_use(), so none is enqueued while they are taken away;
+// only that waits for them.  A sequence may be enqueued for as long as it runs
+// (the queue is bounded), and nothing else of one thread waits for another's.
 // The blocks of the last few destroyed solvers are kept for the next ones (an
 // allocation costs a short run more than it gains): at most kSpares,
 // kSpareBytes in all.
@@ -54,8 +56,8 @@ class SecondBuffers {
 
     // Gives these (of one device) their second buffers, those without one in a
     // block together; false if they have to do without.
+    // Under in_use() they may have gone again.
     bool take(const std::vector<SecondBuffer *> &all) {
-        std::unique_lock<std::shared_mutex> lock(mutex_);
         std::vector<SecondBuffer *> without;
         size_t bytes = 0;
         for (SecondBuffer *s : all) {
@@ -65,6 +67,7 @@ class SecondBuffers {
             bytes += aligned(s->bytes);
         }
         if (without.empty()) return true;
+        const std::lock_guard<std::mutex> lock(mutex_);
         const int device = without[0]->device;
         SecondBlock *b = nullptr;
         for (auto it = spares_.rbegin(); it != spares_.rend(); ++it) {
@@ -98,13 +101,15 @@ class SecondBuffers {
     // give_all is at work on this buffer, `at` may be null already with other
     // members still to be written, and the solver is freed when this returns.
     void give(SecondBuffer &s) {
-        std::unique_lock<std::shared_mutex> lock(mutex_);
+        const std::lock_guard<std::mutex> lock(mutex_);
         drop(s);
     }
 
     // Takes away every second buffer and spare of the device; whether there were any.
     bool give_all(int device) {
-        std::unique_lock<std::shared_mutex> lock(mutex_);
+        const std::lock_guard<std::mutex> gate(gate_);
+        const std::unique_lock<std::shared_mutex> none_launching(launches_);
+        const std::lock_guard<std::mutex> lock(mutex_);
         std::vector<SecondBuffer *> here;
         for (SecondBuffer *s : held_)
             if (s->device == device) here.push_back(s);
@@ -115,7 +120,10 @@ class SecondBuffers {
         return true;
     }
 
-    std::shared_lock<std::shared_mutex> in_use() { return std::shared_lock<std::shared_mutex>(mutex_); }
+    std::shared_lock<std::shared_mutex> in_use() {
+        const std::lock_guard<std::mutex> gate(gate_);  // behind a give_all that waits: its turn comes
+        return std::shared_lock<std::shared_mutex>(launches_);
+    }
 
   private:
     static size_t aligned(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
@@ -142,7 +150,9 @@ class SecondBuffers {
     }
 
     SecondMemory &memory_;
-    std::shared_mutex mutex_;
+    std::mutex gate_;
+    std::shared_mutex launches_;
+    std::mutex mutex_;  // of what follows and of every buffer's block
     std::set<SecondBuffer *> held_;
     std::vector<SecondBlock *> spares_;  // oldest first
     size_t spare_bytes_ = 0;
