@@ -9,7 +9,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 from turbulent_lbm_multigpu_amd import _capi  # noqa: E402
-from turbulent_lbm_multigpu_amd.solver import LbmSolver  # noqa: E402
+from turbulent_lbm_multigpu_amd.solver import LbmGroup, LbmSolver  # noqa: E402
 
 F32, F64 = _capi.STORAGE_F32, _capi.STORAGE_F64
 
@@ -57,3 +57,53 @@ def test_threads_with_a_solver_each():
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+def x_chain(dims, n, storage):
+    """n members joined in x."""
+    solvers = [build(dims, storage, i, (8 if i else 1, 8 if i < n - 1 else 1, 1, 1, 1, 1)) for i in range(n)]
+    g = LbmGroup(solvers)
+    size = (1, dims[1], dims[2])
+    for i in range(n):
+        if i:
+            g.add_comm(i, i - 1, (1, 0, 0), (0, 0, 0), size, (1, 0, 0))
+        if i < n - 1:
+            g.add_comm(i, i + 1, (dims[0] - 2, 0, 0), (dims[0] - 1, 0, 0), size, (-1, 0, 0))
+    return g
+
+
+def test_a_stopping_member_joins_a_paired_group():
+    """The plan of the two joined members, who run as pairs, does not outlive
+    the third's arrival, whose stop refuses pairs; nor does the refusal."""
+    dims = (104, 104, 104)
+    a, b = x_chain(dims, 2, F32), x_chain(dims, 2, F32)
+    late = [build((90, 80, 70), F32, 7) for _ in range(2)]
+
+    def both(n):
+        for _ in range(n):
+            a.step(1)
+        b.step(n)
+        a.wait()
+        b.wait()
+        for x, y in zip(a.solvers, b.solvers):
+            same(x, y)
+
+    both(8)
+    for g, s in ((a, late[0]), (b, late[1])):
+        g.add_member(s)
+        g.set_member_stop(2, 30)
+    both(8)
+    for g in (a, b):
+        g.set_launch(128, 3)  # rebuilds the descriptors, not the plan
+        g.set_alpha_work_group(256)
+    both(8)
+    for g in (a, b):
+        g.set_member_stop(2, -1)
+    both(8)
+    for g in (a, b):
+        g.remove_member(2)
+    both(8)
+    for g in (a, b):
+        g.close()
+    for s in a.solvers + b.solvers + late:
+        s.close()

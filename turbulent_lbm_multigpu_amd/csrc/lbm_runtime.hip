@@ -20,6 +20,7 @@
 #include "../../include/lbm_capi.h"
 #include "device_memory.hpp"
 #include "exchange_plan.hpp"
+#include "face_plan.hpp"
 #include "host_lanes.hpp"
 #include "launch_shape.hpp"
 #include "lbm_device.hpp"
@@ -395,11 +396,6 @@ struct lbm_solver {
     long long stop_at = std::numeric_limits<long long>::max();  // group half-step index of its freeze
 };
 
-struct GroupComm {
-    int member, dst;
-    int send_origin[3], recv_origin[3], size[3], normal[3];
-};
-
 // The launch tables of one work-group size: member descriptors (with their
 // tile ranges), the tile -> member or chain map, and the chain descriptors.
 struct LaunchTables {
@@ -441,27 +437,23 @@ struct lbm_group {
     size_t pair_cap = 0;
     int npair = 0;               // 0: not planned for the present members
     PairLaunch pair_launch{};
-    // Fused pairs of members that exchange faces: per member the faces
-    // (DomDev::layers), the boxes of the layers and, per block, its box, and
-    // the copies after beta ([1]) and alpha ([0]) in the buffer that a pair
-    // ends in ([flip]), with the second buffers they were made for.
-    bool faces_planned = false, faces_pair = false;
-    std::vector<unsigned> layers;
+    // Fused pairs of members that exchange faces: their plan, on the device the
+    // boxes of the layers and, per block, its box, and the copies after beta
+    // ([1]) and alpha ([0]) in the buffer that a pair ends in ([flip]), with the
+    // second buffers they were made for.
+    bool faces_planned = false;
+    FacePlan faces;
     LayerBox *d_layers = nullptr;
     size_t layers_cap = 0;
     int nlayers = 0, layer_blocks = 0;
-    bool seams = false;  // x faces inside pair_kernel: seam_beta_kernel's faces and, per block, its face, and its results
-    SeamFace *d_seams = nullptr;
+    SeamFace *d_seams = nullptr;  // seam_beta_kernel's faces and, per block, its face, and its results
     size_t seams_cap = 0;
     int nseams = 0, seam_blocks = 0;
     char *d_seam_slots = nullptr;
-    size_t seam_slots_cap = 0, seam_bytes = 0;
-    std::vector<size_t> seam_at;  // per member and side, where its part of them starts
-    std::vector<int> seam_nb;     // and the member beyond
+    size_t seam_slots_cap = 0;
     CopyOp *d_face_ops[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     size_t face_cap[2][2] = {{0, 0}, {0, 0}};
     int nface[2] = {0, 0}, face_blocks[2] = {0, 0};
-    std::vector<HOp> face_hops[2];
     std::vector<void *> face_seconds;
     std::vector<unsigned> seen_versions;
     std::vector<GroupComm> comms;
@@ -1761,6 +1753,7 @@ static void group_free_plan(lbm_group *g) {
         }
     g->face_seconds.clear();
     g->faces_planned = false;
+    g->faces = FacePlan{};
     for (int k = 0; k < 2; ++k)
         for (int p = 0; p < 4; ++p) {
             if (g->d_ops[k][p]) (void)hipFree(g->d_ops[k][p]);
@@ -1818,15 +1811,16 @@ static int build_tables(lbm_group *g, int wg, LaunchTables &T) {
         descs[i] = m->host_desc;
         if (i < g->xfuse.size())
             for (int side = 0; side < 2; ++side) descs[i].xmask_a[side] = g->xfuse[i].mask[side];
-        if (i < g->layers.size()) {
-            descs[i].layers = g->layers[i];
-            if (g->seams) {
+        if (i < g->faces.layers.size()) {
+            const FacePlan &P = g->faces;
+            descs[i].layers = P.layers[i];
+            if (P.seams) {
                 descs[i].seam = g->d_seam_slots;
-                descs[i].seam_bytes = (unsigned)g->seam_bytes;
+                descs[i].seam_bytes = (unsigned)P.seam_bytes;
                 descs[i].seam_all = g->exchange_mode != 1;
                 for (int side = 0; side < 2; ++side) {
-                    descs[i].seam_at[side] = (unsigned)g->seam_at[2 * i + side];
-                    descs[i].seam_nb[side] = g->seam_nb[2 * i + side];
+                    descs[i].seam_at[side] = (unsigned)P.seam_at[2 * i + side];
+                    descs[i].seam_nb[side] = P.seam_nb[2 * i + side];
                 }
             }
         }
@@ -2216,29 +2210,6 @@ static void plan_chains(lbm_group *g, const std::vector<char> &fuse) {
     }
 }
 
-// The counterpart of a comm: its partner's comm across the same face.
-static const GroupComm *partner_of(const lbm_group *g, const GroupComm &c) {
-    for (const GroupComm &q : g->comms)
-        if (q.member == c.dst && q.dst == c.member && q.normal[0] == -c.normal[0] && q.normal[1] == -c.normal[1] &&
-            q.normal[2] == -c.normal[2])
-            return &q;
-    return nullptr;
-}
-
-// The two copies of a comm and its counterpart: [0] after alpha, [1] after beta.
-static void comm_copies(const lbm_group *g, const GroupComm &c, const GroupComm &p, HOp *h) {
-    h[0] = HOp{c.dst, c.member, {}, {}, {}, alpha_mask(g, c)};
-    // after beta: neighbour's ghost layer -> my inner layer, n.e > 0 only (src/CController.hpp:322-383)
-    h[1] = HOp{c.dst, c.member, {}, {}, {}, norm_mask(c.normal)};
-    for (int ax = 0; ax < 3; ++ax) {
-        h[0].so[ax] = p.send_origin[ax];
-        h[0].dof[ax] = c.recv_origin[ax];
-        h[1].so[ax] = p.recv_origin[ax];
-        h[1].dof[ax] = c.send_origin[ax];
-        h[0].sz[ax] = h[1].sz[ax] = c.size[ax];
-    }
-}
-
 // A table of copies on the device: the ops, then the op index of every block
 // (exchange_kernel).  The host vectors are read until the stream is waited for.
 static int upload_ops(lbm_group *g, std::vector<CopyOp> &ops, std::vector<int> &block_op, CopyOp *&d_ops, size_t &cap,
@@ -2270,7 +2241,7 @@ static int build_plan(lbm_group *g) {
     std::vector<char> fuse(g->comms.size(), 0);
     for (size_t ci = 0; ci < g->comms.size(); ++ci) {
         const GroupComm &c = g->comms[ci];
-        partner[ci] = partner_of(g, c);
+        partner[ci] = partner_of(g->comms, c);
         if (!partner[ci])
             return gfail(g, LBM_ERR_STATE,
                          "comm of member " + std::to_string(c.member) + " toward " + std::to_string(c.dst) +
@@ -2287,7 +2258,7 @@ static int build_plan(lbm_group *g) {
         const bool fused = fuse[ci] && g->xfuse[c.member].nb[c.normal[0] == 1 ? 0 : 1] == c.dst;
         const int slot = fused ? 3 : axis;
         HOp copies[2];
-        comm_copies(g, c, *p, copies);
+        comm_copies(c, *p, alpha_mask(g, c), norm_mask(c.normal), copies);
         const HOp &a = copies[0], &b = copies[1];
         // each box is checked against both subdomains before any merging
         CopyOp chk;
@@ -2329,8 +2300,8 @@ static int build_plan(lbm_group *g) {
     GCHK(hipStreamSynchronize(g->stream));
     g->plan_built = true;
     g->faces_planned = false;
+    g->faces = FacePlan{};
     g->face_seconds.clear();
-    g->layers.clear();
     g->descs_dirty = true;  // the descriptors carry the fused faces
     return LBM_OK;
 }
@@ -2432,91 +2403,17 @@ static void group_advance_counters(lbm_group *g, long long before, long long don
     g->step_counter = before + done;
 }
 
-// Whether members that exchange faces can run as fused pairs: every comm joins
-// a whole face, ghost layer and the one next to it, with its counterpart, no
-// member stops, and the copies of the three axes resolve to one set.  In such
-// a pair the cells of the layers, whose alpha needs the exchange after beta,
-// keep beta's values in the new buffer; there follow the copies after beta,
-// alpha of the layers (layer_alpha_kernel) and the copies after alpha.  x faces
-// are pair_kernel's own (SeamRows).  256^3 FP32 in 2x2x2: pair_kernel 620 us,
-// before it seam_beta_kernel 89, after it 12 + 13 + 9, where beta, alpha and
-// two copies in place took 858.
-static void plan_faces(lbm_group *g) {
+static void group_plan_faces(lbm_group *g) {
+    std::vector<std::array<int, 3>> dims;
+    bool stops = false;
+    for (const lbm_solver *m : g->members) {
+        dims.push_back({m->cfg.dims[0], m->cfg.dims[1], m->cfg.dims[2]});
+        stops |= m->stop_at != std::numeric_limits<long long>::max();
+    }
+    g->faces = plan_faces(dims, stops, g->comms, elem_size(g->storage), [g](const GroupComm &c, int k) {
+        return k ? norm_mask(c.normal) : alpha_mask(g, c);
+    });
     g->faces_planned = true;
-    g->faces_pair = false;
-    g->layers.assign(g->members.size(), 0u);
-    std::vector<HOp> phase[2][3];
-    for (const lbm_solver *m : g->members)
-        if (m->stop_at != std::numeric_limits<long long>::max()) return;
-    for (const GroupComm &c : g->comms) {
-        const GroupComm *p = partner_of(g, c);
-        const int a = c.normal[0] ? 0 : c.normal[1] ? 1 : 2, side = c.normal[a] == 1 ? 0 : 1;
-        for (const GroupComm *q : {&c, p}) {
-            const int *d = g->members[q->member]->cfg.dims;
-            const bool low = q->normal[a] == 1;
-            for (int ax = 0; ax < 3; ++ax) {
-                if (q->normal[ax] != (ax == a ? (low ? 1 : -1) : 0)) return;
-                if (q->size[ax] != (ax == a ? 1 : d[ax])) return;
-                if (q->send_origin[ax] != (ax != a ? 0 : low ? 1 : d[a] - 2)) return;
-                if (q->recv_origin[ax] != (ax != a ? 0 : low ? 0 : d[a] - 1)) return;
-            }
-            if (d[a] < 4) return;
-        }
-        g->layers[(size_t)c.member] |= 1u << (2 * a + side);
-        HOp h[2];
-        comm_copies(g, c, *p, h);
-        for (int k = 0; k < 2; ++k) phase[k][a].push_back(h[k]);
-    }
-    for (int k = 0; k < 2; ++k) {
-        g->face_hops[k].clear();
-        if (!merge_phases(phase[k], g->face_hops[k])) return;
-    }
-    // The columns of x faces lie a row apart, each in a cache line of its own, so
-    // going through them again costs far more than their cells (with copies and
-    // layer_alpha_kernel for them too, those took 194 us of the above pair, not
-    // 34): pair_kernel exchanges them itself, in the rows that both sides of
-    // every x face step this way.
-    g->seams = true;
-    for (const GroupComm &c : g->comms) {
-        if (!c.normal[0]) continue;
-        const lbm_solver *m = g->members[c.member], *n = g->members[c.dst];
-        for (int ax = 0; ax < 3; ++ax) g->seams = g->seams && m->cfg.dims[ax] == n->cfg.dims[ax];
-        g->seams = g->seams && (g->layers[(size_t)c.member] >> 2) == (g->layers[(size_t)c.dst] >> 2);
-    }
-    g->seam_at.assign(2 * g->members.size(), 0);
-    g->seam_nb.assign(2 * g->members.size(), 0);
-    for (const GroupComm &c : g->comms)
-        if (c.normal[0]) g->seam_nb[2 * (size_t)c.member + (c.normal[0] == 1 ? 0 : 1)] = c.dst;
-    g->seam_bytes = 0;
-    for (size_t i = 0; i < g->members.size(); ++i)
-        for (int side = 0; side < 2; ++side) {
-            if (!(g->layers[i] >> side & 1u)) continue;
-            const int *d = g->members[i]->cfg.dims;
-            g->seam_at[2 * i + side] = g->seam_bytes;
-            const int n = SeamRows(g->layers[i], d[1], d[2]).count();
-            if (n <= 0 || SeamRows(g->layers[i], d[1], d[2]).ny <= 0) g->seams = false;
-            g->seam_bytes += (size_t)kSeamPops * std::max(n, 0) * elem_size(g->storage);
-        }
-    if (g->seam_bytes == 0 || g->seam_bytes >= (size_t)1 << 31) g->seams = false;
-    // the copies in those rows are that kernel's
-    for (int k = 0; k < 2 && g->seams; ++k) {
-        std::vector<HOp> kept;
-        for (const HOp &h : g->face_hops[k]) {
-            const int *d = g->members[(size_t)h.dm]->cfg.dims;
-            const SeamRows R(g->layers[(size_t)h.dm], d[1], d[2]);
-            const int o[3] = {0, R.y0, R.z0}, sz[3] = {d[0], R.ny, R.nz};
-            int io[3], is[3];
-            if (!box_isect(h.dof, h.sz, o, sz, io, is)) {
-                kept.push_back(h);
-                continue;
-            }
-            std::vector<std::array<int, 6>> rest;
-            box_minus(h.dof, h.sz, io, is, rest);
-            for (const auto &b : rest) kept.push_back(op_at_dst(h, &b[0], &b[3]));
-        }
-        g->face_hops[k].swap(kept);
-    }
-    g->faces_pair = true;
     g->descs_dirty = true;  // the descriptors carry the layers
 }
 
@@ -2527,7 +2424,7 @@ static int upload_faces(lbm_group *g) {
     if (seconds == g->face_seconds) return LBM_OK;
     std::vector<LayerBox> boxes;
     std::vector<int> block_box;
-    for (size_t i = 0; i < g->members.size(); ++i) layer_boxes((int)i, g->layers[i], g->members[i]->cfg.dims, g->seams, boxes);
+    for (size_t i = 0; i < g->members.size(); ++i) layer_boxes((int)i, g->faces.layers[i], g->members[i]->cfg.dims, g->faces.seams, boxes);
     for (size_t i = 0; i < boxes.size(); ++i) {
         boxes[i].block_begin = (int)block_box.size();
         const long long n = (long long)boxes[i].s[0] * boxes[i].s[1] * boxes[i].s[2];
@@ -2546,9 +2443,9 @@ static int upload_faces(lbm_group *g) {
     std::vector<SeamFace> faces;
     std::vector<int> block_face;
     for (const GroupComm &c : g->comms) {
-        if (!g->seams || !c.normal[0]) continue;
+        if (!g->faces.seams || !c.normal[0]) continue;
         const int *d = g->members[(size_t)c.member]->cfg.dims;
-        const SeamRows R(g->layers[(size_t)c.member], d[1], d[2]);
+        const SeamRows R(g->faces.layers[(size_t)c.member], d[1], d[2]);
         const int n = (R.ny + 2) * (R.nz + 2);
         faces.push_back(SeamFace{c.member, c.normal[0] == 1 ? 0 : 1, c.dst, (int)block_face.size()});
         block_face.insert(block_face.end(), (size_t)((n + 255) / 256), (int)faces.size() - 1);
@@ -2556,7 +2453,7 @@ static int upload_faces(lbm_group *g) {
     const size_t face_extra = (sizeof(int) * block_face.size() + sizeof(SeamFace) - 1) / sizeof(SeamFace);
     GCHK(grow_table(g->d_seams, g->seams_cap, faces.size() + face_extra));
     void *const slots = g->d_seam_slots;
-    GCHK(grow_table(g->d_seam_slots, g->seam_slots_cap, g->seams ? g->seam_bytes : 1));
+    GCHK(grow_table(g->d_seam_slots, g->seam_slots_cap, g->faces.seams ? g->faces.seam_bytes : 1));
     if (slots != g->d_seam_slots) g->descs_dirty = true;
     g->nseams = (int)faces.size();
     g->seam_blocks = (int)block_face.size();
@@ -2570,7 +2467,7 @@ static int upload_faces(lbm_group *g) {
     std::vector<int> block_op[2][2];
     for (int f = 0; f < 2; ++f)
         for (int k = 0; k < 2; ++k) {
-            for (const HOp &h : g->face_hops[k]) {
+            for (const HOp &h : g->faces.hops[k]) {
                 if (!h.mask) continue;
                 CopyOp op;
                 std::string why;
@@ -2613,8 +2510,8 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
         if (!face_pairs_pay(g->members, g->storage, x_only)) return LBM_OK;
         int rc = group_prepare(g);  // refuses comms without a counterpart
         if (rc) return rc;
-        if (!g->faces_planned) plan_faces(g);
-        if (!g->faces_pair) return LBM_OK;
+        if (!g->faces_planned) group_plan_faces(g);
+        if (!g->faces.pairs()) return LBM_OK;
     }
     if (!take_seconds(g->members)) return LBM_OK;
     if (!g->comms.empty()) {
