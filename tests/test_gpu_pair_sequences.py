@@ -1,6 +1,8 @@
 """What surrounds the fused pairs of a step sequence: threads with a solver
-each, changes of a group between sequences.  Stated tolerance: 0, every stored
-bit against single steps, which launch the half-step kernels."""
+each, changes of a group between sequences, a caller's recording.  Stated
+tolerance: 0, every stored bit against single steps, which launch the half-step
+kernels."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -8,7 +10,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-from turbulent_lbm_multigpu_amd import _capi  # noqa: E402
+from turbulent_lbm_multigpu_amd import _capi, serving  # noqa: E402
 from turbulent_lbm_multigpu_amd.solver import LbmGroup, LbmSolver  # noqa: E402
 
 F32, F64 = _capi.STORAGE_F32, _capi.STORAGE_F64
@@ -106,4 +108,45 @@ def test_a_stopping_member_joins_a_paired_group():
     for g in (a, b):
         g.close()
     for s in a.solvers + b.solvers + late:
+        s.close()
+
+
+@pytest.mark.parametrize("paired_before", [False, True])
+def test_a_recorded_sequence_steps_in_place(paired_before):
+    """A caller who records the group's stream gets launches that do not
+    depend on second buffers: replays after these are gone, with eager steps
+    in between, are still the same."""
+    dims, sizes = (96, 90, 88), 2
+    a, b = [build(dims, F32, k) for k in range(sizes)], [build(dims, F32, k) for k in range(sizes)]
+    g = LbmGroup(b)
+    g.set_graph(False)
+    first = 8 if paired_before else 2
+    g.step(first)
+    g.wait()
+    lib, stream = _capi.load_library(), C.c_void_p()
+    assert lib.lbm_group_get_stream(g._h, C.byref(stream)) == 0
+    graph, replay = C.c_void_p(), C.c_void_p()
+    assert lib.hipStreamBeginCapture(stream, 1) == 0
+    g.step(8)
+    assert lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert lib.hipGraphInstantiate(C.byref(replay), graph, None, None, C.c_size_t(0)) == 0
+    n = first
+    for k in range(4):
+        assert lib.hipGraphLaunch(replay, stream) == 0
+        g.wait()
+        n += 8
+        if k == 1:
+            with pytest.raises(_capi.LbmError):
+                serving.Server(4e12)  # takes the second buffers away
+        if k % 2:
+            g.step(2)
+            g.wait()
+            n += 2
+        for x in a:
+            single_steps(x, n - x.step_counter)
+        for x, y in zip(a, b):
+            np.testing.assert_array_equal(x.store(_capi.FIELD_DD_RAW), y.store(_capi.FIELD_DD_RAW))
+    assert lib.hipGraphExecDestroy(replay) == 0 and lib.hipGraphDestroy(graph) == 0
+    g.close()
+    for s in a + b:
         s.close()

@@ -726,6 +726,15 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage) {
     return P;
 }
 
+// Whether a caller records the stream: what is recorded steps in place, for a
+// replay would not know that the second buffers it wrote to are gone.
+bool recording(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Second buffers for all of them; false: they have to do without.
 bool take_seconds(const std::vector<lbm_solver *> &solvers) {
     std::vector<SecondBuffer *> all;
@@ -736,7 +745,7 @@ bool take_seconds(const std::vector<lbm_solver *> &solvers) {
 // Second buffer and tile table of a solver stepped on its own; false: the run
 // steps in place.
 bool solver_pairs_ready(lbm_solver *s) {
-    if (s->external || s->npair < 0) return false;  // no memory beyond the caller's
+    if (s->external || s->npair < 0 || recording(s->stream)) return false;  // no memory beyond the caller's
     if (!s->d_pair) {
         PairPlan P = plan_pairs({s}, s->cfg.storage);
         s->npair = P.tiles.empty() ? -1 : (int)P.tiles.size();
@@ -2499,7 +2508,7 @@ static int upload_faces(lbm_group *g) {
 // the wrong buffer).  Brings the pair tiles and descriptors up to date.
 static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
     *ready = false;
-    if (steps < 4 || g->timing || !walks_pay(g->members, g->storage)) return LBM_OK;
+    if (steps < 4 || g->timing || !walks_pay(g->members, g->storage) || recording(g->stream)) return LBM_OK;
     for (const lbm_solver *m : g->members)
         if (m->external) return LBM_OK;
     for (const lbm_solver *m : g->members)
