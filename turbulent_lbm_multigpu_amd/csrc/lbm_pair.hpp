@@ -15,6 +15,7 @@
 #include <limits>
 
 #include "lbm_device.hpp"
+#include "once_per_device.hpp"
 #include "pair_plan.hpp"
 
 namespace lbm {
@@ -594,37 +595,45 @@ __global__ void __launch_bounds__(NT)
     }
 }
 
+// Calls f(kernel, work-items, bytes of LDS) with the kernel of a launch.
+template <int ST, class F>
+hipError_t with_pair_kernel(const PairLaunch &L, F &&f) {
+    constexpr int per_cell = 19 * (int)Storage<ST>::kBytes + 1;
+    constexpr int NT = ST == 1 ? 512 : 1024;
+    constexpr int NB = box_threads(ST), CB = box_large(ST);
+    if (L.box_cells == kBoxSmall) return f(pair_box_kernel<ST, kBoxSmall, kBoxSmall>, kBoxSmall, kBoxSmall * per_cell);
+    if (L.box_cells == CB) return f(pair_box_kernel<ST, NB, CB>, NB, CB * per_cell);
+    if (L.box_cells > 0) return hipErrorInvalidValue;
+    if (L.layers) return f(pair_kernel<ST, NT, true>, NT, 2 * NT * per_cell);
+    return f(pair_kernel<ST, NT, false>, NT, 2 * NT * per_cell);
+}
+
+// Lets the kernel of a launch use its LDS, on the current device: the
+// attribute belongs to the function as it is loaded there.
+template <int ST>
+hipError_t allow_pair_lds(const PairLaunch &L, int device) {
+    static OncePerDevice once;
+    return with_pair_kernel<ST>(L, [&](auto *kernel, int, int lds) -> hipError_t {
+        hipError_t e = hipSuccess;
+        once((const void *)kernel, device, [&] {
+            e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            return e == hipSuccess;
+        });
+        return e;
+    });
+}
+
 // Launch of a pair kernel: beta and alpha of every tile from one buffer into
 // the other (flip 0: from dd, 1: back into it).  `second`: the second buffer
 // of a single domain, or null for the one its descriptor names.
 template <int ST>
 hipError_t launch_pair_storage(const PairLaunch &L, int ntiles, const DomDev *descs, const PairTile *tiles,
                                void *second, hipStream_t stream, long long *ctr, int flip) {
-    constexpr int per_cell = 19 * (int)Storage<ST>::kBytes + 1;
-    auto go = [&](auto *kernel, int threads, int lds, hipError_t attr) -> hipError_t {
-        if (attr != hipSuccess) return attr;
+    return with_pair_kernel<ST>(L, [&](auto *kernel, int threads, int lds) -> hipError_t {
         if (L.threads != threads) return hipErrorInvalidValue;
         kernel<<<ntiles, threads, lds, stream>>>(descs, tiles, second, flip, L.xcd_map, ctr);
         return hipGetLastError();
-    };
-#define LBM_PAIR_GO(kernel, threads, lds)                                                                            \
-    do {                                                                                                              \
-        static const hipError_t attr =                                                                                \
-            hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);               \
-        return go(kernel, threads, lds, attr);                                                                        \
-    } while (0)
-    if (L.box_cells == kBoxSmall) LBM_PAIR_GO((pair_box_kernel<ST, kBoxSmall, kBoxSmall>), kBoxSmall, kBoxSmall * per_cell);
-    if (L.box_cells > 0) {
-        if (L.box_cells != box_large(ST)) return hipErrorInvalidValue;
-        LBM_PAIR_GO((pair_box_kernel<ST, box_threads(ST), box_large(ST)>), box_threads(ST), box_large(ST) * per_cell);
-    }
-    if constexpr (ST < 2) {
-        constexpr int NT = ST == 1 ? 512 : 1024;
-        if (L.layers) LBM_PAIR_GO((pair_kernel<ST, NT, true>), NT, 2 * NT * per_cell);
-        LBM_PAIR_GO((pair_kernel<ST, NT, false>), NT, 2 * NT * per_cell);
-    }
-    return hipErrorInvalidValue;
-#undef LBM_PAIR_GO
+    });
 }
 
 }  // namespace lbm

@@ -735,6 +735,15 @@ bool recording(hipStream_t stream) {
     return true;
 }
 
+// Whether the launch's kernel can run on the device (its LDS is more than a
+// kernel gets unasked).
+bool pair_kernel_ready(int storage, const PairLaunch &L, int device) {
+    const OnDevice on(device);
+    const hipError_t e = storage == LBM_STORAGE_F32 ? allow_pair_lds<0>(L, device) : allow_pair_lds<1>(L, device);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
 // Second buffers for all of them; false: they have to do without.
 bool take_seconds(const std::vector<lbm_solver *> &solvers) {
     std::vector<SecondBuffer *> all;
@@ -765,7 +774,7 @@ bool solver_pairs_ready(lbm_solver *s) {
         }
         s->pair_launch = P.launch;
     }
-    return take_seconds({s});
+    return pair_kernel_ready(s->cfg.storage, s->pair_launch, s->cfg.device) && take_seconds({s});
 }
 
 int launch_step(lbm_solver *s, bool beta) {
@@ -2537,6 +2546,7 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
         g->pair_launch = P.launch;
     }
     g->pair_launch.layers = !g->comms.empty();
+    if (!pair_kernel_ready(g->storage, g->pair_launch, g->device)) return LBM_OK;
     int rc = group_prepare(g);  // the descriptors carry the second buffers
     if (rc) return rc;
     *ready = true;
