@@ -153,6 +153,9 @@ int lbm_solver_simulation_step_beta(lbm_solver *s);
  * lbm_group_step's (same results; taken only while half the device's memory
  * stays free, given up when an allocation of this library fails) */
 int lbm_solver_run(lbm_solver *s, int steps);
+/* pairs that lbm_solver_run has launched that way so far (two half-steps
+ * each), and whether the solver holds a second buffer now (new) */
+int lbm_solver_get_pair_count(const lbm_solver *s, long long *pairs, int *second_buffer);
 /* wait(): clFinish (src/CLbmSolver.hpp:681-683) */
 int lbm_solver_wait(lbm_solver *s);
 int lbm_solver_get_step_counter(const lbm_solver *s, long long *out);
@@ -253,6 +256,9 @@ int lbm_group_prepare_steps(lbm_group *g, int steps);
  * launched without a graph, and graphs captured (new) */
 int lbm_group_get_launch_counts(const lbm_group *g, long long *graph_launches, long long *eager_half_steps,
                                 long long *graphs_captured);
+/* pairs of half-steps that lbm_group_step has launched through the members'
+ * second buffers so far (see lbm_solver_run; new) */
+int lbm_group_get_pair_count(const lbm_group *g, long long *pairs);
 /* computeNextStep() for all members, `steps` times (src/CController.hpp:385-391) */
 int lbm_group_step(lbm_group *g, int steps);
 /* one exchange on its own: syncAlpha (after_beta = 0) or syncBeta

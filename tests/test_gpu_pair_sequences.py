@@ -150,3 +150,65 @@ def test_a_recorded_sequence_steps_in_place(paired_before):
     g.close()
     for s in a + b:
         s.close()
+
+
+# Domains whose sequences take pairs: walks, then boxes.
+@pytest.mark.parametrize("dims,storage", [((83, 79, 77), F32), ((150, 141, 133), F32), ((61, 67, 63), F64),
+                                          ((24, 20, 16), F32), ((16, 16, 16), F64)])
+def test_sequences_take_pairs(dims, storage):
+    a, b = build(dims, storage), build(dims, storage)
+    assert b.pair_count() == {"pairs": 0, "second_buffer": False}
+    b.run(3)
+    assert b.pair_count() == {"pairs": 0, "second_buffer": False}  # too short
+    b.run(12)  # on an odd step: one half-step, then 2 x 2 pairs, then three half-steps
+    assert b.pair_count() == {"pairs": 4, "second_buffer": True}
+    b.step()
+    b.run(8)
+    assert b.pair_count()["pairs"] == 8
+    single_steps(a, 24)
+    assert a.pair_count() == {"pairs": 0, "second_buffer": False}
+    same(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_groups_take_pairs(graph):
+    """With and without exchange, in graphs and launched one by one."""
+    free = LbmGroup([build((96, 70, 64), F32, k) for k in range(3)])
+    joined = x_chain((104, 104, 104), 2, F32)
+    two = LbmGroup([build((60, 70, 64), F64, k) for k in range(3)])
+    for g in (free, joined, two):
+        g.set_graph(graph)
+        g.step(2)
+        assert g.pair_count() == 0
+        g.step(10)  # five pairs, of which the last has none to go back with
+        assert g.pair_count() == 4
+        g.step(64)
+        assert g.pair_count() == 36
+        g.set_timing(True)  # times the half-step kernels
+        g.step(8)
+        assert g.pair_count() == 36
+        g.set_timing(False)
+        assert all(s.pair_count() == {"pairs": 0, "second_buffer": True} for s in g.solvers)
+        g.close()
+        for s in g.solvers:
+            s.close()
+
+
+def test_a_failed_allocation_takes_the_second_buffers():
+    """They are held, gone after an allocation that does not fit, and taken
+    again by the next sequence."""
+    a, b = build((96, 90, 88), F32), build((96, 90, 88), F32)
+    for k in range(2):
+        b.run(8)
+        assert b.pair_count() == {"pairs": 4 * (k + 1), "second_buffer": True}
+        with pytest.raises(_capi.LbmError):
+            serving.Server(4e12)
+        assert not b.pair_count()["second_buffer"]
+    b.run(8)
+    assert b.pair_count() == {"pairs": 12, "second_buffer": True}
+    single_steps(a, 24)
+    same(a, b)
+    a.close()
+    b.close()

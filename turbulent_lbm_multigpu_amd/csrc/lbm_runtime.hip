@@ -389,6 +389,7 @@ struct lbm_solver {
     std::vector<PairTile> pair_tiles;  // their copy on the host (the upload reads it)
     int npair = 0;               // their number; 0: not planned yet, -1: this domain steps in place
     PairLaunch pair_launch{};
+    long long fused_pairs = 0;   // pairs its runs have launched
     std::atomic<unsigned> version{0};  // bumps when kernel parameters change
     lbm_group *group = nullptr;
     bool external = false;     // buffers live in caller-provided device memory
@@ -486,6 +487,7 @@ struct lbm_group {
     long long graph_launches = 0;        // hipGraphLaunch calls of lbm_group_step
     long long eager_half_steps = 0;      // half-steps lbm_group_step launched without a graph
     long long graphs_captured = 0;       // graphs captured and instantiated
+    long long fused_pairs = 0;           // pairs launched as such, in graphs or not
     bool timing = false;
     struct Ev {
         hipEvent_t a, b;
@@ -1221,6 +1223,7 @@ extern "C" int lbm_solver_run(lbm_solver *s, int steps) {
                 SCHK(launch_pair_kernel(s->cfg.storage, s->pair_launch, s->npair, s->d_desc, s->d_pair, two, s->stream,
                                         nullptr, flip));
             s->step_counter += 4;
+            s->fused_pairs += 2;
         }
     }
     for (; i < steps; ++i) {
@@ -2659,6 +2662,7 @@ static int group_walk(lbm_group *g, int steps, bool run, bool fused, int *done_o
             if (run) {
                 GCHK(hipGraphLaunch(exec, g->stream));
                 g->graph_launches += 1;
+                if (fused && P >= 2) g->fused_pairs += P / 2 * 2;
             }
             h += 2 * P;
             done += 2 * P;
@@ -2667,6 +2671,7 @@ static int group_walk(lbm_group *g, int steps, bool run, bool fused, int *done_o
                 int rc = group_launch_two_pairs(g);
                 if (rc) return rc;
                 g->eager_half_steps += 4;
+                g->fused_pairs += 2;
             }
             h += 4;
             done += 4;
@@ -2731,6 +2736,19 @@ extern "C" int lbm_group_get_launch_counts(const lbm_group *g, long long *graph_
     if (graph_launches) *graph_launches = g->graph_launches;
     if (eager_half_steps) *eager_half_steps = g->eager_half_steps;
     if (graphs_captured) *graphs_captured = g->graphs_captured;
+    return LBM_OK;
+}
+
+extern "C" int lbm_solver_get_pair_count(const lbm_solver *s, long long *pairs, int *second_buffer) {
+    if (!s) return record(nullptr, LBM_ERR_INVALID_ARGUMENT, "null solver");
+    if (pairs) *pairs = s->fused_pairs;
+    if (second_buffer) *second_buffer = s->second.at != nullptr;
+    return LBM_OK;
+}
+
+extern "C" int lbm_group_get_pair_count(const lbm_group *g, long long *pairs) {
+    if (!g || !pairs) return record(nullptr, LBM_ERR_INVALID_ARGUMENT, "null argument");
+    *pairs = g->fused_pairs;
     return LBM_OK;
 }
 

@@ -136,6 +136,12 @@ class LbmSolver:
     def run(self, steps: int):
         self._check(self._lib.lbm_solver_run(self._h, int(steps)))
 
+    def pair_count(self) -> dict:
+        """Fused pairs run() has launched so far, and whether a second buffer is held."""
+        n, held = C.c_longlong(), C.c_int()
+        self._check(self._lib.lbm_solver_get_pair_count(self._h, C.byref(n), C.byref(held)))
+        return {"pairs": n.value, "second_buffer": bool(held.value)}
+
     def wait(self):
         self._check(self._lib.lbm_solver_wait(self._h))
 
@@ -341,6 +347,12 @@ class LbmGroup:
         a, b, c = C.c_longlong(), C.c_longlong(), C.c_longlong()
         self._check(self._lib.lbm_group_get_launch_counts(self._h, C.byref(a), C.byref(b), C.byref(c)))
         return {"graph_launches": a.value, "eager_half_steps": b.value, "graphs_captured": c.value}
+
+    def pair_count(self) -> int:
+        """Fused pairs step() has launched so far, in graphs or not."""
+        n = C.c_longlong()
+        self._check(self._lib.lbm_group_get_pair_count(self._h, C.byref(n)))
+        return n.value
 
     def step(self, steps: int = 1):
         self._check(self._lib.lbm_group_step(self._h, int(steps)))
