@@ -1,0 +1,89 @@
+// Checks the choice between fused pairs and half-steps in place against shapes
+// that were measured both ways: the faster way where they differ by more than
+// the fit's error.
+#include <cstdio>
+
+#include "pair_cost.hpp"
+
+using namespace lbm;
+
+// us a half-step in place and by pairs, `n` domains of x * y * z
+struct Measured {
+    int n, x, y, z;
+    double in_place, pairs;
+};
+
+static const Measured F32[] = {
+    {1, 400, 401, 3, 14.0, 12.7},    {1, 300, 300, 6, 16.1, 14.0},    {1, 12, 200, 210, 14.7, 13.4},
+    {1, 500, 4, 250, 13.9, 11.4},    {1, 83, 79, 77, 14.8, 14.2},     {1, 90, 90, 90, 20.5, 16.1},
+    {1, 96, 96, 96, 23.4, 17.1},     {1, 128, 128, 128, 48.8, 39.4},  {1, 160, 160, 160, 98.8, 73.8},
+    {1, 256, 256, 256, 462, 327},    {1, 2000, 1500, 3, 248, 203},    {1, 3, 1000, 1000, 68.3, 55.7},
+    {1, 30, 30, 1200, 27.3, 20.3},   {1, 1000, 1000, 3, 66.6, 74.0},  {1, 16, 16, 8000, 48.2, 53.8},
+    {1, 8, 8, 20000, 32.1, 94.5},    {1, 4, 4, 60000, 24.8, 274},     {1, 257, 130, 15, 13.9, 14.6},
+    {118, 16, 16, 16, 14.1, 18.4},   {500, 16, 16, 16, 47.0, 62.6},   {300, 12, 12, 12, 14.9, 32.8},
+    {3000, 8, 8, 8, 37.8, 133},      {40, 3, 50, 100, 17.9, 29.1},    {40, 100, 50, 3, 17.1, 18.7},
+    {400, 8, 8, 64, 38.9, 148},      {200, 20, 20, 20, 38.5, 43.1},   {3000, 12, 12, 12, 148, 229},
+    {5, 48, 48, 48, 17.0, 13.7},     {16, 48, 48, 48, 41.8, 35.6},    {600, 24, 24, 24, 231, 149},
+    {400, 100, 50, 3, 169, 127},     {40, 64, 64, 64, 285, 205},        {1, 512, 512, 6, 37.7, 32.2},
+};
+static const Measured F64[] = {
+    {1, 64, 64, 64, 14.2, 13.0},     {1, 68, 68, 68, 17.1, 14.6},     {1, 80, 80, 80, 25.1, 20.2},
+    {1, 96, 96, 96, 40.9, 32.2},     {1, 160, 160, 160, 231, 145},    {1, 16, 16, 4000, 46.6, 39.6},
+    {1, 3, 700, 700, 64.9, 50.7},    {1, 700, 700, 5, 119, 105},      {1, 300, 300, 3, 15.1, 18.5},
+    {1, 520, 33, 17, 15.9, 17.5},    {1, 500, 500, 4, 46.0, 50.5},    {1, 8, 8, 10000, 30.9, 55.6},
+    {1, 130, 130, 20, 18.6, 19.1},   {600, 8, 8, 8, 16.9, 37.3},      {400, 12, 12, 12, 33.5, 50.6},
+    {80, 16, 16, 16, 18.4, 21.8},    {20, 100, 50, 3, 16.5, 18.6},    {4000, 8, 8, 8, 98.5, 214},
+    {2000, 16, 16, 16, 447, 284},    {20, 64, 64, 64, 288, 186},      {40, 20, 20, 20, 18.6, 15.3},
+    {200, 100, 50, 3, 170, 142},     {8, 48, 48, 48, 40.7, 36.5},
+};
+// with non-temporal accesses in place
+static const Measured NT32[] = {
+    {1, 256, 256, 256, 421, 327}, {500, 16, 16, 16, 49.8, 62.7}, {2000, 16, 16, 16, 195, 212}, {1, 96, 96, 96, 23.5, 17.1},
+};
+static const Measured NT64[] = {
+    {1, 128, 128, 128, 94.5, 99.6}, {1, 1000, 1000, 3, 141, 145}, {1, 160, 160, 160, 194, 145}, {1, 80, 80, 80, 26.6, 20.1},
+};
+
+static int fails = 0;
+
+template <size_t N>
+static void check(const Measured (&table)[N], bool f64, bool nt) {
+    for (const Measured &m : table) {
+        const std::vector<std::array<int, 3>> dims((size_t)m.n, {m.x, m.y, m.z});
+        const WalkPlan W = plan_walks(dims, f64);
+        const long long cells = (long long)m.n * m.x * m.y * m.z;
+        const double in_place = in_place_us(cells, f64, nt), walks = walks_us(W.sets, f64) / 2;
+        const bool want = m.pairs < m.in_place, got = walks_pay(W.sets, f64, nt);
+        // both fits within a fifth, and the faster way taken
+        const bool fit = in_place > 0.8 * m.in_place && in_place < 1.2 * m.in_place && walks > 0.78 * m.pairs && walks < 1.25 * m.pairs;
+        if (want == got && fit) continue;
+        ++fails;
+        printf("FAIL: %d of %dx%dx%d f%d nt %d: in place %.1f (measured %.1f), pairs %.1f (%.1f), pairs taken %d\n", m.n,
+               m.x, m.y, m.z, f64 ? 64 : 32, (int)nt, in_place, m.in_place, walks, m.pairs, (int)got);
+    }
+}
+
+int main() {
+    check(F32, false, false);
+    check(F64, true, false);
+    check(NT32, false, true);
+    check(NT64, true, true);
+    if (!walks_pay(plan_walks({{{96, 96, 96}}}, false).sets, false, false) ||
+        walks_pay(plan_walks({{{72, 72, 72}}}, false).sets, false, false)) {
+        ++fails;
+        printf("FAIL: the least cells\n");
+    }
+    // unequal members: the long ones decide how the last slots empty
+    std::vector<std::array<int, 3>> mixed(40, {64, 64, 64});
+    mixed.resize(60, {24, 24, 24});
+    if (!walks_pay(plan_walks(mixed, false).sets, false, false)) {
+        ++fails;
+        printf("FAIL: unequal members\n");
+    }
+    if (fails) {
+        printf("%d failures\n", fails);
+        return 1;
+    }
+    printf("pair cost: ok\n");
+    return 0;
+}

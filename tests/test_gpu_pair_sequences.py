@@ -152,9 +152,13 @@ def test_a_recorded_sequence_steps_in_place(paired_before):
         s.close()
 
 
-# Domains whose sequences take pairs: walks, then boxes.
-@pytest.mark.parametrize("dims,storage", [((83, 79, 77), F32), ((150, 141, 133), F32), ((61, 67, 63), F64),
-                                          ((24, 20, 16), F32), ((16, 16, 16), F64)])
+# Domains whose sequences take pairs: walks by runs of positions and by
+# rectangles, one column wide to rows longer than a work-group, thin and ragged;
+# then boxes.
+@pytest.mark.parametrize("dims,storage", [
+    ((83, 79, 77), F32), ((150, 141, 133), F32), ((12, 200, 210), F32), ((400, 401, 3), F32), ((500, 4, 250), F32),
+    ((1100, 60, 30), F32), ((330, 100, 60), F32), ((61, 67, 63), F64), ((3, 700, 700), F64), ((520, 60, 40), F64),
+    ((300, 61, 30), F64), ((24, 20, 16), F32), ((16, 16, 16), F64)])
 def test_sequences_take_pairs(dims, storage):
     a, b = build(dims, storage), build(dims, storage)
     assert b.pair_count() == {"pairs": 0, "second_buffer": False}
@@ -177,7 +181,7 @@ def test_groups_take_pairs(graph):
     """With and without exchange, in graphs and launched one by one."""
     free = LbmGroup([build((96, 70, 64), F32, k) for k in range(3)])
     joined = x_chain((104, 104, 104), 2, F32)
-    two = LbmGroup([build((60, 70, 64), F64, k) for k in range(3)])
+    two = LbmGroup([build((64, 70, 64), F64, k) for k in range(5)])
     for g in (free, joined, two):
         g.set_graph(graph)
         g.step(2)
@@ -212,3 +216,21 @@ def test_a_failed_allocation_takes_the_second_buffers():
     same(a, b)
     a.close()
     b.close()
+
+
+# Walks of few columns, or of few planes beside the two of their halo, lose
+# against the half-steps: by 3.5 and 11 times the first two.
+@pytest.mark.parametrize("count,dims,storage", [(1500, (8, 8, 8), F32), (1, (4, 4, 60000), F32), (1, (1000, 1000, 3), F32),
+                                                (200, (16, 16, 16), F32), (1, (300, 300, 3), F64), (400, (12, 12, 12), F64)])
+def test_shapes_that_step_in_place(count, dims, storage):
+    solvers = [build(dims, storage, k) for k in range(count)]
+    if count == 1:
+        solvers[0].run(8)
+        assert solvers[0].pair_count() == {"pairs": 0, "second_buffer": False}
+    else:
+        g = LbmGroup(solvers)
+        g.step(8)
+        assert g.pair_count() == 0 and not any(s.pair_count()["second_buffer"] for s in solvers)
+        g.close()
+    for s in solvers:
+        s.close()

@@ -25,6 +25,7 @@
 #include "launch_shape.hpp"
 #include "lbm_device.hpp"
 #include "lbm_pair.hpp"
+#include "pair_cost.hpp"
 #include "second_buffers.hpp"
 
 using namespace lbm;
@@ -436,7 +437,8 @@ struct lbm_group {
     long long *d_ctr = nullptr;  // device half-step counter (two slots, see step_kernel)
     PairTile *d_pair = nullptr;  // tiles of the fused pairs
     size_t pair_cap = 0;
-    int npair = 0;               // 0: not planned for the present members
+    int npair = 0;               // 0: not planned for the present members and variant, -1: they step in place
+    std::vector<PairTile> pair_tiles;  // planned, not on the device yet
     PairLaunch pair_launch{};
     // Fused pairs of members that exchange faces: their plan, on the device the
     // boxes of the layers and, per block, its box, and the copies after beta
@@ -628,24 +630,10 @@ struct PairPlan {
     PairLaunch launch;
 };
 
-// Work-groups of the pair kernel that run at once: the LDS of one takes a compute unit.
-constexpr long long kPairSlots = 256;
-
 long long cells_of(const std::vector<lbm_solver *> &doms) {
     long long n = 0;
     for (const lbm_solver *m : doms) n += m->cells;
     return n;
-}
-
-// Whether pair_kernel's walks are the better way through a step sequence of
-// these domains.  In place against walks, us a step of a cube: FP32 LES 64^3
-// 8.7 / 10.3, 72^3 10.4 / 10.8, 80^3 14.3 / 13.2, 96^3 23.2 / 17.0, 160^3
-// 100.5 / 78.2, 256^3 464 / 336; FP64 LES 48^3 7.7 / 10.0, 64^3 14.1 / 12.9,
-// 96^3 40.7 / 31.6, 160^3 231 / 147, 256^3 922 / 563.  Small domains have too
-// few columns to hide a walk's latency.  The two-byte storages move half the
-// bytes with as many instructions, and are bound by those already.
-bool walks_pay(const std::vector<lbm_solver *> &doms, int storage) {
-    return elem_size(storage) >= 4 && cells_of(doms) >= (storage == LBM_STORAGE_F64 ? 250000 : 480000);
 }
 
 // Whether fused pairs pay for domains that exchange faces (plan_faces), whose
@@ -689,10 +677,14 @@ bool boxes_pay(const lbm_solver *m, int storage, BoxShape *shape, PairLaunch *la
     return boxes < 0.96 * in_place;
 }
 
-// Tiles and launch of fused pairs over the domains; none: they step in place.
-PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage) {
+// Tiles and launch of fused pairs over the domains; none: they step in place
+// (with kernel variant `variant`).  The two-byte storages move half the bytes
+// with as many instructions, and are bound by those already.
+PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage, int variant) {
     PairPlan P;
-    if (!walks_pay(doms, storage)) {
+    const bool f64 = storage == LBM_STORAGE_F64, nt = (variant & 3) == (kVarNtLoad | kVarNtStore);
+    if (elem_size(storage) == 2) return P;
+    if (cells_of(doms) < walk_cells(f64)) {
         BoxShape shape;
         if (doms.size() == 1 && boxes_pay(doms[0], storage, &shape, &P.launch)) {
             const int *d = doms[0]->cfg.dims;
@@ -700,26 +692,17 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage) {
         }
         return P;
     }
-    // The most work-items whose two LDS planes fit a compute unit (160 KB): the
-    // larger the tile, the smaller its halo's share.  FP32 256^3 in tiles of
-    // 1024 against 512: 336 and 343-375 us a step.
-    P.launch.threads = storage == LBM_STORAGE_F64 ? 512 : 1024;
-    std::vector<PairShape> shape;
-    std::vector<std::pair<long long, int>> planes;  // tiles per plane, planes
+    std::vector<std::array<int, 3>> dims;
     size_t bytes = 0;
     for (const lbm_solver *m : doms) {
-        const int *d = m->cfg.dims;
-        shape.push_back(pair_shape(d[0], d[1], P.launch.threads));
-        planes.push_back({shape.back().tiles(), d[2]});
+        dims.push_back({m->cfg.dims[0], m->cfg.dims[1], m->cfg.dims[2]});
         bytes += (size_t)19 * m->padded * elem_size(storage);
     }
-    const int depth = doms.size() == 1 ? pair_depth(planes[0].second, planes[0].first, kPairSlots)
-                                       : pair_depth_of_many(planes, kPairSlots);
-    for (size_t i = 0; i < doms.size(); ++i) {
-        const int *d = doms[i]->cfg.dims;
-        const int chunks = (d[2] + depth - 1) / depth;
-        pair_tiles((int)i, d[0], d[1], d[2], shape[i], (d[2] + chunks - 1) / chunks, P.tiles);
-    }
+    const WalkPlan W = plan_walks(dims, f64);
+    if (!walks_pay(W.sets, f64, nt)) return P;
+    P.launch.threads = W.threads;
+    for (size_t i = 0; i < doms.size(); ++i)
+        pair_tiles((int)i, dims[i][0], dims[i][1], dims[i][2], W.shape[i], W.sets[i].nz, P.tiles);
     // Tiles dealt to the XCDs in chunks of 8 once the state is well past the
     // 256 MB memory-side cache, in contiguous eighths below (us a step, chunks
     // / eighths): FP32 256^3 335 / 356, 192^3 132 / 130; FP64 256^3 563 / 608,
@@ -758,7 +741,7 @@ bool take_seconds(const std::vector<lbm_solver *> &solvers) {
 bool solver_pairs_ready(lbm_solver *s) {
     if (s->external || s->npair < 0 || recording(s->stream)) return false;  // no memory beyond the caller's
     if (!s->d_pair) {
-        PairPlan P = plan_pairs({s}, s->cfg.storage);
+        PairPlan P = plan_pairs({s}, s->cfg.storage, s->cfg.kernel_variant);
         s->npair = P.tiles.empty() ? -1 : (int)P.tiles.size();
         if (s->npair < 0) return false;
         const OnDevice on(s->cfg.device);
@@ -2520,11 +2503,18 @@ static int upload_faces(lbm_group *g) {
 // the wrong buffer).  Brings the pair tiles and descriptors up to date.
 static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
     *ready = false;
-    if (steps < 4 || g->timing || !walks_pay(g->members, g->storage) || recording(g->stream)) return LBM_OK;
+    if (steps < 4 || g->timing || g->npair < 0 || recording(g->stream)) return LBM_OK;
     for (const lbm_solver *m : g->members)
         if (m->external) return LBM_OK;
     for (const lbm_solver *m : g->members)
         if (m->stop_at > g->step_counter && m->stop_at < g->step_counter + steps) return LBM_OK;
+    if (!g->npair) {
+        PairPlan P = plan_pairs(g->members, g->storage, g->variant);
+        g->npair = P.tiles.empty() || P.launch.box_cells ? -1 : (int)P.tiles.size();
+        if (g->npair < 0) return LBM_OK;
+        g->pair_tiles.swap(P.tiles);
+        g->pair_launch = P.launch;
+    }
     if (!g->comms.empty()) {
         bool x_only = true;
         for (const GroupComm &c : g->comms) x_only = x_only && c.normal[0] != 0;
@@ -2539,14 +2529,12 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
         int rc = upload_faces(g);
         if (rc) return rc;
     }
-    if (!g->npair) {
-        const PairPlan P = plan_pairs(g->members, g->storage);
-        GCHK(grow_table(g->d_pair, g->pair_cap, P.tiles.size()));
-        GCHK(hipMemcpyAsync(g->d_pair, P.tiles.data(), sizeof(PairTile) * P.tiles.size(), hipMemcpyHostToDevice,
-                            g->stream));
+    if (!g->pair_tiles.empty()) {
+        GCHK(grow_table(g->d_pair, g->pair_cap, g->pair_tiles.size()));
+        GCHK(hipMemcpyAsync(g->d_pair, g->pair_tiles.data(), sizeof(PairTile) * g->pair_tiles.size(),
+                            hipMemcpyHostToDevice, g->stream));
         GCHK(hipStreamSynchronize(g->stream));
-        g->npair = (int)P.tiles.size();
-        g->pair_launch = P.launch;
+        std::vector<PairTile>().swap(g->pair_tiles);
     }
     g->pair_launch.layers = !g->comms.empty();
     if (!pair_kernel_ready(g->storage, g->pair_launch, g->device)) return LBM_OK;
@@ -2765,6 +2753,7 @@ extern "C" int lbm_group_set_launch(lbm_group *g, int work_group_size, int kerne
         return gfail(g, LBM_ERR_INVALID_ARGUMENT, "unsupported launch shape");
     GCHK(hipStreamSynchronize(g->stream));
     g->wg = work_group_size;
+    if (g->variant != kernel_variant) g->npair = 0;  // the half-steps' side of the choice
     g->variant = kernel_variant;
     group_drop_graph(g);
     if (g->fuse_x) g->plan_built = false;  // which chains a work-group holds depends on its size
