@@ -44,6 +44,36 @@ static const Measured NT64[] = {
     {1, 128, 128, 128, 94.5, 99.6}, {1, 1000, 1000, 3, 141, 145}, {1, 160, 160, 160, 194, 145}, {1, 80, 80, 80, 26.6, 20.1},
 };
 
+// Members nx * ny * nz of x * y * z that exchange all their faces.
+struct Joined {
+    int n[3];
+    int d[3];
+    bool f64, nt, pairs;
+};
+static const Joined FACES[] = {
+    {{2, 2, 2}, {128, 128, 128}, false, false, true},  // 480-570 / 374
+    {{2, 2, 2}, {128, 128, 128}, false, true, true},   // 421-496 / 374
+    {{5, 5, 5}, {40, 40, 40}, false, false, true},     // 357 / 275
+    {{2, 2, 2}, {300, 300, 10}, false, false, true},   // 222-249 / 195
+    {{2, 2, 2}, {88, 88, 88}, false, false, true},     // 184 / 143
+    {{2, 1, 1}, {160, 160, 160}, false, false, true},  // 277 / 175
+    {{10, 10, 1}, {16, 16, 200}, false, false, false}, // 221 / 280
+    {{1, 1, 8}, {512, 512, 4}, false, false, false},   // 257 / 264
+    {{4, 1, 4}, {70, 70, 70}, false, true, false},     // 160 / 173
+    {{5, 5, 5}, {32, 32, 32}, false, false, false},    // 148 / 162
+    {{8, 8, 8}, {20, 20, 20}, false, false, false},    // 200 / 230
+    {{2, 2, 2}, {12, 200, 200}, false, false, false},  // 118-122 / 127
+    {{2, 1, 1}, {60, 140, 140}, false, false, false},  // 57 / 62
+    {{2, 1, 1}, {60, 140, 140}, false, true, true},    // 67-73 / 61
+    {{3, 1, 1}, {40, 100, 100}, false, true, true},    // 42-52 / 40
+    {{2, 2, 2}, {80, 80, 80}, true, false, true},      // 257-279 / 183
+    {{2, 2, 2}, {96, 96, 96}, true, true, true},       // 364-398 / 327
+    {{4, 4, 4}, {40, 40, 40}, true, false, true},      // 284-315 / 236
+    {{2, 2, 2}, {300, 300, 4}, true, false, false},    // 339 / 370
+    {{2, 2, 2}, {150, 150, 10}, true, false, false},   // 101-121 / 131
+    {{4, 4, 4}, {32, 32, 32}, true, false, false},     // 114 / 135
+};
+
 static int fails = 0;
 
 template <size_t N>
@@ -63,7 +93,23 @@ static void check(const Measured (&table)[N], bool f64, bool nt) {
     }
 }
 
+static void check_faces() {
+    for (const Joined &m : FACES) {
+        const std::vector<std::array<int, 3>> dims((size_t)(m.n[0] * m.n[1] * m.n[2]), {m.d[0], m.d[1], m.d[2]});
+        FaceCells f;
+        f.x = 2ll * (m.n[0] - 1) * m.n[1] * m.n[2] * m.d[1] * m.d[2];
+        f.yz = 2ll * (m.n[1] - 1) * m.n[0] * m.n[2] * m.d[0] * m.d[2] +
+               2ll * (m.n[2] - 1) * m.n[0] * m.n[1] * m.d[0] * m.d[1];
+        const WalkPlan W = plan_walks(dims, m.f64);
+        if ((walks_pay(W.sets, m.f64, m.nt) && face_pairs_pay(W.sets, f, m.f64, m.nt)) == m.pairs) continue;
+        ++fails;
+        printf("FAIL: %dx%dx%d of %dx%dx%d f%d nt %d: pairs are to be taken: %d\n", m.n[0], m.n[1], m.n[2], m.d[0],
+               m.d[1], m.d[2], m.f64 ? 64 : 32, (int)m.nt, (int)m.pairs);
+    }
+}
+
 int main() {
+    check_faces();
     check(F32, false, false);
     check(F64, true, false);
     check(NT32, false, true);

@@ -10,6 +10,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+from tests.test_gpu_parity import build_gpu_group  # noqa: E402
 from turbulent_lbm_multigpu_amd import _capi, serving  # noqa: E402
 from turbulent_lbm_multigpu_amd.solver import LbmGroup, LbmSolver  # noqa: E402
 
@@ -77,7 +78,7 @@ def x_chain(dims, n, storage):
 def test_a_stopping_member_joins_a_paired_group():
     """The plan of the two joined members, who run as pairs, does not outlive
     the third's arrival, whose stop refuses pairs; nor does the refusal."""
-    dims = (104, 104, 104)
+    dims = (130, 140, 140)
     a, b = x_chain(dims, 2, F32), x_chain(dims, 2, F32)
     late = [build((90, 80, 70), F32, 7) for _ in range(2)]
 
@@ -91,6 +92,7 @@ def test_a_stopping_member_joins_a_paired_group():
             same(x, y)
 
     both(8)
+    assert b.pair_count() == 4
     for g, s in ((a, late[0]), (b, late[1])):
         g.add_member(s)
         g.set_member_stop(2, 30)
@@ -101,7 +103,9 @@ def test_a_stopping_member_joins_a_paired_group():
     both(8)
     for g in (a, b):
         g.set_member_stop(2, -1)
+    assert b.pair_count() == 4
     both(8)
+    assert b.pair_count() == 8
     for g in (a, b):
         g.remove_member(2)
     both(8)
@@ -180,7 +184,7 @@ def test_sequences_take_pairs(dims, storage):
 def test_groups_take_pairs(graph):
     """With and without exchange, in graphs and launched one by one."""
     free = LbmGroup([build((96, 70, 64), F32, k) for k in range(3)])
-    joined = x_chain((104, 104, 104), 2, F32)
+    joined = x_chain((130, 140, 140), 2, F32)
     two = LbmGroup([build((64, 70, 64), F64, k) for k in range(5)])
     for g in (free, joined, two):
         g.set_graph(graph)
@@ -233,4 +237,63 @@ def test_shapes_that_step_in_place(count, dims, storage):
         assert g.pair_count() == 0 and not any(s.pair_count()["second_buffer"] for s in solvers)
         g.close()
     for s in solvers:
+        s.close()
+
+
+# domain, subdomains, periodic axes, storage, exchange mode, x faces in the kernel, kernel variant
+FACES = [
+    ((170, 164, 166), (2, 2, 2), (0, 0, 0), F32, 1, 1, 0),  # edges and corners of three axes
+    ((170, 164, 166), (2, 2, 2), (0, 0, 0), F32, 0, 0, 0),  # every slot of the ghost layers is copied
+    ((180, 168, 166), (3, 1, 2), (1, 1, 1), F32, 1, 2, 0),  # every face has a neighbour, some the domain itself
+    ((260, 150, 130), (1, 1, 1), (1, 0, 1), F32, 1, 0, 0),  # a domain next to itself along two axes
+    ((16, 400, 420), (4, 1, 1), (0, 0, 0), F32, 1, 0, 3),   # four cells wide: ghost and inner layers only
+    ((300, 64, 68), (3, 1, 1), (1, 0, 0), F32, 0, 1, 35),
+    ((400, 112, 104), (1, 2, 1), (0, 0, 0), F32, 1, 1, 0),  # several tile columns
+    ((122, 140, 150), (2, 2, 1), (0, 1, 0), F64, 1, 2, 0),
+    ((60, 230, 240), (1, 2, 2), (1, 0, 0), F64, 0, 0, 0),
+]
+
+
+@pytest.mark.parametrize("case,graph", [(c, True) for c in FACES] + [(FACES[0], False), (FACES[-1], False)])
+def test_groups_with_faces_take_pairs(case, graph):
+    size, nums, periodic, storage, mode, fused, variant = case
+    print(f"case: {case} graph {graph}", flush=True)
+    groups = []
+    for _ in range(2):
+        g, _, _ = build_gpu_group(size, nums, lid=0.08, amp=1e-2, seed=11, storage=storage, mode=mode, graph=graph,
+                                  periodic=tuple(bool(p) for p in periodic), inv_tau=1 / 0.51, tau=0.51,
+                                  smagorinsky_cs=0.17, kernel_variant=variant)
+        for i, s in enumerate(g.solvers):
+            s.place_spheres(5 + i, 0.04, 1.0, 2.5)
+        g.set_fused_x(fused)
+        groups.append(g)
+    a, b = groups
+    for n in (4, 1, 7):
+        for _ in range(n):
+            a.step(1)
+        b.step(n)
+    a.wait()
+    b.wait()
+    assert a.pair_count() == 0 and b.pair_count() == 4
+    for x, y in zip(a.solvers, b.solvers):
+        same(x, y)
+        for field in (_capi.FIELD_VELOCITY, _capi.FIELD_DENSITY):
+            np.testing.assert_array_equal(x.store(field), y.store(field))
+    for g in groups:
+        g.close()
+        for s in g.solvers:
+            s.close()
+
+
+@pytest.mark.parametrize("nums,dims,storage", [((5, 5, 5), (32, 32, 32), F32), ((10, 10, 1), (16, 16, 200), F32),
+                                               ((2, 2, 2), (300, 300, 4), F64)])
+def test_joined_shapes_that_step_in_place(nums, dims, storage):
+    """Above 240 MB, and slower in pairs."""
+    mono = tuple(n * d for n, d in zip(nums, dims))
+    g, _, _ = build_gpu_group(mono, nums, lid=0.08, amp=1e-2, seed=11, storage=storage, mode=1, inv_tau=1 / 0.51,
+                              tau=0.51, smagorinsky_cs=0.17)
+    g.step(8)
+    assert g.pair_count() == 0 and not any(s.pair_count()["second_buffer"] for s in g.solvers)
+    g.close()
+    for s in g.solvers:
         s.close()

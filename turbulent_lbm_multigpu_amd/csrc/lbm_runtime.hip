@@ -437,7 +437,7 @@ struct lbm_group {
     long long *d_ctr = nullptr;  // device half-step counter (two slots, see step_kernel)
     PairTile *d_pair = nullptr;  // tiles of the fused pairs
     size_t pair_cap = 0;
-    int npair = 0;               // 0: not planned for the present members and variant, -1: they step in place
+    int npair = 0;               // 0: not planned for the present members, comms and variant, -1: they step in place
     std::vector<PairTile> pair_tiles;  // planned, not on the device yet
     PairLaunch pair_launch{};
     // Fused pairs of members that exchange faces: their plan, on the device the
@@ -636,21 +636,6 @@ long long cells_of(const std::vector<lbm_solver *> &doms) {
     return n;
 }
 
-// Whether fused pairs pay for domains that exchange faces (plan_faces), whose
-// pair takes five launches, or two with x faces only, and some of the work
-// again.  In place and its copies against pairs, us a half-step of a group.
-// In place, a state that stays in the last-level cache (256 MB) is moved
-// faster than one that does not: FP32 8 x 64^3 57 / 65, 8 x 72^3 128 / 91, 8 x
-// 96^3 194 / 164, 8 x 128^3 423 / 364, 4 of 120x90x90 in y and z 103 / 103;
-// FP64 8 x 52^3 62 / 74, 8 x 64^3 151 / 122, 8 x 80^3 315 / 203.  Joined in x
-// only, FP32: 2 of 100x100x50 34 / 36, 3 of 40x100x100 47 / 43, 2 of 100^3 57 /
-// 56; with x faces in the step kernel 39 / 36, 51 / 40, 68 / 54.  FP64 2 x 80^3
-// 57 / 68.
-bool face_pairs_pay(const std::vector<lbm_solver *> &doms, int storage, bool x_only) {
-    const long long bytes = 19ll * (long long)elem_size(storage) * cells_of(doms);
-    return bytes >= (x_only && storage == LBM_STORAGE_F32 ? 84000000ll : 240000000ll);
-}
-
 // The boxes of a domain too small for walks, and whether they beat the
 // half-step launches: both sides as fitted to measurements of cubes from 16^3
 // to 72^3 and of flat and long domains, us a pair of a run on its own.  In
@@ -677,10 +662,10 @@ bool boxes_pay(const lbm_solver *m, int storage, BoxShape *shape, PairLaunch *la
     return boxes < 0.96 * in_place;
 }
 
-// Tiles and launch of fused pairs over the domains; none: they step in place
-// (with kernel variant `variant`).  The two-byte storages move half the bytes
+// Tiles and launch of fused pairs over the domains, which exchange `faces`;
+// none: they step in place (with kernel variant `variant`).  The two-byte storages move half the bytes
 // with as many instructions, and are bound by those already.
-PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage, int variant) {
+PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage, int variant, const FaceCells *faces = nullptr) {
     PairPlan P;
     const bool f64 = storage == LBM_STORAGE_F64, nt = (variant & 3) == (kVarNtLoad | kVarNtStore);
     if (elem_size(storage) == 2) return P;
@@ -699,7 +684,7 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage, int vari
         bytes += (size_t)19 * m->padded * elem_size(storage);
     }
     const WalkPlan W = plan_walks(dims, f64);
-    if (!walks_pay(W.sets, f64, nt)) return P;
+    if (!walks_pay(W.sets, f64, nt) || (faces && !face_pairs_pay(W.sets, *faces, f64, nt))) return P;
     P.launch.threads = W.threads;
     for (size_t i = 0; i < doms.size(); ++i)
         pair_tiles((int)i, dims[i][0], dims[i][1], dims[i][2], W.shape[i], W.sets[i].nz, P.tiles);
@@ -2128,6 +2113,7 @@ extern "C" int lbm_group_add_comm(lbm_group *g, int member, int dst_member, cons
     }
     g->comms.push_back(c);
     g->plan_built = false;
+    g->npair = 0;
     return LBM_OK;
 }
 
@@ -2509,16 +2495,16 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
     for (const lbm_solver *m : g->members)
         if (m->stop_at > g->step_counter && m->stop_at < g->step_counter + steps) return LBM_OK;
     if (!g->npair) {
-        PairPlan P = plan_pairs(g->members, g->storage, g->variant);
+        FaceCells faces;
+        for (const GroupComm &c : g->comms)
+            (c.normal[0] ? faces.x : faces.yz) += (long long)c.size[0] * c.size[1] * c.size[2];
+        PairPlan P = plan_pairs(g->members, g->storage, g->variant, g->comms.empty() ? nullptr : &faces);
         g->npair = P.tiles.empty() || P.launch.box_cells ? -1 : (int)P.tiles.size();
         if (g->npair < 0) return LBM_OK;
         g->pair_tiles.swap(P.tiles);
         g->pair_launch = P.launch;
     }
     if (!g->comms.empty()) {
-        bool x_only = true;
-        for (const GroupComm &c : g->comms) x_only = x_only && c.normal[0] != 0;
-        if (!face_pairs_pay(g->members, g->storage, x_only)) return LBM_OK;
         int rc = group_prepare(g);  // refuses comms without a counterpart
         if (rc) return rc;
         if (!g->faces_planned) group_plan_faces(g);

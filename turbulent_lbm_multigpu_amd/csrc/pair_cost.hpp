@@ -124,4 +124,37 @@ inline bool walks_pay(const std::vector<WalkSet> &sets, bool f64, bool nt) {
     return walks_us(sets, f64) * margin <= 2.0 * in_place_us(cells, f64, nt);
 }
 
+// The same for domains that exchange faces (plan_faces): cells of the x faces
+// and of the y and z faces, each from both sides.
+struct FaceCells {
+    long long x = 0, yz = 0;
+};
+
+// The pair takes five launches, or two with x faces only, and steps some cells
+// again; the half-steps take their copies, or x faces in the step kernel, whose
+// time varies more.  Below 335 MB, most of it in the last-level cache, either
+// way can win by a quarter: us a half-step, in place / pairs, FP32 8 of 80^3
+// with x faces in the kernel 140 / 117, copied 121 / 117, 125 of 32^3 148 /
+// 162, 512 of 20^3 200 / 230; FP64 8 of 64^3 114 / 111, 4 of 150x150x20 98 /
+// 121.  Above: FP32 8 of 128^3 480-570 / 374, 125 of 40^3 357 / 275, 100 of
+// 16x16x200 221 / 280, 8 of 512x512x4 257 / 264; FP64 8 of 96^3 416-473 / 327,
+// 8 of 300x300x4 339 / 370.  FP32 joined in x only with non-temporal accesses
+// gains down to 84 MB (2 of 100^3 56-69 / 54, 3 of 40x100x100 42-52 / 40, with
+// the default policy 52 / 54 and 38-44 / 40).  The non-temporal margin is the
+// fit's error there.
+inline bool face_pairs_pay(const std::vector<WalkSet> &sets, const FaceCells &faces, bool f64, bool nt) {
+    long long cells = 0;
+    for (const WalkSet &s : sets) cells += s.cells;
+    const double state = 19e-6 * (double)cells * (f64 ? 8 : 4);  // MB
+    if (!f64 && nt && faces.yz == 0) return state >= 84.0;
+    if (state < 335.0) return false;
+    const double x = 1e-5 * (double)faces.x, yz = 1e-5 * (double)faces.yz;
+    const double half = 2.0 * in_place_us(cells, f64, nt);
+    const double in_place = f64 ? (nt ? 1.080 * half + 31.3 * x + 6.1 * yz : 1.127 * half + 25.1 * x + 5.6 * yz)
+                                : (nt ? 1.155 * half + 20.4 * x + 2.4 * yz : 1.204 * half + 16.2 * x + 1.5 * yz);
+    const double pair = f64 ? 3.0 + 1.19 * walks_us(sets, f64) + 35.7 * x + 9.5 * yz
+                            : 15.7 + 1.23 * walks_us(sets, f64) + 25.8 * x + 4.7 * yz;
+    return pair * (nt ? 1.065 : 1.0) <= in_place;
+}
+
 }  // namespace lbm
