@@ -223,9 +223,11 @@ def test_a_failed_allocation_takes_the_second_buffers():
 
 
 # Walks of few columns, or of few planes beside the two of their halo, lose
-# against the half-steps: by 3.5 and 11 times the first two.
+# against the half-steps (by 3.5 and 11 times the first two), large boxes where
+# several solvers run side by side.
 @pytest.mark.parametrize("count,dims,storage", [(1500, (8, 8, 8), F32), (1, (4, 4, 60000), F32), (1, (1000, 1000, 3), F32),
-                                                (200, (16, 16, 16), F32), (1, (300, 300, 3), F64), (400, (12, 12, 12), F64)])
+                                                (200, (16, 16, 16), F32), (1, (300, 300, 3), F64), (400, (12, 12, 12), F64),
+                                                (1, (48, 48, 48), F32), (1, (40, 40, 40), F64)])
 def test_shapes_that_step_in_place(count, dims, storage):
     solvers = [build(dims, storage, k) for k in range(count)]
     if count == 1:

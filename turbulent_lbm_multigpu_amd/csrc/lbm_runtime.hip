@@ -639,15 +639,16 @@ long long cells_of(const std::vector<lbm_solver *> &doms) {
 // The boxes of a domain too small for walks, and whether they beat the
 // half-step launches: both sides as fitted to measurements of cubes from 16^3
 // to 72^3 and of flat and long domains, us a pair of a run on its own.  In
-// place / boxes: FP32 LES 16^3 8.8 / 6.0, 32^3 9.2 / 7.5, 48^3 11.8 / 10.4,
-// 64^3 17.2 / 16.1, 33x50x97 14.4 / 14.8; FP64 16^3 10.6 / 6.6, 32^3 11.6 /
-// 8.6, 48^3 15.6 / 15.0, 56^3 19.6 / 24.  Above the cell limits runs of several
-// solvers side by side fill the device, and the halo's share decides: three
-// 64^3 BGK runs at once, 6.06 us a step each in place, 6.44 in boxes.
+// place / boxes: FP32 LES 16^3 8.8 / 6.0, 32^3 9.2 / 7.5; FP64 16^3 10.6 / 6.6,
+// 32^3 11.6 / 8.6.  Above the cell limits runs of several solvers side by side
+// fill the device, and the halo's share decides; us a half-step of eight
+// solvers of one thread (in place between the two, as the host launches): FP32
+// 40^3 24-33 / 22, 44^3 26-34 / 30, 48^3 27-34 / 37; FP64 28^3 25-32 / 27, 36^3
+// 31-36 / 32, 40^3 32-36 / 39.
 bool boxes_pay(const lbm_solver *m, int storage, BoxShape *shape, PairLaunch *launch) {
     const int *d = m->cfg.dims;
     const bool f64 = storage == LBM_STORAGE_F64;
-    if (elem_size(storage) == 2 || m->cells > (f64 ? 70000 : 120000)) return false;
+    if (elem_size(storage) == 2 || m->cells > (f64 ? 47000 : 66000)) return false;
     const int large = box_large(f64), threads = box_threads(f64);
     const BoxShape a = box_shape(d[0], d[1], d[2], kBoxSmall, kBoxSmall, f64 ? 1 : 2, kPairSlots);
     const BoxShape b = box_shape(d[0], d[1], d[2], large, threads, 1, kPairSlots);
@@ -695,6 +696,23 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage, int vari
     P.launch.xcd_map = bytes > ((size_t)600 << 20) ? 8 : -1;
     return P;
 }
+
+// Threads that enqueue step sequences on a device at the moment.
+class Enqueuing {
+  public:
+    explicit Enqueuing(int device) : n_(counter(device)) { ++n_; }
+    ~Enqueuing() { --n_; }
+    Enqueuing(const Enqueuing &) = delete;
+    Enqueuing &operator=(const Enqueuing &) = delete;
+    bool alone() const { return n_.load(std::memory_order_relaxed) == 1; }
+
+  private:
+    static std::atomic<int> &counter(int device) {
+        static std::atomic<int> n[64];
+        return n[device & 63];
+    }
+    std::atomic<int> &n_;
+};
 
 // Whether a caller records the stream: what is recorded steps in place, for a
 // replay would not know that the second buffers it wrote to are gone.
@@ -1177,6 +1195,7 @@ extern "C" int lbm_solver_simulation_step(lbm_solver *s) {
 extern "C" int lbm_solver_run(lbm_solver *s, int steps) {
     if (!s) return record(nullptr, LBM_ERR_INVALID_ARGUMENT, "null solver");
     if (steps < 0) return fail(s, LBM_ERR_INVALID_ARGUMENT, "steps must be >= 0");
+    const Enqueuing enqueuing(s->cfg.device);
     int i = 0;
     if (steps >= 5 && (s->step_counter & 1)) {  // pairs start on a beta step
         int rc = lbm_solver_simulation_step(s);
@@ -1185,8 +1204,20 @@ extern "C" int lbm_solver_run(lbm_solver *s, int steps) {
     }
     if (steps - i >= 4 && (s->step_counter & 1) == 0 && solver_pairs_ready(s)) {
         const auto lock = second_buffers().in_use();
-        // two pairs at a time: into the second buffer and back
+        // Two pairs at a time: into the second buffer and back.  Boxes, of which
+        // each takes much of a compute unit's LDS, only while no other thread's
+        // launches could run beside them.  Four threads with a solver each, us a
+        // half-step, in place / boxes: FP32 24^3 7.9 / 6.8, 40^3 9.9 / 11.1; FP64
+        // 24^3 9.1 / 11.0, 32^3 10.9 / 15.0.
+        const bool boxes = s->pair_launch.box_cells > 0;
         for (void *two = s->second.at; two && steps - i >= 4; i += 4) {
+            if (boxes && !enqueuing.alone()) {
+                for (int k = 0; k < 4; ++k) {
+                    const int rc = lbm_solver_simulation_step(s);
+                    if (rc) return rc;
+                }
+                continue;
+            }
             for (int flip = 0; flip < 2; ++flip)
                 SCHK(launch_pair_kernel(s->cfg.storage, s->pair_launch, s->npair, s->d_desc, s->d_pair, two, s->stream,
                                         nullptr, flip));
@@ -2681,6 +2712,7 @@ extern "C" int lbm_group_step(lbm_group *g, int steps) {
     GCHK(hipSetDevice(g->device));
     int rc = group_prepare(g);
     if (rc) return rc;
+    const Enqueuing enqueuing(g->device);
     const long long before = g->step_counter;
     if (g->lt[0].ntiles == 0) {  // no members: counters only (re-published with the next upload)
         g->descs_dirty = true;
