@@ -117,13 +117,18 @@ hipError_t move_fields(int device, hipStream_t stream, long long n, int comps, s
     // A launch adds about 16 us to a chunk's time on the bus (19 us a MB), small
     // chunks start the copies on the host sooner: 173 MB take 8.8 / 6.3 / 5.4 /
     // 5.8 ms in chunks of 0.5 / 1 / 2 / 4 MB, 13 MB 1.13 / 1.09 / 1.12 / 1.25 ms.
+    // Into the device no fresh pages slow the host down, and the kernels' launches
+    // count more: 4.9 MB take 0.23 / 0.16 ms in chunks of 1 / 2 MB, 8.4 MB 0.35 /
+    // 0.29 (with a lane for each chunk; with one for two 0.31), 16 MB 0.58 / 0.47.
+    // The runtime's own copy to a staging buffer on the device took 0.18, 0.28, 0.49.
     const size_t bytes = (size_t)n * (size_t)comps * elem;
-    const size_t chunk = bytes >= (size_t)32 << 20 ? HostLane::kChunk : HostLane::kChunk / 2;
+    const bool large = bytes >= (size_t)(OUT ? 32 : 4) << 20;
+    const size_t chunk = large ? HostLane::kChunk : HostLane::kChunk / 2;
     const long long per = (long long)(chunk / ((size_t)comps * elem)) / 64 * 64;
     const long long chunks = (n + per - 1) / per;
     // A thread costs about 30 us to start, a fresh megabyte up to 300 us; with 4
     // threads the 173 MB take 5.9 ms, with more than 6 what they take with 6.
-    const int want = (int)std::max<long long>(1, std::min<long long>(6, chunks / 2));
+    const int want = (int)std::max<long long>(1, std::min<long long>(6, !OUT && large ? chunks : chunks / 2));
     int before = device;  // the caller's device, current again when this returns
     if (hipGetDevice(&before) != hipSuccess) before = device;
     if (before != device) {
