@@ -101,6 +101,11 @@ const char *lbm_version(void);
 /* message of the last failed call on this thread (creation failures included) */
 const char *lbm_last_error(void);
 int lbm_device_synchronize(int device);
+/* gives back the memory that is kept for objects to come (new): the second
+ * buffers of destroyed solvers (at most 8, 4 GiB in all; lbm_solver_run) and the
+ * pinned buffers of finished transfers (48 MB), which otherwise stay until this
+ * library needs them or the process ends */
+int lbm_release_kept_memory(void);
 void lbm_solver_config_default(lbm_solver_config *cfg);
 /* read+write bandwidth of a plain device copy of `bytes`, averaged over `reps`
  * launches (variant 0: grid-stride float4, 1: four float4 per work-item,
@@ -148,10 +153,16 @@ int lbm_solver_init_perturbed(lbm_solver *s, double amplitude, uint64_t seed, ui
 int lbm_solver_simulation_step(lbm_solver *s);
 int lbm_solver_simulation_step_alpha(lbm_solver *s);
 int lbm_solver_simulation_step_beta(lbm_solver *s);
-/* a sequence of at least 4 half-steps in FP32 or FP64 may go through a second
- * buffer of the distributions that the solver then keeps, as may
- * lbm_group_step's (same results; taken only while half the device's memory
- * stays free, given up when an allocation of this library fails) */
+/* `steps` half-steps.  A sequence of at least 4 in FP32 or FP64 may go through
+ * a second buffer of the distributions, two half-steps in one pass, as may
+ * lbm_group_step's: same results, in the same place.  Where the pass is the
+ * faster way the buffer is taken by the first such sequence, doubles the
+ * distributions' memory and stays with the solver.  It is taken only while half
+ * the device's memory stays free (else the sequence steps in place, and asks
+ * again after 63 more) and given up when an allocation of this library fails.
+ * Solvers in caller-provided memory step in place, as does a sequence that a
+ * caller records on the group's stream.  lbm_release_kept_memory gives back the
+ * buffers of destroyed solvers. */
 int lbm_solver_run(lbm_solver *s, int steps);
 /* pairs that lbm_solver_run has launched that way so far (two half-steps
  * each), and whether the solver holds a second buffer now (new) */

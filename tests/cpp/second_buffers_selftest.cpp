@@ -164,14 +164,43 @@ static void blocks_and_spares() {
     }
     sb.give_all(0);
     CHECK(mem.blocks == 0 && !sb.give_all(0));
+    {
+        Solver e(100);
+        CHECK(sb.take({&e.second}) && mem.blocks == 1);
+        sb.give(e.second);
+        CHECK(mem.blocks == 1);
+        sb.release_spares();
+        CHECK(mem.blocks == 0);
+    }
+}
+
+// A refusal holds for what was asked for, and for some sequences.
+static void refused_for_a_while() {
+    HostMemory mem;
+    SecondBuffers sb(mem);
+    Solver a(1000), b(5000), c(400);
     mem.full = true;
-    Solver e(100);
+    CHECK(!sb.take({&a.second, &b.second}) && mem.asked == 1 && !a.second.at && !b.second.at);
+    mem.full = false;  // as when another library has given its memory back
+    CHECK(sb.take({&a.second}) && mem.asked == 2);  // less than was refused
+    CHECK(sb.take({&b.second, &c.second}) && mem.asked == 3);
+    Solver d(7000);
+    mem.full = true;
+    CHECK(!sb.take({&d.second}) && mem.asked == 4);
+    mem.full = false;
+    for (int k = 0; k < SecondBuffers::kWait; ++k) CHECK(!sb.take({&d.second}));
+    CHECK(mem.asked == 4);
+    CHECK(sb.take({&d.second}) && mem.asked == 5 && d.second.at);
+    for (Solver *s : {&a, &b, &c, &d}) sb.give(s->second);
+    mem.full = true;
+    Solver e(100000);
     CHECK(!sb.take({&e.second}) && !e.second.at);
     sb.give(e.second);
 }
 
 int main() {
     blocks_and_spares();
+    refused_for_a_while();
     launches_keep_nobody_waiting();
     destroyed_while_taken_away();
     if (fails) {

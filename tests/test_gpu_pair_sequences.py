@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 from tests.test_gpu_parity import build_gpu_group  # noqa: E402
 from turbulent_lbm_multigpu_amd import _capi, serving  # noqa: E402
-from turbulent_lbm_multigpu_amd.solver import LbmGroup, LbmSolver  # noqa: E402
+from turbulent_lbm_multigpu_amd.solver import LbmGroup, LbmSolver, release_kept_memory  # noqa: E402
 
 F32, F64 = _capi.STORAGE_F32, _capi.STORAGE_F64
 
@@ -299,3 +299,30 @@ def test_joined_shapes_that_step_in_place(nums, dims, storage):
     g.close()
     for s in g.solvers:
         s.close()
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert _capi.load_library().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_kept_memory_is_given_back():
+    """A closed solver's second buffer (here 209 MB) is kept for the next one
+    until it is asked for."""
+    release_kept_memory()
+    before = free_bytes()
+    s = build((140, 140, 140), F32)
+    s.run(8)
+    assert s.pair_count()["second_buffer"]
+    s.close()
+    assert before - free_bytes() > 200e6
+    release_kept_memory()
+    assert before - free_bytes() < 50e6
+    a, b = build((96, 90, 88), F32), build((96, 90, 88), F32)  # and goes on all the same
+    b.run(8)
+    single_steps(a, 8)
+    same(a, b)
+    assert b.pair_count()["second_buffer"]
+    a.close()
+    b.close()

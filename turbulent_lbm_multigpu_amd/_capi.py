@@ -51,7 +51,7 @@ CASE_DONE = 2
 CASE_FAILED = 3
 
 EXPORTED_SYMBOLS = (
-    "lbm_version", "lbm_last_error", "lbm_device_synchronize", "lbm_solver_config_default",
+    "lbm_version", "lbm_last_error", "lbm_device_synchronize", "lbm_release_kept_memory", "lbm_solver_config_default",
     "lbm_device_copy_bandwidth",
     "lbm_solver_create", "lbm_solver_destroy", "lbm_solver_error", "lbm_solver_reset",
     "lbm_solver_init_perturbed", "lbm_solver_simulation_step", "lbm_solver_simulation_step_alpha",
@@ -194,6 +194,7 @@ def load_library(path: str | None = None):
     sig("lbm_version", C.c_char_p)
     sig("lbm_last_error", C.c_char_p)
     sig("lbm_device_synchronize", I, I)
+    sig("lbm_release_kept_memory", I)
     sig("lbm_solver_config_default", None, C.POINTER(SolverConfig))
     sig("lbm_device_copy_bandwidth", I, I, C.c_size_t, I, I, C.POINTER(D), C.POINTER(D))
     sig("lbm_solver_create", I, C.POINTER(SolverConfig), C.POINTER(P))

@@ -31,7 +31,7 @@ struct HostLane {
     int device = 0;
 };
 
-// The process's lanes, at most kLanes (48 MB pinned), kept until it ends.
+// The process's lanes, at most kLanes (48 MB pinned), kept until release().
 class HostLanes {
   public:
     static constexpr int kLanes = 12;
@@ -74,6 +74,14 @@ class HostLanes {
         std::lock_guard<std::mutex> lock(mutex_);
         idle_.insert(idle_.end(), lanes.begin(), lanes.end());
         given_.notify_all();
+    }
+    // Frees the lanes that no transfer holds.
+    void release() {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (HostLane *l : idle_) destroy(l);
+        made_ -= (int)idle_.size();
+        idle_.clear();
+        given_.notify_all();  // one may be made now
     }
 
   private:

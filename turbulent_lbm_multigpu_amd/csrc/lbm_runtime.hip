@@ -849,6 +849,12 @@ extern "C" int lbm_device_synchronize(int device) {
     return LBM_OK;
 }
 
+extern "C" int lbm_release_kept_memory(void) {
+    second_buffers().release_spares();
+    HostLanes::get().release();
+    return LBM_OK;
+}
+
 extern "C" void lbm_solver_config_default(lbm_solver_config *c) {
     if (!c) return;
     std::memset(c, 0, sizeof(*c));

@@ -30,7 +30,8 @@ struct SecondBuffer {
     std::atomic<unsigned> *version = nullptr;  // bumped when `at` changes
     size_t bytes = 0;                          // what the solver needs
     int device = 0;
-    bool refused = false;                      // there was no memory for it
+    size_t refused = 0;                        // > 0: there was no memory for so much,
+    int wait = 0;                              // and as many sequences go by before it is asked for again
     SecondBlock *block = nullptr;
 };
 
@@ -48,10 +49,13 @@ struct SecondMemory {
 // (the queue is bounded), and nothing else of one thread waits for another's.
 // The blocks of the last few destroyed solvers are kept for the next ones (an
 // allocation costs a short run more than it gains): at most kSpares,
-// kSpareBytes in all.
+// kSpareBytes in all, until release_spares().
 class SecondBuffers {
   public:
     static constexpr size_t kSpares = 8, kSpareBytes = (size_t)4 << 30;
+    // Sequences that step in place after a refusal: asking takes the runtime a
+    // good part of a short one, and the memory may be there later.
+    static constexpr int kWait = 63;
     explicit SecondBuffers(SecondMemory &memory) : memory_(memory) {}
 
     // Gives these (of one device) their second buffers, those without one in a
@@ -62,11 +66,17 @@ class SecondBuffers {
         size_t bytes = 0;
         for (SecondBuffer *s : all) {
             if (s->at) continue;
-            if (s->refused) return false;
             without.push_back(s);
             bytes += aligned(s->bytes);
         }
         if (without.empty()) return true;
+        bool wait = false;
+        for (SecondBuffer *s : without) {
+            if (s->wait == 0 || bytes < s->refused) continue;
+            --s->wait;
+            wait = true;
+        }
+        if (wait) return false;
         const std::lock_guard<std::mutex> lock(mutex_);
         const int device = without[0]->device;
         SecondBlock *b = nullptr;
@@ -80,7 +90,10 @@ class SecondBuffers {
         if (!b) {
             void *const p = memory_.allocate(device, bytes);
             if (!p) {
-                for (SecondBuffer *s : without) s->refused = true;
+                for (SecondBuffer *s : without) {
+                    s->refused = bytes;
+                    s->wait = kWait;
+                }
                 return false;
             }
             b = new SecondBlock{p, bytes, device, 0};
@@ -89,6 +102,7 @@ class SecondBuffers {
         for (SecondBuffer *s : without) {
             s->block = b;
             b->refs++;
+            s->wait = 0;
             s->at = (char *)b->base + off;
             off += aligned(s->bytes);
             held_.insert(s);
@@ -118,6 +132,12 @@ class SecondBuffers {
         for (SecondBuffer *s : here) drop(*s);
         free_spares(0, 0);
         return true;
+    }
+
+    // Frees the blocks that are kept for solvers to come.
+    void release_spares() {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        free_spares(0, 0);
     }
 
     std::shared_lock<std::shared_mutex> in_use() {

@@ -240,6 +240,12 @@ class LbmSolver:
         return rho, j
 
 
+def release_kept_memory():
+    """Gives back the memory kept for objects to come: second buffers of closed
+    solvers, pinned transfer buffers (lbm_release_kept_memory)."""
+    _capi.load_library().lbm_release_kept_memory()
+
+
 def copy_box(src: LbmSolver, src_origin, dst: LbmSolver, dst_origin, size, norm=None):
     """Device-to-device box copy of distributions (one CComm transfer)."""
     rc = src._lib.lbm_copy_box(src.handle, ivec(src_origin), dst.handle, ivec(dst_origin), ivec(size), ivec(norm))
