@@ -486,9 +486,9 @@ __device__ __forceinline__ int wrap_idx(int a, int cells) {
 // FP32), far below the storage's rounding.  Only these storages take this
 // form: the FP32 and FP64 kernels keep the reference's expression order, which
 // their bit parity with the CPU oracle rests on.
-template <bool BETA, class PP>
-__device__ __forceinline__ bool cell_update_pairs(float *f, int flag, const PP *D, float &vx, float &vy, float &vz,
-                                                  float &dens_out) {
+template <bool BETA>
+__device__ __forceinline__ bool cell_update_pairs(float *f, int flag, const DomDev *D, float &vx, float &vy,
+                                                  float &vz, float &dens_out) {
     float s[9], d[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) {

@@ -79,8 +79,6 @@ template <typename U>
 __device__ __forceinline__ U buf_ld(PairBuf b, unsigned off, unsigned pop) {
     if constexpr (sizeof(U) == 4) {
         return (U)__builtin_amdgcn_raw_buffer_load_b32(b, (int)off, (int)pop, 0);
-    } else if constexpr (sizeof(U) == 2) {
-        return (U)__builtin_amdgcn_raw_buffer_load_b16(b, (int)off, (int)pop, 0);
     } else {
         return __builtin_bit_cast(U, __builtin_amdgcn_raw_buffer_load_b64(b, (int)off, (int)pop, 0));
     }
@@ -89,8 +87,6 @@ template <typename U>
 __device__ __forceinline__ void buf_st(PairBuf b, unsigned off, unsigned pop, U v) {
     if constexpr (sizeof(U) == 4) {
         __builtin_amdgcn_raw_buffer_store_b32((unsigned)v, b, (int)off, (int)pop, 0);
-    } else if constexpr (sizeof(U) == 2) {
-        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)v, b, (int)off, (int)pop, 0);
     } else {
         typedef unsigned V2 __attribute__((ext_vector_type(2)));
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), b, (int)off, (int)pop, 0);
@@ -162,20 +158,20 @@ __device__ __forceinline__ void pair_gather_cell(PairBuf src, const PairRows &r,
 // way out against the rest: a beta cell that bounces back, an alpha cell that
 // keeps its slots (where the others store f[opp(k)] in slot k); the stores do
 // that by their addresses.
-template <typename T, bool BETA, bool SHIFT>
+template <typename T, bool BETA>
 __device__ __forceinline__ bool pair_update(T *f, int flag, const PairPhys<T> &ph, bool macros, T &vx, T &vy, T &vz,
                                             T &dens) {
-    if (flag == kFlagFluid) (void)cell_update<T, BETA, SHIFT>(f, kFlagFluid, &ph, vx, vy, vz, dens);
+    if (flag == kFlagFluid) (void)cell_update<T, BETA>(f, kFlagFluid, &ph, vx, vy, vz, dens);
     if (__ballot(flag != kFlagFluid) == 0ull) return false;
     int fl = flag;
     asm volatile("" : "+v"(fl));
-    if (fl == kFlagInjection) (void)cell_update<T, BETA, SHIFT>(f, kFlagInjection, &ph, vx, vy, vz, dens);
+    if (fl == kFlagInjection) (void)cell_update<T, BETA>(f, kFlagInjection, &ph, vx, vy, vz, dens);
     int fo = flag;
     asm volatile("" : "+v"(fo));
     if (BETA) return fo == kFlagObstacle;
     const bool keep = fo != kFlagFluid && fo != kFlagInjection;
     // a cell that stores nothing leaves f as it is
-    if (macros && keep) (void)cell_update<T, BETA, SHIFT>(f, fo, &ph, vx, vy, vz, dens);
+    if (macros && keep) (void)cell_update<T, BETA>(f, fo, &ph, vx, vy, vz, dens);
     return keep;
 }
 
@@ -280,7 +276,7 @@ __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
 #pragma unroll
         for (int i = 0; i < 19; ++i) f[i] = kin<SP>(u[i], i);
         const PairPhys<T> ph = pair_phys_here(phys);
-        const bool bounce = pair_update<T, true, SP::kShifted>(f, flag, ph, false, vx, vy, vz, dens);
+        const bool bounce = pair_update<T, true>(f, flag, ph, false, vx, vy, vz, dens);
         U *const even = buf + (bounce ? NT : 0), *const odd = buf + (bounce ? 0 : NT);
 #pragma unroll
         for (int i = 0; i < 18; i += 2) {
@@ -370,7 +366,7 @@ __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
                 ++q;
             }
         }
-        const bool keep = pair_update<T, false, SP::kShifted>(f, flag, ph, macros, vx, vy, vz, dens);
+        const bool keep = pair_update<T, false>(f, flag, ph, macros, vx, vy, vz, dens);
         // The next plane's loads are waited for before the stores: at the top
         // of the next plane the wait would cover the stores as well.
         loads_arrived();
@@ -448,7 +444,7 @@ __global__ void __launch_bounds__(256)
     T f[19], vx, vy, vz, dens;
 #pragma unroll
     for (int i = 0; i < 19; ++i) f[i] = kin<SP>(raw_ld<false, U>(own + i * pop, 0u), i);
-    if (cell_update<T, false, SP::kShifted>(f, flag, D, vx, vy, vz, dens)) {
+    if (cell_update<T, false>(f, flag, D, vx, vy, vz, dens)) {
 #pragma unroll
         for (int k = 0; k < 19; ++k) raw_st<false, U>(own + k * pop, 0u, kout<SP>(f[opp(k)], k));
     }
@@ -489,7 +485,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int i = 0; i < 19; ++i) f[i] = kin<SP>(u[i], i);
     const PairPhys<T> ph = pair_phys_here(pair_phys<T>(N));
-    const bool bounce = pair_update<T, true, SP::kShifted>(f, flag, ph, false, vx, vy, vz, dens);
+    const bool bounce = pair_update<T, true>(f, flag, ph, false, vx, vy, vz, dens);
     gchar *const to = (gchar *)N->seam + doms[F.dom].seam_at[F.side];
     int q = 0;
 #pragma unroll
@@ -560,7 +556,7 @@ __global__ void __launch_bounds__(NT)
 #pragma unroll
         for (int i = 0; i < 19; ++i) f[i] = kin<SP>(u[i], i);
         const PairPhys<T> ph = pair_phys_here(phys);
-        const bool bounce = pair_update<T, true, SP::kShifted>(f, flag, ph, false, vx, vy, vz, dens);
+        const bool bounce = pair_update<T, true>(f, flag, ph, false, vx, vy, vz, dens);
         U *const even = lds + e + (bounce ? CELLS : 0), *const odd = lds + e + (bounce ? 0 : CELLS);
 #pragma unroll
         for (int i = 0; i < 18; i += 2) {
@@ -580,7 +576,7 @@ __global__ void __launch_bounds__(NT)
         for (int i = 0; i < 19; ++i) f[i] = kin<SP>(lds[i * CELLS + pos - (ex(i) + w * ey(i) + wh * ez(i))], i);
         const int flag = lds_flags[pos];
         const PairPhys<T> ph = pair_phys_here(phys);
-        const bool keep = pair_update<T, false, SP::kShifted>(f, flag, ph, macros, vx, vy, vz, dens);
+        const bool keep = pair_update<T, false>(f, flag, ph, macros, vx, vy, vz, dens);
         const unsigned gs = (unsigned)(P.org + tx + 1 + X * (ty + 1) + XY * (P.z0 + tz));
         const unsigned own = cell_base(gs) * SP::kBytes;
         constexpr unsigned pop = kBlk * SP::kBytes;
