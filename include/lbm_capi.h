@@ -278,7 +278,7 @@ int lbm_group_sync(lbm_group *g, int after_beta);
 int lbm_group_wait(lbm_group *g);
 /* average device time per launch of the step kernels and the exchange kernels
  * since the last reset, measured with events on the group's stream when
- * timing is on */
+ * timing is on; a group that is timed steps in half-steps, without fused pairs */
 int lbm_group_set_timing(lbm_group *g, int enable);
 int lbm_group_get_timing(lbm_group *g, double *step_kernel_ms, long long *step_kernel_launches,
                          double *exchange_ms, long long *exchange_launches);
@@ -304,7 +304,9 @@ int lbm_group_get_alpha_work_group(const lbm_group *g, int *work_group_size);
  * lbm_group_get_alpha_work_group; a size set before is replaced); last, the
  * chosen shape with the two other XCD tile maps (eighths, chunks, none:
  * variant bits 32 and 4).  The timed steps are real steps of the simulation
- * (42 * (pairs + 1) of them, plus one if the counter was odd) */
+ * (42 * (pairs + 1) of them, plus one if the counter was odd).  They are
+ * half-steps in place: sequences that take fused pairs (lbm_solver_run) use the
+ * shape for the half-steps left over */
 int lbm_group_autotune(lbm_group *g, int pairs, int *best_wg, int *best_variant, double *best_ms_per_step);
 /* the same averages split into beta and alpha step kernels */
 int lbm_group_get_timing_detail(lbm_group *g, double *beta_ms, double *alpha_ms, double *exchange_ms);

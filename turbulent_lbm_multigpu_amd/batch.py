@@ -3,11 +3,11 @@
 The cavity set (seeded): every edge uniform in 16..96 cells per axis, lid
 speed uniform in [0.02, 0.1], tau = max(0.5002, lognormal(ln 0.52, 0.01)),
 Cs = 0.17, FP32, walls on every face and the lid layer at y = ny-2, starting
-from f = w_i.  ``run_batched`` puts all cases into one group (one step kernel
-launch per half-step over every case's tiles, the beta+alpha pair replayed as
-a hipGraph) with the launch shape chosen by the group autotuner;
-``run_sequential`` steps each case on its own, one launch per half-step, as a
-caller of the plain solver would.
+from f = w_i.  ``run_batched`` puts all cases into one group (one kernel launch
+over every case's tiles per half-step, or per fused pair of them, replayed as a
+hipGraph) with the half-steps' launch shape chosen by the group autotuner;
+``run_sequential`` steps each case on its own, as a caller of the plain solver
+would.
 
     python -m turbulent_lbm_multigpu_amd.batch --cases 512 --steps 1000
 """
@@ -72,8 +72,9 @@ def run_batched(cases: Sequence[Cavity], steps: int, *, autotune_pairs: int = 2,
     batch (16 launch shapes, then alpha at 3 work-group sizes of its own,
     then the XCD tile map switched, (pairs + 1) step pairs each): every launch shape computes the same
     arithmetic, so those are `steps` of every case like any other, and the
-    rest run as one graph launch (one fused step-kernel node per
-    half-step).  If tuning took more steps than `steps`, the cases restart
+    rest run as one graph launch (one node for all cases per half-step, or
+    per pair of half-steps where FP32 and FP64 batches take fused pairs, which
+    have a launch shape of their own).  If tuning took more steps than `steps`, the cases restart
     from their initial state and all `steps` run in the graph.  Tuning is
     counted in the wall time."""
     solvers = [build_solver(c, storage=storage) for c in cases]

@@ -267,8 +267,9 @@ def colocate(solvers: Sequence[LbmSolver]):
 
 
 class LbmGroup:
-    """Subdomains stepped by one fused kernel per half-step plus on-device
-    ghost-layer exchange (x faces, then y, then z)."""
+    """Subdomains stepped by one fused kernel per half-step, or per pair of them
+    in longer sequences, plus on-device ghost-layer exchange (x faces, then y,
+    then z)."""
 
     def __init__(self, solvers: Sequence[LbmSolver]):
         self._lib = _capi.load_library()
