@@ -939,7 +939,7 @@ __device__ __forceinline__ void pair_st_wrap(gchar *p, int s, int cells, unsigne
 // (index, block split, straddle check), for each of beta's 36 shifted accesses.
 // The two-byte kernels issue vector instructions near the SIMDs' limit, so
 // these count.  Chosen per access: a wavefront with one run across a block's
-// end keeps the others' (384x192x192 FP16 channel: beta 236 -> 214 us).
+// end keeps the others' (384x192x192 FP16 channel: beta 230 -> 204-212 us).
 struct PairRun {
     unsigned c0, span, lo;
 };

@@ -179,10 +179,11 @@ __device__ __forceinline__ bool pair_update(T *f, int flag, const PairPhys<T> &p
 // scalar counters untouched).
 __device__ __forceinline__ void loads_arrived() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
-// What bounds it: FP32 with LES issues about 1000 vector instructions per cell
-// and pair (beta on the halo included), 70-88 % of the SIMDs' issue slots;
-// HBM carries about 3.0 GB a pair at 256^3 where two half-step launches move
-// 5.1 GB.  256^3 LES: FP32 336 us a step against 464 in place (419 with the
+// What bounds it: FP32 with LES issues 1270 vector instructions per cell and
+// pair (beta on the halo included; 1070 with 128-cell rows), 91 % (76 %) of the
+// SIMDs' issue slots at 256^3; FP64 45 %, with two wavefronts to a SIMD that
+// wait for each other's planes.  HBM carries 2.85 GB a pair at 256^3 FP32 where
+// two half-step launches move 5.15 GB.  256^3 LES: FP32 336 us a step against 464 in place (419 with the
 // best launch shape), FP64 563 against 922 (863).
 template <int ST, int NT, bool LAYERS>
 __global__ void __launch_bounds__(NT, ST == 1 ? 2 : 4)
