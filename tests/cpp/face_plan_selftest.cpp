@@ -1,6 +1,7 @@
 // Checks the plan by which members that exchange faces run as fused pairs: it
 // is whole for the present members or empty, and its copies and rows cover
 // every exchanged cell once.
+#include <chrono>
 #include <cstdio>
 
 #include "face_plan.hpp"
@@ -111,6 +112,22 @@ int main() {
                 if (P.seams) CHECK(!box_isect(h.dof, h.sz, o, sz, io, is), "a copy in the rows of pair_kernel");
                 for (int a = 0; a < 3; ++a) CHECK(h.dof[a] >= 0 && h.dof[a] + h.sz[a] <= d[a], "copy outside");
             }
+    }
+    // many members: the plan's time grows with them, not with their square
+    {
+        const int n = 10;
+        Dims many(n * n * n, {12, 12, 12});
+        std::vector<GroupComm> c;
+        for (int i = 0; i < n * n * n; ++i) {
+            const int at[3] = {i % n, i / n % n, i / n / n}, step[3] = {1, n, n * n};
+            for (int a = 0; a < 3; ++a)
+                if (at[a] < n - 1) join(c, many, i, i + step[a], a);
+        }
+        const auto t0 = std::chrono::steady_clock::now();
+        P = plan(many, c);
+        const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        check_whole(P, many.size(), "a thousand");
+        CHECK(s < 2.0, "a thousand members: %.1f s", s);
     }
     if (fails) {
         printf("%d failures\n", fails);

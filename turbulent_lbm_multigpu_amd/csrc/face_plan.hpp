@@ -4,6 +4,8 @@
 
 #include <stddef.h>
 
+#include <map>
+
 #include "exchange_plan.hpp"
 #include "pair_plan.hpp"
 
@@ -15,14 +17,24 @@ struct GroupComm {
     int send_origin[3], recv_origin[3], size[3], normal[3];
 };
 
-// The counterpart of a comm: its partner's comm across the same face.
-inline const GroupComm *partner_of(const std::vector<GroupComm> &comms, const GroupComm &c) {
-    for (const GroupComm &q : comms)
-        if (q.member == c.dst && q.dst == c.member && q.normal[0] == -c.normal[0] && q.normal[1] == -c.normal[1] &&
-            q.normal[2] == -c.normal[2])
-            return &q;
-    return nullptr;
-}
+// The counterparts of comms: the partner's comm across the same face (its first).
+class Partners {
+  public:
+    explicit Partners(const std::vector<GroupComm> &comms) {
+        for (const GroupComm &c : comms) at_.insert({key(c.member, c.dst, c.normal, 1), &c});
+    }
+    const GroupComm *of(const GroupComm &c) const {
+        const auto it = at_.find(key(c.dst, c.member, c.normal, -1));
+        return it == at_.end() ? nullptr : it->second;
+    }
+
+  private:
+    typedef std::array<int, 5> Key;
+    static Key key(int member, int dst, const int *n, int sign) {
+        return Key{{member, dst, sign * n[0], sign * n[1], sign * n[2]}};
+    }
+    std::map<Key, const GroupComm *> at_;
+};
 
 // The two copies of a comm and its counterpart: [0] after alpha, [1] after
 // beta, with the populations each of them takes.
@@ -66,8 +78,9 @@ FacePlan plan_faces(const std::vector<std::array<int, 3>> &dims, bool stops, con
     FacePlan P;
     P.layers.assign(dims.size(), 0u);
     std::vector<HOp> phase[2][3];
+    const Partners partners(comms);
     for (const GroupComm &c : comms) {
-        const GroupComm *p = partner_of(comms, c);
+        const GroupComm *p = partners.of(c);
         if (!p) return FacePlan{};
         const int a = c.normal[0] ? 0 : c.normal[1] ? 1 : 2, side = c.normal[a] == 1 ? 0 : 1;
         for (const GroupComm *q : {&c, p}) {

@@ -2264,11 +2264,12 @@ static int upload_ops(lbm_group *g, std::vector<CopyOp> &ops, std::vector<int> &
 static int build_plan(lbm_group *g) {
     std::vector<CopyOp> ops[2][4];
     std::vector<HOp> hops[2][4];
+    const Partners partners(g->comms);
     std::vector<const GroupComm *> partner(g->comms.size(), nullptr);
     std::vector<char> fuse(g->comms.size(), 0);
     for (size_t ci = 0; ci < g->comms.size(); ++ci) {
         const GroupComm &c = g->comms[ci];
-        partner[ci] = partner_of(g->comms, c);
+        partner[ci] = partners.of(c);
         if (!partner[ci])
             return gfail(g, LBM_ERR_STATE,
                          "comm of member " + std::to_string(c.member) + " toward " + std::to_string(c.dst) +
