@@ -156,8 +156,9 @@ int lbm_solver_simulation_step_beta(lbm_solver *s);
 /* `steps` half-steps.  A sequence of at least 4 in FP32 or FP64 may go through
  * a second buffer of the distributions, two half-steps in one pass, as may
  * lbm_group_step's: same results, in the same place.  Where the pass is the
- * faster way the buffer is taken by the first such sequence, doubles the
- * distributions' memory and stays with the solver.  It is taken only while half
+ * faster way the buffer is taken once the half-steps of such sequences would
+ * repay it (from lbm_group_prepare_steps at once), doubles the distributions'
+ * memory and stays with the solver.  It is taken only while half
  * the device's memory stays free (else the sequence steps in place, and asks
  * again after 63 more) and given up when an allocation of this library fails.
  * Solvers in caller-provided memory step in place, as does a sequence that a

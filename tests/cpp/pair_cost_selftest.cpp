@@ -119,6 +119,16 @@ int main() {
         ++fails;
         printf("FAIL: the least cells\n");
     }
+    // the second buffer: not for a first short run, but for a long one or for many
+    {
+        const std::vector<WalkSet> sets = plan_walks({{{96, 96, 96}}}, false).sets;
+        const double gain = pairs_gain_us(sets, nullptr, false, false), setup = pairs_setup_us(67.2, false, 0);
+        if (setup_repaid(gain, setup, 0, 4) || !setup_repaid(gain, setup, 0, 200) || !setup_repaid(gain, setup, 196, 4) ||
+            pairs_setup_us(67.2, true, 24) <= setup) {
+            ++fails;
+            printf("FAIL: gain %.1f a half-step, setup %.1f\n", gain, setup);
+        }
+    }
     // unequal members: the long ones decide how the last slots empty
     std::vector<std::array<int, 3>> mixed(40, {64, 64, 64});
     mixed.resize(60, {24, 24, 24});

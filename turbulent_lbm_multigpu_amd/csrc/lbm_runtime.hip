@@ -390,6 +390,8 @@ struct lbm_solver {
     std::vector<PairTile> pair_tiles;  // their copy on the host (the upload reads it)
     int npair = 0;               // their number; 0: not planned yet, -1: this domain steps in place
     PairLaunch pair_launch{};
+    double pair_gain_us = 0;     // of a half-step in a pair
+    long long waited = 0;        // half-steps in place that could have gone in pairs (setup_repaid)
     long long fused_pairs = 0;   // pairs its runs have launched
     std::atomic<unsigned> version{0};  // bumps when kernel parameters change
     lbm_group *group = nullptr;
@@ -439,6 +441,8 @@ struct lbm_group {
     size_t pair_cap = 0;
     int npair = 0;               // 0: not planned for the present members, comms and variant, -1: they step in place
     std::vector<PairTile> pair_tiles;  // planned, not on the device yet
+    double pair_gain_us = 0;     // of a half-step in a pair
+    long long waited = 0;        // half-steps in place that could have gone in pairs (setup_repaid)
     PairLaunch pair_launch{};
     // Fused pairs of members that exchange faces: their plan, on the device the
     // boxes of the layers and, per block, its box, and the copies after beta
@@ -628,6 +632,7 @@ hipError_t launch_pair_kernel(int storage, const PairLaunch &L, int ntiles, cons
 struct PairPlan {
     std::vector<PairTile> tiles;
     PairLaunch launch;
+    double gain_us = 0;  // on a half-step
 };
 
 long long cells_of(const std::vector<lbm_solver *> &doms) {
@@ -645,7 +650,7 @@ long long cells_of(const std::vector<lbm_solver *> &doms) {
 // solvers of one thread (in place between the two, as the host launches): FP32
 // 40^3 24-33 / 22, 44^3 26-34 / 30, 48^3 27-34 / 37; FP64 28^3 25-32 / 27, 36^3
 // 31-36 / 32, 40^3 32-36 / 39.
-bool boxes_pay(const lbm_solver *m, int storage, BoxShape *shape, PairLaunch *launch) {
+bool boxes_pay(const lbm_solver *m, int storage, BoxShape *shape, PairLaunch *launch, double *gain_us) {
     const int *d = m->cfg.dims;
     const bool f64 = storage == LBM_STORAGE_F64;
     if (elem_size(storage) == 2 || m->cells > (f64 ? 47000 : 66000)) return false;
@@ -660,6 +665,7 @@ bool boxes_pay(const lbm_solver *m, int storage, BoxShape *shape, PairLaunch *la
     if (shape->cost < 0.0) return false;
     const double boxes = f64 ? 3.5 + 0.30 * shape->cost : 3.0 + 0.21 * shape->cost;
     const double in_place = f64 ? 9.0 + 6.8e-5 * (double)m->cells : 8.2 + 3.4e-5 * (double)m->cells;
+    *gain_us = 0.5 * (in_place - boxes);
     return boxes < 0.96 * in_place;
 }
 
@@ -672,7 +678,7 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage, int vari
     if (elem_size(storage) == 2) return P;
     if (cells_of(doms) < walk_cells(f64)) {
         BoxShape shape;
-        if (doms.size() == 1 && boxes_pay(doms[0], storage, &shape, &P.launch)) {
+        if (doms.size() == 1 && boxes_pay(doms[0], storage, &shape, &P.launch, &P.gain_us)) {
             const int *d = doms[0]->cfg.dims;
             box_tiles(0, d[0], d[1], d[2], shape, P.tiles);
         }
@@ -687,6 +693,7 @@ PairPlan plan_pairs(const std::vector<lbm_solver *> &doms, int storage, int vari
     const WalkPlan W = plan_walks(dims, f64);
     if (!walks_pay(W.sets, f64, nt) || (faces && !face_pairs_pay(W.sets, *faces, f64, nt))) return P;
     P.launch.threads = W.threads;
+    P.gain_us = pairs_gain_us(W.sets, faces, f64, nt);
     for (size_t i = 0; i < doms.size(); ++i)
         pair_tiles((int)i, dims[i][0], dims[i][1], dims[i][2], W.shape[i], W.sets[i].nz, P.tiles);
     // Tiles dealt to the XCDs in chunks of 8 once the state is well past the
@@ -739,28 +746,43 @@ bool take_seconds(const std::vector<lbm_solver *> &solvers) {
     return second_buffers().take(all);
 }
 
-// Second buffer and tile table of a solver stepped on its own; false: the run
-// steps in place.
-bool solver_pairs_ready(lbm_solver *s) {
+// Second buffer and tile table of a solver stepped on its own, for a run of
+// `steps`; false: it steps in place.
+bool solver_pairs_ready(lbm_solver *s, int steps) {
     if (s->external || s->npair < 0 || recording(s->stream)) return false;  // no memory beyond the caller's
-    if (!s->d_pair) {
+    if (!s->npair) {
         PairPlan P = plan_pairs({s}, s->cfg.storage, s->cfg.kernel_variant);
         s->npair = P.tiles.empty() ? -1 : (int)P.tiles.size();
         if (s->npair < 0) return false;
+        s->pair_tiles.swap(P.tiles);
+        s->pair_launch = P.launch;
+        s->pair_gain_us = P.gain_us;
+    }
+    if (!s->second.at && !setup_repaid(s->pair_gain_us, pairs_setup_us(1e-6 * (double)s->second.bytes, false, 0),
+                                       s->waited, steps)) {
+        s->waited += steps;
+        return false;
+    }
+    if (!s->d_pair) {
         const OnDevice on(s->cfg.device);
-        if (hipMalloc((void **)&s->d_pair, sizeof(PairTile) * P.tiles.size()) != hipSuccess) {
+        if (hipMalloc((void **)&s->d_pair, sizeof(PairTile) * s->pair_tiles.size()) != hipSuccess) {
             (void)hipGetLastError();
             s->d_pair = nullptr;
             return false;
         }
-        s->pair_tiles.swap(P.tiles);
-        if (hipMemcpyAsync(s->d_pair, s->pair_tiles.data(), sizeof(PairTile) * s->pair_tiles.size(),
-                           hipMemcpyHostToDevice, s->stream) != hipSuccess) {
+        // in pieces: a process's first copy of more than 16 KB takes 6 ms
+        const size_t bytes = sizeof(PairTile) * s->pair_tiles.size(), piece = (size_t)16 << 10;
+        hipError_t e = hipSuccess;
+        for (size_t at = 0; at < bytes && e == hipSuccess; at += piece)
+            e = hipMemcpyAsync((char *)s->d_pair + at, (const char *)s->pair_tiles.data() + at,
+                               std::min(piece, bytes - at), hipMemcpyHostToDevice, s->stream);
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(s->stream);  // a piece may still be on its way
+            (void)hipGetLastError();
             (void)hipFree(s->d_pair);
             s->d_pair = nullptr;
             return false;
         }
-        s->pair_launch = P.launch;
     }
     return pair_kernel_ready(s->cfg.storage, s->pair_launch, s->cfg.device) && take_seconds({s});
 }
@@ -1208,7 +1230,7 @@ extern "C" int lbm_solver_run(lbm_solver *s, int steps) {
         if (rc) return rc;
         ++i;
     }
-    if (steps - i >= 4 && (s->step_counter & 1) == 0 && solver_pairs_ready(s)) {
+    if (steps - i >= 4 && (s->step_counter & 1) == 0 && solver_pairs_ready(s, steps - i)) {
         const auto lock = second_buffers().in_use();
         // Two pairs at a time: into the second buffer and back.  Boxes, of which
         // each takes much of a compute unit's LDS, only while no other thread's
@@ -2524,8 +2546,9 @@ static int upload_faces(lbm_group *g) {
 // pairs: second buffers for every member, faces that are exchanged in a way
 // plan_faces knows, and no member that freezes on the way (a member frozen
 // already keeps its state; one that freezes between two pairs would keep it in
-// the wrong buffer).  Brings the pair tiles and descriptors up to date.
-static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
+// the wrong buffer), enough steps to repay the setup (`prepare`: as if).  Brings
+// the pair tiles and descriptors up to date.
+static int group_pairs_ready(lbm_group *g, int steps, bool prepare, bool *ready) {
     *ready = false;
     if (steps < 4 || g->timing || g->npair < 0 || recording(g->stream)) return LBM_OK;
     for (const lbm_solver *m : g->members)
@@ -2541,6 +2564,19 @@ static int group_pairs_ready(lbm_group *g, int steps, bool *ready) {
         if (g->npair < 0) return LBM_OK;
         g->pair_tiles.swap(P.tiles);
         g->pair_launch = P.launch;
+        g->pair_gain_us = P.gain_us;
+        g->waited = 0;
+    }
+    bool held = true;
+    size_t bytes = 0;
+    for (const lbm_solver *m : g->members) {
+        held = held && m->second.at;
+        bytes += m->second.bytes;
+    }
+    if (!held && !prepare &&
+        !setup_repaid(g->pair_gain_us, pairs_setup_us(1e-6 * (double)bytes, true, g->comms.size()), g->waited, steps)) {
+        g->waited += steps;
+        return LBM_OK;
     }
     if (!g->comms.empty()) {
         int rc = group_prepare(g);  // refuses comms without a counterpart
@@ -2705,7 +2741,7 @@ static int group_walk(lbm_group *g, int steps, bool run, bool fused, int *done_o
 // that use second buffers hold them.
 static int group_advance(lbm_group *g, int steps, bool run, int *done) {
     bool fused = false;
-    int rc = group_pairs_ready(g, steps, &fused);
+    int rc = group_pairs_ready(g, steps, !run, &fused);
     if (rc) return rc;
     if (!fused) return group_walk(g, steps, run, false, done);
     const auto lock = second_buffers().in_use();

@@ -142,19 +142,53 @@ struct FaceCells {
 // gains down to 84 MB (2 of 100^3 56-69 / 54, 3 of 40x100x100 42-52 / 40, with
 // the default policy 52 / 54 and 38-44 / 40).  The non-temporal margin is the
 // fit's error there.
+struct FaceTimes {
+    double in_place, pairs;  // two half-steps
+};
+inline FaceTimes face_times(const std::vector<WalkSet> &sets, long long cells, const FaceCells &faces, bool f64, bool nt) {
+    const double x = 1e-5 * (double)faces.x, yz = 1e-5 * (double)faces.yz;
+    const double half = 2.0 * in_place_us(cells, f64, nt);
+    return FaceTimes{f64 ? (nt ? 1.080 * half + 31.3 * x + 6.1 * yz : 1.127 * half + 25.1 * x + 5.6 * yz)
+                         : (nt ? 1.155 * half + 20.4 * x + 2.4 * yz : 1.204 * half + 16.2 * x + 1.5 * yz),
+                     f64 ? 3.0 + 1.19 * walks_us(sets, f64) + 35.7 * x + 9.5 * yz
+                         : 15.7 + 1.23 * walks_us(sets, f64) + 25.8 * x + 4.7 * yz};
+}
 inline bool face_pairs_pay(const std::vector<WalkSet> &sets, const FaceCells &faces, bool f64, bool nt) {
     long long cells = 0;
     for (const WalkSet &s : sets) cells += s.cells;
     const double state = 19e-6 * (double)cells * (f64 ? 8 : 4);  // MB
     if (!f64 && nt && faces.yz == 0) return state >= 84.0;
     if (state < 335.0) return false;
-    const double x = 1e-5 * (double)faces.x, yz = 1e-5 * (double)faces.yz;
-    const double half = 2.0 * in_place_us(cells, f64, nt);
-    const double in_place = f64 ? (nt ? 1.080 * half + 31.3 * x + 6.1 * yz : 1.127 * half + 25.1 * x + 5.6 * yz)
-                                : (nt ? 1.155 * half + 20.4 * x + 2.4 * yz : 1.204 * half + 16.2 * x + 1.5 * yz);
-    const double pair = f64 ? 3.0 + 1.19 * walks_us(sets, f64) + 35.7 * x + 9.5 * yz
-                            : 15.7 + 1.23 * walks_us(sets, f64) + 25.8 * x + 4.7 * yz;
-    return pair * (nt ? 1.065 : 1.0) <= in_place;
+    const FaceTimes t = face_times(sets, cells, faces, f64, nt);
+    return t.pairs * (nt ? 1.065 : 1.0) <= t.in_place;
+}
+
+// What pairs gain on a half-step, us (at least a twentieth, where they pay at all).
+inline double pairs_gain_us(const std::vector<WalkSet> &sets, const FaceCells *faces, bool f64, bool nt) {
+    long long cells = 0;
+    for (const WalkSet &s : sets) cells += s.cells;
+    FaceTimes t{2.0 * in_place_us(cells, f64, nt), 0.0};
+    if (faces) t = face_times(sets, cells, *faces, f64, nt);
+    else t.pairs = walks_us(sets, f64);
+    return 0.5 * std::max(t.in_place - t.pairs, 0.05 * t.in_place);
+}
+
+// What the first pairs cost besides, us: the second buffers, tile tables and,
+// of a group, its descriptors and the copies of its `comms`; an allocation takes
+// about a microsecond a megabyte.  Of a solver, first run(4) in place / with
+// that: 20^3 29 / 46-105, 96^3 110 / 240, 160^3 440 / 560; of a group, first
+// step(4): 40 of 48^3 640 / 850-1200, 2x2x2 of 128^3 2350 / 2850-4800, 4x4x4 of
+// 64^3 3400 / 6500.
+inline double pairs_setup_us(double state_mb, bool group, size_t comms) {
+    return (group ? 250.0 : 80.0) + state_mb + 10.5 * (double)comms;
+}
+
+// Whether a sequence of `steps` half-steps is to pay that: once what it gains,
+// with what `before` half-steps that went in place would have gained, makes up
+// for it.  So short runs from new states stay as they were, and long ones and
+// repeated ones lose at most that much again.
+inline bool setup_repaid(double gain_us, double setup_us, long long before, long long steps) {
+    return gain_us * (double)(before + steps) >= setup_us;
 }
 
 }  // namespace lbm
