@@ -1,6 +1,7 @@
 // Checks the choice between fused pairs and half-steps in place against shapes
 // that were measured both ways: the faster way where they differ by more than
 // the fit's error.
+#include <cmath>
 #include <cstdio>
 
 #include "pair_cost.hpp"
@@ -59,7 +60,8 @@ static const Joined FACES[] = {
     {{2, 1, 1}, {160, 160, 160}, false, false, true},  // 277 / 175
     {{10, 10, 1}, {16, 16, 200}, false, false, false}, // 221 / 280
     {{1, 1, 8}, {512, 512, 4}, false, false, false},   // 257 / 264
-    {{4, 1, 4}, {70, 70, 70}, false, true, false},     // 160 / 173
+    {{4, 1, 4}, {70, 70, 70}, false, true, true},      // 160 / 166, among others 189 / 155
+    {{2, 3, 2}, {92, 70, 65}, false, true, true},      // 177 / 146, among others 188 / 136
     {{5, 5, 5}, {32, 32, 32}, false, false, false},    // 148 / 162
     {{8, 8, 8}, {20, 20, 20}, false, false, false},    // 200 / 230
     {{2, 2, 2}, {12, 200, 200}, false, false, false},  // 118-122 / 127
@@ -128,6 +130,22 @@ int main() {
             ++fails;
             printf("FAIL: gain %.1f a half-step, setup %.1f\n", gain, setup);
         }
+    }
+    // idle slots at a launch's end count half: nearly equal lengths that fill
+    // them, and one round and a bit of unequal ones
+    {
+        const std::vector<WalkSet> even = plan_walks(std::vector<std::array<int, 3>>(200, {24, 24, 24}), false).sets;
+        std::vector<std::array<int, 3>> few;
+        for (int n = 17; n <= 58; n += 4) few.push_back({n, 60 - n / 2, n});
+        const std::vector<WalkSet> ragged = plan_walks(few, false).sets;
+        for (const auto &sets : {even, ragged}) {
+            const double own = walks_us(sets, false), filled = walks_us(sets, false, true), e = expected_walks_us(sets, false);
+            if (filled <= own + 1e-9 && std::abs(e - 0.5 * (own + filled)) < 1e-9) continue;
+            ++fails;
+            printf("FAIL: own %.1f, filled %.1f, expected %.1f\n", own, filled, e);
+        }
+        const std::vector<WalkSet> one = plan_walks({{{100, 100, 100}}}, false).sets;
+        if (expected_walks_us(one, false) != walks_us(one, false)) ++fails, printf("FAIL: a domain on its own\n");
     }
     // unequal members: the long ones decide how the last slots empty
     std::vector<std::array<int, 3>> mixed(40, {64, 64, 64});

@@ -70,8 +70,9 @@ inline WalkPlan plan_walks(const std::vector<std::array<int, 3>> &dims, bool f64
 // pair: FP32 96^3 34 / 38, 160^3 147 / 150, 256^3 655 / 677, 400x401x3 25 / 25,
 // 1000x1000x3 148 / 136, 8x8x20000 189 / 174, 3000 of 8^3 266 / 259, 500 of
 // 16^3 125 / 123; FP64 64^3 26 / 25, 128^3 199 / 180, 160^3 289 / 287,
-// 300x300x3 37 / 38, 4000 of 8^3 428 / 410.
-inline double walks_us(const std::vector<WalkSet> &sets, bool f64) {
+// 300x300x3 37 / 38, 4000 of 8^3 428 / 410.  `filled`: where other streams'
+// launches take the slots that are idle at its end.
+inline double walks_us(const std::vector<WalkSet> &sets, bool f64, bool filled = false) {
     auto walk_us = [f64](const WalkSet &s) {
         return ((double)s.nz + 2.5) * (f64 ? 1.84 + 0.0385 * s.waves : 1.70 + 0.0167 * s.waves);
     };
@@ -86,7 +87,9 @@ inline double walks_us(const std::vector<WalkSet> &sets, bool f64) {
         cells += s.cells;
     }
     double rounds = longest * (double)((groups + kPairSlots - 1) / kPairSlots);
-    if (shortest < longest) {  // each walk takes the slot that is free first
+    if (filled) {
+        rounds = sum / (double)kPairSlots;
+    } else if (shortest < longest) {  // each walk takes the slot that is free first
         if (groups > 64 * kPairSlots) {
             rounds = sum / (double)kPairSlots + 0.5 * longest;
         } else {
@@ -105,6 +108,16 @@ inline double walks_us(const std::vector<WalkSet> &sets, bool f64) {
     return (f64 ? 2.4 : 3.2) + rounds + (f64 ? 37.2e-6 : 20.4e-6) * (double)cells;
 }
 
+// The time to choose by.  A group's walks leave slots idle at their end, most of
+// all where members differ, so that groups of several streams gain from pairs
+// what one group on its own loses; as often the one as the other is assumed.  In
+// place / pairs, us a half-step on its own and among others: 10 members of 17 to
+// 58 cells an edge 17 / 21 and 12.5 / 10.9, 14 of 14 to 79 34 / 35 and 31 / 26.
+inline double expected_walks_us(const std::vector<WalkSet> &sets, bool f64) {
+    const double own = walks_us(sets, f64);
+    return sets.size() > 1 ? 0.5 * (own + walks_us(sets, f64, true)) : own;
+}
+
 // Domains of fewer cells have too few columns to hide a walk's latency; us a
 // step, in place / walks: FP32 64^3 8.7 / 10.3, 72^3 10.4 / 10.8, 80^3 14.3 /
 // 13.2; FP64 48^3 7.7 / 10.0, 64^3 14.1 / 12.9.
@@ -121,7 +134,7 @@ inline bool walks_pay(const std::vector<WalkSet> &sets, bool f64, bool nt) {
     for (const WalkSet &s : sets) cells += s.cells;
     if (cells < walk_cells(f64)) return false;
     const double margin = f64 ? (nt ? 1.10 : 1.06) : (nt ? 1.07 : 1.045);
-    return walks_us(sets, f64) * margin <= 2.0 * in_place_us(cells, f64, nt);
+    return expected_walks_us(sets, f64) * margin <= 2.0 * in_place_us(cells, f64, nt);
 }
 
 // The same for domains that exchange faces (plan_faces): cells of the x faces
@@ -140,8 +153,10 @@ struct FaceCells {
 // 16x16x200 221 / 280, 8 of 512x512x4 257 / 264; FP64 8 of 96^3 416-473 / 327,
 // 8 of 300x300x4 339 / 370.  FP32 joined in x only with non-temporal accesses
 // gains down to 84 MB (2 of 100^3 56-69 / 54, 3 of 40x100x100 42-52 / 40, with
-// the default policy 52 / 54 and 38-44 / 40).  The non-temporal margin is the
-// fit's error there.
+// the default policy 52 / 54 and 38-44 / 40).  The FP64 non-temporal margin is the
+// fit's error there; FP32 goes by equal times, since pairs lose less to other
+// streams: 16 of 70^3 160 / 166 and, among others, 189 / 155, 12 of 92x70x65 177 /
+// 146 and 188 / 136.
 struct FaceTimes {
     double in_place, pairs;  // two half-steps
 };
@@ -160,7 +175,7 @@ inline bool face_pairs_pay(const std::vector<WalkSet> &sets, const FaceCells &fa
     if (!f64 && nt && faces.yz == 0) return state >= 84.0;
     if (state < 335.0) return false;
     const FaceTimes t = face_times(sets, cells, faces, f64, nt);
-    return t.pairs * (nt ? 1.065 : 1.0) <= t.in_place;
+    return t.pairs * (nt && f64 ? 1.065 : 1.0) <= t.in_place;
 }
 
 // What pairs gain on a half-step, us (at least a twentieth, where they pay at all).
@@ -169,7 +184,7 @@ inline double pairs_gain_us(const std::vector<WalkSet> &sets, const FaceCells *f
     for (const WalkSet &s : sets) cells += s.cells;
     FaceTimes t{2.0 * in_place_us(cells, f64, nt), 0.0};
     if (faces) t = face_times(sets, cells, *faces, f64, nt);
-    else t.pairs = walks_us(sets, f64);
+    else t.pairs = expected_walks_us(sets, f64);
     return 0.5 * std::max(t.in_place - t.pairs, 0.05 * t.in_place);
 }
 
