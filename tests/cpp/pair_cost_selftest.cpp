@@ -124,11 +124,18 @@ int main() {
     // the second buffer: not for a first short run, but for a long one or for many
     {
         const std::vector<WalkSet> sets = plan_walks({{{96, 96, 96}}}, false).sets;
-        const double gain = pairs_gain_us(sets, nullptr, false, false), setup = pairs_setup_us(67.2, false, 0);
+        const double gain = pairs_gain_us(sets, nullptr, false, false), setup = pairs_setup_us(67.2, false, 0, false);
         if (setup_repaid(gain, setup, 0, 4) || !setup_repaid(gain, setup, 0, 200) || !setup_repaid(gain, setup, 196, 4) ||
-            pairs_setup_us(67.2, true, 24) <= setup) {
+            pairs_setup_us(67.2, true, 24, false) <= setup) {
             ++fails;
             printf("FAIL: gain %.1f a half-step, setup %.1f\n", gain, setup);
+        }
+        // with a buffer at hand the size does not count: a first run of 12 has them at once
+        const double at_hand = pairs_setup_us(67.2, false, 0, true);
+        if (setup_repaid(gain, setup, 0, 12) || !setup_repaid(gain, at_hand, 0, 12) || at_hand >= setup ||
+            at_hand != pairs_setup_us(1000, false, 0, true) || pairs_setup_us(67.2, true, 24, true) <= at_hand) {
+            ++fails;
+            printf("FAIL: gain %.1f a half-step, setup %.1f and with a spare %.1f\n", gain, setup, at_hand);
         }
     }
     // idle slots at a launch's end count half: nearly equal lengths that fill

@@ -150,7 +150,9 @@ static void blocks_and_spares() {
         sb.give(c.second);
         sb.give(c.second);
     }
-    Solver d(900);
+    Solver d(900), far(300, 1), large(40000);
+    CHECK(sb.has_spare({&d.second}) && sb.has_spare({&far.second}) && !sb.has_spare({&large.second}));
+    CHECK(!sb.has_spare({&d.second, &large.second}) && !sb.has_spare({}));
     CHECK(sb.take({&d.second}) && mem.blocks == 3);
     sb.give(d.second);
     {

@@ -365,6 +365,20 @@ def test_short_runs_of_new_states_step_in_place(dims, storage):
         g.close()
 
 
+def test_a_buffer_at_hand_is_taken_sooner():
+    """One that a destroyed solver left costs no allocation."""
+    release_kept_memory()
+    with build((128, 128, 128), F32) as s:
+        s.run(8)
+        assert s.pair_count()["pairs"] == 0
+        settle(s)
+    with build((128, 128, 128), F32) as a, build((128, 128, 128), F32) as b:
+        a.run(8)
+        assert a.pair_count()["pairs"] == 4
+        single_steps(b, 8)
+        same(a, b)
+
+
 # Every form of a domain that pairs take, after a second buffer is there: forcing, outputs, faces of
 # all kinds, BGK and LES; walks by runs and rectangles, boxes.
 FORMS = [

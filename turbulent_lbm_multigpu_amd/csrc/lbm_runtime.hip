@@ -739,12 +739,17 @@ bool pair_kernel_ready(int storage, const PairLaunch &L, int device) {
     return e == hipSuccess;
 }
 
-// Second buffers for all of them; false: they have to do without.
-bool take_seconds(const std::vector<lbm_solver *> &solvers) {
+std::vector<SecondBuffer *> seconds_of(const std::vector<lbm_solver *> &solvers) {
     std::vector<SecondBuffer *> all;
     for (lbm_solver *s : solvers) all.push_back(&s->second);
-    return second_buffers().take(all);
+    return all;
 }
+
+// Second buffers for all of them; false: they have to do without.
+bool take_seconds(const std::vector<lbm_solver *> &solvers) { return second_buffers().take(seconds_of(solvers)); }
+
+// Whether that needs no allocation.
+bool spare_at_hand(const std::vector<lbm_solver *> &solvers) { return second_buffers().has_spare(seconds_of(solvers)); }
 
 // Second buffer and tile table of a solver stepped on its own, for a run of
 // `steps`; false: it steps in place.
@@ -758,7 +763,7 @@ bool solver_pairs_ready(lbm_solver *s, int steps) {
         s->pair_launch = P.launch;
         s->pair_gain_us = P.gain_us;
     }
-    if (!s->second.at && !setup_repaid(s->pair_gain_us, pairs_setup_us(1e-6 * (double)s->second.bytes, false, 0),
+    if (!s->second.at && !setup_repaid(s->pair_gain_us, pairs_setup_us(1e-6 * (double)s->second.bytes, false, 0, spare_at_hand({s})),
                                        s->waited, steps)) {
         s->waited += steps;
         return false;
@@ -2574,7 +2579,8 @@ static int group_pairs_ready(lbm_group *g, int steps, bool prepare, bool *ready)
         bytes += m->second.bytes;
     }
     if (!held && !prepare &&
-        !setup_repaid(g->pair_gain_us, pairs_setup_us(1e-6 * (double)bytes, true, g->comms.size()), g->waited, steps)) {
+        !setup_repaid(g->pair_gain_us, pairs_setup_us(1e-6 * (double)bytes, true, g->comms.size(), spare_at_hand(g->members)),
+                      g->waited, steps)) {
         g->waited += steps;
         return LBM_OK;
     }

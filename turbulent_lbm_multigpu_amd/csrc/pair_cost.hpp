@@ -193,9 +193,9 @@ inline double pairs_gain_us(const std::vector<WalkSet> &sets, const FaceCells *f
 // about a microsecond a megabyte.  Of a solver, first run(4) in place / with
 // that: 20^3 29 / 46-105, 96^3 110 / 240, 160^3 440 / 560; of a group, first
 // step(4): 40 of 48^3 640 / 850-1200, 2x2x2 of 128^3 2350 / 2850-4800, 4x4x4 of
-// 64^3 3400 / 6500.
-inline double pairs_setup_us(double state_mb, bool group, size_t comms) {
-    return (group ? 250.0 : 80.0) + state_mb + 10.5 * (double)comms;
+// 64^3 3400 / 6500.  `spare`: a destroyed solver's buffer is at hand.
+inline double pairs_setup_us(double state_mb, bool group, size_t comms, bool spare) {
+    return (spare ? (group ? 150.0 : 30.0) : (group ? 250.0 : 80.0) + state_mb) + 10.5 * (double)comms;
 }
 
 // Whether a sequence of `steps` half-steps is to pay that: once what it gains,

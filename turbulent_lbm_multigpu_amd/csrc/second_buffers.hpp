@@ -80,14 +80,12 @@ class SecondBuffers {
         const std::lock_guard<std::mutex> lock(mutex_);
         const int device = without[0]->device;
         SecondBlock *b = nullptr;
-        for (auto it = spares_.rbegin(); it != spares_.rend(); ++it) {
-            if ((*it)->device != device || (*it)->bytes < bytes || (*it)->bytes > 2 * bytes) continue;
-            b = *it;
+        const auto spare = spare_for(device, bytes);
+        if (spare != spares_.end()) {
+            b = *spare;
             spare_bytes_ -= b->bytes;
-            spares_.erase(std::next(it).base());
-            break;
-        }
-        if (!b) {
+            spares_.erase(spare);
+        } else {
             void *const p = memory_.allocate(device, bytes);
             if (!p) {
                 for (SecondBuffer *s : without) {
@@ -109,6 +107,15 @@ class SecondBuffers {
             (*s->version)++;
         }
         return true;
+    }
+
+    // Whether a block that is kept would do for these, so that none is allocated.
+    bool has_spare(const std::vector<SecondBuffer *> &all) {
+        size_t bytes = 0;
+        for (SecondBuffer *s : all)
+            if (!s->at) bytes += aligned(s->bytes);
+        const std::lock_guard<std::mutex> lock(mutex_);
+        return !all.empty() && spare_for(all[0]->device, bytes) != spares_.end();
     }
 
     // A solver's last call.  The lock is taken before `at` is looked at: while
@@ -147,6 +154,14 @@ class SecondBuffers {
 
   private:
     static size_t aligned(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+    // The newest that is not more than twice as large.
+    std::vector<SecondBlock *>::iterator spare_for(int device, size_t bytes) {
+        for (auto it = spares_.end(); it != spares_.begin();) {
+            --it;
+            if ((*it)->device == device && (*it)->bytes >= bytes && (*it)->bytes <= 2 * bytes) return it;
+        }
+        return spares_.end();
+    }
     void free_spares(size_t keep_bytes, size_t keep) {
         while (!spares_.empty() && (spare_bytes_ > keep_bytes || spares_.size() > keep)) {
             SecondBlock *b = spares_.front();
