@@ -128,7 +128,9 @@ constexpr long long walk_cells(bool f64) { return f64 ? 250000 : 480000; }
 // 3000 of 8^3 37.8 / 133, 500 of 16^3 47 / 63, 4x4x60000 25 / 275, 1000x1000x3
 // 67 / 74; FP64 300x300x3 15.1 / 18.5, 400 of 12^3 33 / 51.  The margins keep
 // the fit's error around equal times from costing more than 3 % on any of about
-// 170 measured shapes and policies.
+// 170 measured shapes and policies of one domain or equal members, each on its own.
+// Of 24 batches of unequal members, 10 gain by pairs either way, 6 lose 2 to 4 % (one
+// 16) on their own and gain 8 to 44 among others (one loses 2.5), 8 step in place.
 inline bool walks_pay(const std::vector<WalkSet> &sets, bool f64, bool nt) {
     long long cells = 0;
     for (const WalkSet &s : sets) cells += s.cells;
