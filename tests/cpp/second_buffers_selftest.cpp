@@ -176,6 +176,28 @@ static void blocks_and_spares() {
     }
 }
 
+// While a thread allocates, another one's question about the spares is answered at once.
+static void asking_does_not_wait() {
+    struct Slow : HostMemory {
+        std::atomic<bool> within{false}, go{false};
+        void *allocate(int device, size_t bytes) override {
+            within = true;
+            for (int k = 0; k < 5000 && !go; ++k) std::this_thread::sleep_for(std::chrono::milliseconds(1));
+            return HostMemory::allocate(device, bytes);
+        }
+    } mem;
+    SecondBuffers sb(mem);
+    Solver a(1000), b(1000);
+    std::thread t([&] { CHECK(sb.take({&a.second})); });
+    while (!mem.within) std::this_thread::yield();
+    CHECK(!sb.has_spare({&b.second}) && !a.second.at);
+    mem.go = true;
+    t.join();
+    sb.give(a.second);
+    CHECK(sb.has_spare({&b.second}));
+    sb.give_all(0);
+}
+
 // A refusal holds for what was asked for, and for some sequences.
 static void refused_for_a_while() {
     HostMemory mem;
@@ -202,6 +224,7 @@ static void refused_for_a_while() {
 
 int main() {
     blocks_and_spares();
+    asking_does_not_wait();
     refused_for_a_while();
     launches_keep_nobody_waiting();
     destroyed_while_taken_away();

@@ -109,13 +109,14 @@ class SecondBuffers {
         return true;
     }
 
-    // Whether a block that is kept would do for these, so that none is allocated.
+    // Whether a block that is kept would do for these, so that none is allocated;
+    // not, while another thread allocates or takes away: asking does not wait.
     bool has_spare(const std::vector<SecondBuffer *> &all) {
         size_t bytes = 0;
         for (SecondBuffer *s : all)
             if (!s->at) bytes += aligned(s->bytes);
-        const std::lock_guard<std::mutex> lock(mutex_);
-        return !all.empty() && spare_for(all[0]->device, bytes) != spares_.end();
+        const std::unique_lock<std::mutex> lock(mutex_, std::try_to_lock);
+        return lock.owns_lock() && !all.empty() && spare_for(all[0]->device, bytes) != spares_.end();
     }
 
     // A solver's last call.  The lock is taken before `at` is looked at: while
